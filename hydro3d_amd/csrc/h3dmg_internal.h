@@ -69,7 +69,7 @@ struct FineDev {
   double cx, cy, cz;
   double *p[2];  // [colour]
   double *f[2];  // [colour]
-  double dx, dy, dz;     // spacing (the variable-density projection's volume factors)
+  double dx, dy, dz;     // spacing
   const double *dens;    // variable-density operator: density, interior (nk, nj, ni), or null
 };
 
@@ -226,6 +226,44 @@ size_t tdma_sweep_lds_bytes(const LevelDev &L, bool pipelined);
 hipError_t tdma_sweep_allow_lds(size_t lds_bytes);
 // fill LevelDev::tdma of every descriptor that has one (32*(ni+nj+nk) doubles)
 void launch_tdma_tables(hipStream_t s, const LevelDev *levs, int ndesc);
+
+// ---- velocity projection --------------------------------------------------
+// One block's face arrays (dense, i fastest) and, for the projection of one
+// block, its dense su (may be null).
+struct VelDev {
+  const double *us, *vs, *ws;
+  double *u, *v, *w;
+  double *su;
+};
+// dt*alfapr and dt
+struct ProjDt {
+  double dta, dt;
+};
+struct ProjLaunch {
+  int groups;     // workgroups per block (and partials per block)
+  int kb;         // planes per tile
+  int connected;  // near faces belong to the block across them
+  int to_fine;    // su into f and the level-1 rhs (else VelDev::su)
+  int calmas;     // 0: the faces only
+  int lsm, f32;   // variable density; level 1 in FP32
+  int even;       // every block of the launch has an even ni
+};
+constexpr int PROJ_MAX_GROUPS = 1024;
+// tiles of kb planes k_project cuts a block into
+inline int project_tiles(int ni, int nj, int nk, int kb) {
+  const int ne = (ni + 1) / 2;
+  int lp = 1;
+  while (lp < 64 && lp < ne) lp *= 2;
+  const int rows = NTHREADS / lp;
+  return ((ne + lp - 1) / lp) * ((nj + rows - 1) / rows) * ((nk + kb - 1) / kb);
+}
+// calvel + calmas of nblocks blocks from b0: the tables tab/dtab (tab[b] for
+// block b), or one/dt_one for a single block (tab and dtab null).  active may
+// be null (every block).  partials: nblocks x groups (null with calmas = 0).
+// No input array may overlap an output one.
+void launch_project(hipStream_t s, const ProjLaunch &a, const FineDev *fine, const LevelDev *levs,
+                    const int *active, const VelDev *tab, const ProjDt *dtab, const VelDev &one,
+                    const ProjDt &dt_one, int b0, int nblocks, RedPartial *partials);
 
 // velocity projection (calvel per axis over `faces` faces; calmas writes
 // su (optional) and one partial max per workgroup, returns the group count)

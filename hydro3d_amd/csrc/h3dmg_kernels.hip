@@ -2772,6 +2772,260 @@ __global__ void __launch_bounds__(256)
   if (threadIdx.x == 0) partials[blockIdx.x] = RedPartial{0.0, am};
 }
 
+// calvel and calmas of every block in one launch (grid.y: block, from b0).
+// Each is a stream over the faces and cells; separate launches per axis and
+// block read p three times and u, v, w twice, and cost a launch of 2-4 us
+// each (a 64-block handle: 448 launches per step).  Here a lane owns cells
+// 2l, 2l+1 of one row (one entry of both colour arrays of p) and walks kb
+// planes: the west, south and bottom faces of its cells are its own to
+// write, the east face comes from the next lane (DPP), the north face is
+// computed again, the top face carries over as the next plane's bottom, and
+// su and the rmax partial follow from the faces in registers.  Per cell that
+// reads u*, v*, w*, p and writes u, v, w, su once: 64 B instead of 104.
+// Every face and cell value is k_calvel's / k_calvel_nb's / k_calmas'
+// expression.
+//   connected: a near face across which a block lies takes that block's far
+//     face -- its u* and this face's pressures, the value k_face_copy copies;
+//   to_fine: su goes into the block's f arrays and the level-1 rhs in the
+//     level's type T (the next V-cycle starts from it), else to V.su if any;
+//   calmas = 0: faces only (calmas' 4th-order branch follows on its own).
+// Bound by memory: 192^3 takes 113 us (453 MB, 4.0 TB/s) where calvel x 3 +
+// calmas took 174; 128x128x96 28 us where they took 47; the 64 blocks of a
+// 64x8x64 layout 34 us where their 448 launches took ~1.4 ms.
+// A workgroup strides over the tiles of its block (64-entry row segments or
+// whole short rows x kb planes), so gridDim.x bounds the partials:
+// partials[(block - b0) * gridDim.x + blockIdx.x].
+typedef double __attribute__((ext_vector_type(2), aligned(8))) d2u;  // 8-byte aligned pair
+
+// Every load of a plane is issued before its first use, with no branch that
+// depends on a loaded value: ghosts are addresses (the array, row and plane
+// that hold the image), selected per lane.  EVEN: ni even, so a lane's two
+// cells are always a pair inside the row (16-byte accesses).
+template <class T, bool LSM, bool EVEN>
+__global__ void __launch_bounds__(NTHREADS)
+    k_project(const FineDev *__restrict__ fine, const LevelDev *__restrict__ levs,
+              const int *__restrict__ active, const VelDev *__restrict__ tab,
+              const ProjDt *__restrict__ dtab, VelDev one, ProjDt dt_one, int b0, int kb,
+              int connected, int to_fine, int calmas, RedPartial *__restrict__ partials) {
+  typedef typename Vec2<double>::type d2;
+  const int b = b0 + (int)blockIdx.y;
+  const FineDev &F = fine[b];
+  double am = 0.0, ss = 0.0;
+  if (!active || active[b]) {
+    const VelDev V = tab ? tab[b] : one;
+    const ProjDt D = dtab ? *dtab : dt_one;
+    const double dta = D.dta, dt = D.dt, dx = F.dx, dy = F.dy, dz = F.dz;
+    const int ni = F.ni, nj = F.nj, nk = F.nk, H = F.H;
+    const bool open_w = !wall_face(F, 0), open_e = !wall_face(F, 1), open_s = !wall_face(F, 2),
+               open_n = !wall_face(F, 3), open_b = !wall_face(F, 4), open_t = !wall_face(F, 5);
+    // the block across each face (itself on a periodic axis it spans)
+    auto across = [&](int f) -> int { return F.nbr[f] >= 0 ? F.nbr[f] : b; };
+    // lanes per row segment: the whole row's entries, or 64
+    const int ne = (ni + 1) >> 1;
+    const int lg = ne >= 64 ? 6 : ne <= 1 ? 0 : 32 - __clz(ne - 1);
+    const int lp = 1 << lg, rows = NTHREADS >> lg;
+    const int ntx = (ne + lp - 1) >> lg, nty = (nj + rows - 1) / rows, ntz = (nk + kb - 1) / kb;
+    const int tid = (int)threadIdx.x, rl = tid & (lp - 1);
+    typedef const gmem<double> *src;
+    const src P0 = (src)F.p[0], P1 = (src)F.p[1];
+    const src US = (src)V.us, VS = (src)V.vs, WS = (src)V.ws;
+    gmem<double> *const U = (gmem<double> *)V.u, *const Vv = (gmem<double> *)V.v,
+                 *const W = (gmem<double> *)V.w;
+    gmem<double> *const F0 = (gmem<double> *)F.f[0], *const F1 = (gmem<double> *)F.f[1];
+    gmem<T> *const R0 = to_fine ? (gmem<T> *)levs[b].rhs[0] : nullptr,
+                  *const R1 = to_fine ? (gmem<T> *)levs[b].rhs[1] : nullptr;
+    const size_t pu = (size_t)(ni + 1), plane = (size_t)ni * nj;
+    // u = us - dta*(ph - pl)/h, over the face density of an L_LSM handle
+    auto corr = [&](double us, double pl, double ph, double h, double dl, double dh) -> double {
+      if (LSM) return us - dta * (ph - pl) / h / (0.5 * (dl + dh));
+      return us - dta * (ph - pl) / h;
+    };
+    for (int t = (int)blockIdx.x; t < ntx * nty * ntz; t += (int)gridDim.x) {
+      const int tx = t % ntx, tr = t / ntx, ty = tr % nty, tz = tr / nty;
+      const int l = tx * lp + rl, j = ty * rows + (tid >> lg);
+      const int k0 = tz * kb, k1 = min(k0 + kb, nk);
+      const int a = 2 * l;  // cells a, a+1
+      const bool ok = a < ni && j < nj, okb = a + 1 < ni && j < nj;
+      // lanes outside the block read a valid entry and store nothing
+      const int lc = min(l, ne - 1), jc = min(j, nj - 1), ac = 2 * lc;
+      const int bo = EVEN ? 1 : min(1, ni - 1 - ac);  // cell a+1, or a again past an odd row's end
+      // pressures of the lane's two cells in row y of an array pair (A0, A1)
+      // with nr rows per plane: the even cell has colour (y + z) & 1
+      auto pair = [&](src A0, src A1, int nr, int y, int z) -> d2 {
+        const unsigned o = ((unsigned)z * (unsigned)nr + (unsigned)y) * (unsigned)H + (unsigned)lc;
+        const double e0 = A0[o], e1 = A1[o];
+        return ((y + z) & 1) ? d2{e1, e0} : d2{e0, e1};
+      };
+      auto ld = [&](src q, size_t o) -> d2 {
+        if (EVEN) {
+          const d2u v = *(const gmem<d2u> *)(q + o);
+          return d2{v.x, v.y};
+        }
+        return d2{q[o], q[o + bo]};
+      };
+      auto st = [&](gmem<double> *q, size_t o, d2 v) {
+        if (okb)
+          *(gmem<d2u> *)(q + o) = d2u{v.x, v.y};
+        else if (ok)
+          q[o] = v.x;
+      };
+      // (L_LSM) the lane's two densities in row y, plane z
+      auto dens2 = [&](int y, int z) -> d2 {
+        if (!LSM) return d2{1.0, 1.0};
+        return ld((src)F.dens, (size_t)z * plane + (size_t)y * ni + ac);
+      };
+      auto dens1 = [&](int x, int y, int z) -> double {
+        return LSM ? ((src)F.dens)[(size_t)z * plane + (size_t)y * ni + x] : 1.0;
+      };
+      // rows and u* of the y faces: the image row across an open face
+      const int qs = across(2), qn = across(3);
+      const bool at_s = jc == 0, at_n = jc == nj - 1;
+      const int njs = fine[qs].nj;
+      const src S0 = at_s && open_s ? (src)fine[qs].p[0] : P0,
+                S1 = at_s && open_s ? (src)fine[qs].p[1] : P1;
+      const src N0 = at_n && open_n ? (src)fine[qn].p[0] : P0,
+                N1 = at_n && open_n ? (src)fine[qn].p[1] : P1;
+      const int ys = at_s ? (open_s ? njs - 1 : 0) : jc - 1, nrs = at_s && open_s ? njs : nj;
+      const int yn = at_n ? (open_n ? 0 : jc) : jc + 1, nrn = at_n && open_n ? fine[qn].nj : nj;
+      const bool nbr_s = connected && at_s && open_s;
+      const src VSs = nbr_s ? (src)tab[qs].vs : VS;
+      const int fs = nbr_s ? njs : jc, nfs = (nbr_s ? njs : nj) + 1;
+      const bool up_s = !at_s || open_s, up_n = !at_n || open_n;
+      // x edges: the first lane's west neighbour, the last lane's east one
+      const bool edge_w = rl == 0, edge_e = rl == lp - 1 || ac + 2 >= ni;
+      const bool at_w = ac == 0, at_e = ac + 2 >= ni;
+      const int qw_ = across(0), qe = across(1);
+      const int niw = fine[qw_].ni;
+      const int xw = at_w ? (open_w ? niw - 1 : 0) : ac - 1;
+      const int xe = at_e ? (open_e ? 0 : ni - 1) : ac + 2;
+      const int Hw = at_w && open_w ? fine[qw_].H : H, He = at_e && open_e ? fine[qe].H : H;
+      const bool img_w = at_w && open_w, img_e = at_e && open_e;
+      const src W0 = img_w ? (src)fine[qw_].p[0] : P0, W1 = img_w ? (src)fine[qw_].p[1] : P1;
+      const src E0 = img_e ? (src)fine[qe].p[0] : P0, E1 = img_e ? (src)fine[qe].p[1] : P1;
+      const bool nbr_w = connected && img_w;
+      const bool up_w = !at_w || open_w, up_e = !at_e || open_e;
+
+      d2 pc = pair(P0, P1, nj, jc, k0), wb;
+      d2 dc = dens2(jc, k0);
+      {  // bottom faces of the first plane (k0, open_b: uniform)
+        const size_t o = (size_t)jc * ni + ac;
+        const int qb = across(4);
+        wb = connected && k0 == 0 && open_b ? ld((src)tab[qb].ws, (size_t)fine[qb].nk * plane + o)
+                                            : ld(WS, (size_t)k0 * plane + o);
+        if (k0 > 0 || open_b) {
+          const int zb = k0 > 0 ? k0 - 1 : fine[qb].nk - 1;
+          const d2 pm = k0 > 0 ? pair(P0, P1, nj, jc, zb)
+                               : pair((src)fine[qb].p[0], (src)fine[qb].p[1], nj, jc, zb);
+          const d2 dm = dens2(jc, zb);
+          wb.x = corr(wb.x, pm.x, pc.x, dz, dm.x, dc.x);
+          wb.y = corr(wb.y, pm.y, pc.y, dz, dm.y, dc.y);
+        }
+      }
+      for (int k = k0; k < k1; ++k) {
+        const size_t qu = ((size_t)k * nj + jc) * pu + ac;
+        const size_t qv = ((size_t)k * (nj + 1) + jc) * ni + ac;
+        const size_t qw = (size_t)k * plane + (size_t)jc * ni + ac;
+        // loads of the plane
+        const d2u us = *(const gmem<d2u> *)(US + qu);  // faces a, a+1 (a+1 <= ni)
+        d2 vs = ld(VSs, ((size_t)k * nfs + fs) * ni + ac), vn = ld(VS, qv + ni);
+        d2 wt = ld(WS, qw + plane);
+        const d2 ps = pair(S0, S1, nrs, ys, k), pn = pair(N0, N1, nrn, yn, k);
+        const int qt = across(5);
+        const bool top = k + 1 >= nk;
+        const d2 pp = !top || !open_t
+                          ? pair(P0, P1, nj, jc, min(k + 1, nk - 1))
+                          : pair((src)fine[qt].p[0], (src)fine[qt].p[1], nj, jc, 0);
+        double pw = 0.0, pe = 0.0, u0n = 0.0, u2 = 0.0;
+        if (edge_w) {
+          const unsigned o = ((unsigned)k * nj + jc) * (unsigned)Hw + (unsigned)(xw >> 1);
+          pw = ((xw + jc + k) & 1) ? W1[o] : W0[o];
+          if (nbr_w) u0n = ((src)tab[qw_].us)[((size_t)k * nj + jc) * (niw + 1) + niw];
+        }
+        if (edge_e) {
+          const unsigned o = ((unsigned)k * nj + jc) * (unsigned)He + (unsigned)(xe >> 1);
+          pe = ((xe + jc + k) & 1) ? E1[o] : E0[o];
+          if (EVEN || ac + 2 <= ni) u2 = US[qu + 2];
+        }
+        d2 ds, dn, dp;
+        double dw = 1.0, de = 1.0;
+        if (LSM) {
+          ds = dens2(ys, k);
+          dn = dens2(yn, k);
+          dp = dens2(jc, top ? 0 : k + 1);
+          dw = dens1(at_w ? ni - 1 : ac - 1, jc, k);
+          de = dens1(at_e ? 0 : ac + 2, jc, k);
+        }
+        // x faces a, a+1, a+2
+        const double lf = wave_shift(pc.y, 1);
+        if (!edge_w) pw = lf;
+        double u0 = nbr_w ? u0n : us.x, u1 = us.y;
+        if (up_w) u0 = corr(u0, pw, pc.x, dx, dw, dc.x);
+        if (EVEN || bo)
+          u1 = corr(u1, pc.x, pc.y, dx, dc.x, dc.y);
+        else if (open_e)  // an odd row's last cell
+          u1 = corr(u1, pc.x, pe, dx, dc.x, de);
+        const double rt = wave_shift(u0, 0);
+        if (edge_e) {
+          if (up_e) u2 = corr(u2, pc.y, pe, dx, dc.y, de);
+        } else {
+          u2 = rt;
+        }
+        st(U, qu, d2{u0, u1});
+        if (!EVEN && ok && !okb) U[qu + 1] = u1;
+        if (okb && a + 2 == ni) U[qu + 2] = u2;
+        // y faces jc (south) and jc+1 (north)
+        if (up_s) {
+          vs.x = corr(vs.x, ps.x, pc.x, dy, ds.x, dc.x);
+          vs.y = corr(vs.y, ps.y, pc.y, dy, ds.y, dc.y);
+        }
+        if (up_n) {
+          vn.x = corr(vn.x, pc.x, pn.x, dy, dc.x, dn.x);
+          vn.y = corr(vn.y, pc.y, pn.y, dy, dc.y, dn.y);
+        }
+        st(Vv, qv, vs);
+        if (j == nj - 1) st(Vv, qv + ni, vn);
+        // z faces k (bottom, carried) and k+1 (top)
+        if (!top || open_t) {
+          wt.x = corr(wt.x, pc.x, pp.x, dz, dc.x, dp.x);
+          wt.y = corr(wt.y, pc.y, pp.y, dz, dc.y, dp.y);
+        }
+        st(W, qw, wb);
+        if (top) st(W, qw + plane, wt);
+        if (calmas) {
+          const double fa = (u1 - u0) / dx + (vn.x - vs.x) / dy + (wt.x - wb.x) / dz;
+          const double fb = (u2 - u1) / dx + (vn.y - vs.y) / dy + (wt.y - wb.y) / dz;
+          // L_LSM: sup = div(u) dx dy dz / dt (press.for:53-55)
+          const double ra = LSM ? fa * dx * dy * dz / dt : fa / dt;
+          const double rb = LSM ? fb * dx * dy * dz / dt : fb / dt;
+          if (to_fine) {
+            const unsigned o = ((unsigned)k * nj + jc) * (unsigned)H + (unsigned)lc;
+            const bool odd = (jc + k) & 1;
+            if (ok) {
+              (odd ? F1 : F0)[o] = ra;
+              (odd ? R1 : R0)[o] = (T)ra;
+            }
+            if (okb) {
+              (odd ? F0 : F1)[o] = rb;
+              (odd ? R0 : R1)[o] = (T)rb;
+            }
+          } else if (V.su) {
+            st((gmem<double> *)V.su, qw, d2{ra, rb});
+          }
+          if (ok) am = fmax(am, fabs(fa * dx * dy * dz));
+          if (okb) am = fmax(am, fabs(fb * dx * dy * dz));
+        }
+        wb = wt;
+        pc = pp;
+        dc = dp;
+      }
+    }
+  }
+  if (!partials) return;
+  block_reduce(ss, am);
+  if (threadIdx.x == 0)
+    partials[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = RedPartial{0.0, am};
+}
+
 // max of the `amax` fields of n partials into *out (one workgroup; a max is
 // exact in any order)
 __global__ void __launch_bounds__(256)
@@ -3997,6 +4251,19 @@ void launch_unpack_fine_padded(hipStream_t s, const FineDev *fine, int b, double
   const size_t n = (size_t)(ni + 2) * (nj + 2) * (nk + 2);
   hipLaunchKernelGGL(k_unpack_fine_padded, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
                      fine, b, dst);
+}
+
+void launch_project(hipStream_t s, const ProjLaunch &a, const FineDev *fine, const LevelDev *levs,
+                    const int *active, const VelDev *tab, const ProjDt *dtab, const VelDev &one,
+                    const ProjDt &dt_one, int b0, int nblocks, RedPartial *partials) {
+  auto k = a.even ? (a.lsm   ? k_project<double, true, true>
+                     : a.f32 ? k_project<float, false, true>
+                             : k_project<double, false, true>)
+                  : (a.lsm   ? k_project<double, true, false>
+                     : a.f32 ? k_project<float, false, false>
+                             : k_project<double, false, false>);
+  hipLaunchKernelGGL(k, dim3(a.groups, nblocks), dim3(NTHREADS), 0, s, fine, levs, active, tab,
+                     dtab, one, dt_one, b0, a.kb, a.connected, a.to_fine, a.calmas, partials);
 }
 
 int launch_calmas(hipStream_t s, const FineDev *fd, const double *u, const double *v,

@@ -307,6 +307,20 @@ struct h3dmg_handle {
   int differencing = 1;
   double vel_dta = 0.0, vel_dt = 0.0;  // dt*alfapr and dt of the captured step
   bool vel_ready = false;
+  // k_project's launch shape, and the block pointers and time step it reads
+  // (VelDev[nb], then ProjDt): in device memory, so that the captured step
+  // stays valid when a caller brings other arrays or another dt
+  int proj_kb = 1, proj_groups = 1;
+  VelDev *d_vel = nullptr;
+  ProjDt *d_projdt = nullptr;
+  RedPartial *d_pparts = nullptr;  // proj_groups partials per block
+  int *d_pp_begin = nullptr;
+  // an input array of the velocity loop overlaps an output one: per-axis
+  // launches (k_calvel*, k_calmas), which read each face before they write it
+  bool vel_overlap = false;
+  // the level-1 rhs arrays hold su (f) of every enabled block: the velocity
+  // step's V-cycle starts without copying it there
+  bool rhs_is_f = false;
   hipGraph_t vgraph = nullptr;
   hipGraphExec_t vgexec = nullptr;
 
@@ -1235,6 +1249,29 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
   off = align_up(off + (size_t)h->proj_begin[nblocks] * sizeof(RedPartial), 256);
   const size_t pb_off = off;
   off = align_up(off + (nblocks + 1) * sizeof(int), 256);
+  // k_project: as many planes per tile (at most 8) as leave ~1024 tiles over
+  // all blocks, and one workgroup per tile up to PROJ_MAX_GROUPS per block.
+  // Deeper tiles read their bottom plane of p and w* less often, fewer tiles
+  // leave CUs idle: 128x128x96 and 64 blocks of 64x8x64 take 30.2 and 37.0 us
+  // with ~2048 tiles, 28.1 and 34.2 with ~1024, 28.9 and 35.7 with ~512; 192^3
+  // 113 us with 8 planes, 131 with 16
+  {
+    long tiles = 0;
+    for (int b = 0; b < nblocks; ++b)
+      tiles += project_tiles(blocks[b].ni, blocks[b].nj, blocks[b].nk, 1);
+    h->proj_kb = (int)std::min<long>(8, std::max<long>(1, tiles / 1024));
+    h->proj_groups = 1;
+    for (int b = 0; b < nblocks; ++b)
+      h->proj_groups = std::max(
+          h->proj_groups, project_tiles(blocks[b].ni, blocks[b].nj, blocks[b].nk, h->proj_kb));
+    h->proj_groups = std::min(h->proj_groups, PROJ_MAX_GROUPS);
+  }
+  const size_t vel_tab_off = off;
+  off = align_up(off + nblocks * sizeof(VelDev) + sizeof(ProjDt), 256);
+  const size_t pparts_off = off;
+  off = align_up(off + (size_t)nblocks * h->proj_groups * sizeof(RedPartial), 256);
+  const size_t ppb_off = off;
+  off = align_up(off + (nblocks + 1) * sizeof(int), 256);
   const size_t eptr_off = off;
   off = align_up(off + (size_t)nblocks * 8 * sizeof(double *), 256);
 
@@ -1296,6 +1333,9 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
     F.cx = L.cx;
     F.cy = L.cy;
     F.cz = L.cz;
+    F.dx = h->blk[b].spec.dx;
+    F.dy = h->blk[b].spec.dy;
+    F.dz = h->blk[b].spec.dz;
     F.p[0] = (double *)(R[b] + foff[4 * b + 0]);
     F.p[1] = (double *)(R[b] + foff[4 * b + 1]);
     F.f[0] = (double *)(R[b] + foff[4 * b + 2]);
@@ -1330,6 +1370,15 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
   h->d_proj = (RedPartial *)(A + proj_off);
   h->d_proj_begin = (int *)(A + pb_off);
   put(pb_off, h->proj_begin.data(), (nblocks + 1) * sizeof(int));
+  h->d_vel = (VelDev *)(A + vel_tab_off);
+  h->d_projdt = (ProjDt *)(A + vel_tab_off + nblocks * sizeof(VelDev));
+  h->d_pparts = (RedPartial *)(A + pparts_off);
+  h->d_pp_begin = (int *)(A + ppb_off);
+  {
+    std::vector<int> pp_begin(nblocks + 1);
+    for (int b = 0; b <= nblocks; ++b) pp_begin[b] = b * h->proj_groups;
+    put(ppb_off, pp_begin.data(), (nblocks + 1) * sizeof(int));
+  }
   h->vel.assign(nblocks, {});
   if (h->pool) {
     // a run of the pool's pinned statistics entries
@@ -1718,7 +1767,37 @@ void enqueue_calmas(h3dmg_handle *h, int b) {
                   B.spec.dy, B.spec.dz, h->d_proj + h->proj_begin[b], cells);
 }
 
+// k_project over every enabled block from the device tables; with
+// differencing = 2 only the faces, then the 4th-order calmas per block.
+ProjLaunch project_shape(const h3dmg_handle *h) {
+  ProjLaunch a{};
+  a.groups = h->proj_groups;
+  a.kb = h->proj_kb;
+  a.connected = h->connected;
+  a.lsm = h->lsm;
+  a.f32 = is_mixed(h);
+  a.even = 1;
+  for (const BlockInfo &B : h->blk) a.even = a.even && B.spec.ni % 2 == 0;
+  a.calmas = 1;
+  return a;
+}
+
 void enqueue_project(h3dmg_handle *h) {
+  if (!h->vel_overlap) {
+    ProjLaunch a = project_shape(h);
+    a.to_fine = 1;
+    a.calmas = h->differencing == 2 ? 0 : 1;
+    launch_project(h->stream, a, h->d_fine, h->d_levs, h->d_active, h->d_vel, h->d_projdt,
+                   VelDev{}, ProjDt{}, 0, h->nb, a.calmas ? h->d_pparts : nullptr);
+    if (a.calmas) {
+      launch_finalize(h->stream, h->d_pp_begin, h->nb, h->d_pparts, h->d_stats);
+      return;
+    }
+    for (int b = 0; b < h->nb; ++b)
+      if (h->blk[b].enabled) enqueue_calmas(h, b);
+    launch_finalize(h->stream, h->d_proj_begin, h->nb, h->d_proj, h->d_stats);
+    return;
+  }
   if (h->connected) {
     // calvel on the faces each block computes, then exchange(1..3) of the
     // near faces from the blocks across them (press.for:77-144), then calmas
@@ -1775,17 +1854,22 @@ double projected_rmax(const h3dmg_handle *h) {
   return m;
 }
 
-// One iteration of newsolv_mg's loop (newsolv_mg.for:24-55): mgkcyc from su
-// (level-1 rhs <- f, pp = 0), p = p + (pp - 0), calvel + calmas.
-void enqueue_velocity_step(h3dmg_handle *h) {
-  const bool f64 = !is_mixed(h);
-  const TileSet &ft = h->fine_tiles, &ut = h->update_tiles;
-  if (f64)
-    launch_residual<double>(h->stream, ft.d, ft.n(), ft.depth, h->d_fine, h->d_levs, h->d_active,
-                            h->d_partials, 0);
-  else
+// level-1 rhs <- f of the active blocks (the norm's partials are not read)
+void enqueue_rhs_from_f(h3dmg_handle *h) {
+  const TileSet &ft = h->fine_tiles;
+  if (is_mixed(h))
     launch_residual<float>(h->stream, ft.d, ft.n(), ft.depth, h->d_fine, h->d_levs, h->d_active,
                            h->d_partials, 0);
+  else
+    launch_residual<double>(h->stream, ft.d, ft.n(), ft.depth, h->d_fine, h->d_levs, h->d_active,
+                            h->d_partials, 0);
+}
+
+// One iteration of newsolv_mg's loop (newsolv_mg.for:24-55): mgkcyc from su
+// (in the level-1 rhs already, pp = 0), p = p + (pp - 0), calvel + calmas.
+void enqueue_velocity_step(h3dmg_handle *h) {
+  const bool f64 = !is_mixed(h);
+  const TileSet &ut = h->update_tiles;
   enqueue_vcycle(h);
   if (f64)
     launch_update<double>(h->stream, ut.d, ut.n(), h->d_fine, h->d_levs, h->d_active, h->pp_buf);
@@ -1795,6 +1879,9 @@ void enqueue_velocity_step(h3dmg_handle *h) {
 }
 
 h3dmg_status run_velocity_step(h3dmg_handle *h) {
+  if (!h->rhs_is_f) enqueue_rhs_from_f(h);
+  // k_project leaves su in f and in the level-1 rhs, calmas on its own in f
+  h->rhs_is_f = !h->vel_overlap && h->differencing == 1;
   if (h->prm.use_graph) {
     if (!h->vgexec) {
       std::lock_guard<std::mutex> lock(g_device_mutex);
@@ -1811,6 +1898,31 @@ h3dmg_status run_velocity_step(h3dmg_handle *h) {
   }
   HIP_TRY(hipGetLastError());
   return H3DMG_OK;
+}
+
+// whether ranges of `in` and `out` (address, bytes) overlap
+bool ranges_overlap(std::vector<std::pair<const char *, size_t>> in,
+                    std::vector<std::pair<const char *, size_t>> out) {
+  std::sort(in.begin(), in.end());
+  std::sort(out.begin(), out.end());
+  size_t q = 0;
+  const char *reach = nullptr;  // furthest end of the outputs that start before the input's end
+  for (const auto &x : in) {
+    const char *end = x.first + x.second;
+    while (q < out.size() && out[q].first < end) {
+      reach = std::max(reach, out[q].first + out[q].second);
+      ++q;
+    }
+    if (reach && reach > x.first) return true;
+  }
+  return false;
+}
+
+typedef std::vector<std::pair<const char *, size_t>> Ranges;
+void face_ranges(const h3dmg_block &S, const double *const a[3], Ranges &r) {
+  const size_t ni = S.ni, nj = S.nj, nk = S.nk;
+  const size_t n[3] = {(ni + 1) * nj * nk, ni * (nj + 1) * nk, ni * nj * (nk + 1)};
+  for (int q = 0; q < 3; ++q) r.push_back({(const char *)a[q], n[q] * sizeof(double)});
 }
 
 // One outer iteration: V-cycle on the current level-1 rhs, p += pp, new
@@ -2152,6 +2264,7 @@ h3dmg_status h3dmg_set_rhs_device(h3dmg_handle *h, int b, const double *d_su) {
   if (st) return st;
   if (!d_su) return fail(H3DMG_ERR_ARG, "null rhs");
   const FineDev &F = h->fine[b];
+  h->rhs_is_f = false;
   launch_pack_fine(h->stream, h->d_fine + b, 1, d_su, F.ni, F.nj, F.nk);
   // ||f||: residual with use_p = 0 over this block only
   std::vector<int> act(h->nb, 0);
@@ -2445,6 +2558,7 @@ h3dmg_status h3dmg_solve(h3dmg_handle *h, double *hist, int hist_cap, int *ncycl
     B.cycles = 0;
     B.rel = 0.0;
   }
+  h->rhs_is_f = false;
   enqueue_update_residual(h, false);
   HIP_TRY(hipGetLastError());
   st = read_stats(h);
@@ -2632,6 +2746,7 @@ h3dmg_status h3dmg_solve_begin(h3dmg_handle *h, const int *blocks, int n) {
   // (the next V-cycle's right-hand sides) stay as they are
   for (int b = 0; b < h->nb; ++b) h->active[b] = pick[b];
   if ((st = push_active(h))) return st;
+  h->rhs_is_f = false;
   enqueue_update_residual(h, false);
   HIP_TRY(hipGetLastError());
   if ((st = read_stats(h))) return st;
@@ -2657,6 +2772,7 @@ h3dmg_status h3dmg_solve_step(h3dmg_handle *h, int *nrunning) {
     count += h->active[b];
   }
   if (count) {
+    h->rhs_is_f = false;
     if ((st = push_active(h))) return st;
     if ((st = run_cycle(h))) return st;
     if ((st = read_stats(h))) return st;
@@ -2676,6 +2792,32 @@ h3dmg_status h3dmg_solve_step(h3dmg_handle *h, int *nrunning) {
   return H3DMG_OK;
 }
 
+namespace {
+// an output (su included) of one block's projection overlaps an input: the
+// per-axis launches then read each face before they write it
+bool project_one_overlaps(const h3dmg_handle *h, int b, const VelDev &V) {
+  const h3dmg_block &S = h->blk[b].spec;
+  Ranges in, out;
+  const double *const i3[3] = {V.us, V.vs, V.ws}, *const o3[3] = {V.u, V.v, V.w};
+  face_ranges(S, i3, in);
+  face_ranges(S, o3, out);
+  if (V.su) out.push_back({(const char *)V.su, (size_t)S.ni * S.nj * S.nk * sizeof(double)});
+  return ranges_overlap(in, out);
+}
+
+// calvel axis by axis, then calmas, of one block; returns the partials' count
+int enqueue_project_axes(h3dmg_handle *h, int b, const VelDev &V, double dta, RedPartial *parts) {
+  const h3dmg_block &S = h->blk[b].spec;
+  const size_t ni = S.ni, nj = S.nj, nk = S.nk;
+  const FineDev *fd = h->d_fine + b;
+  launch_calvel(h->stream, fd, 0, V.us, V.u, dta, S.dx, (ni + 1) * nj * nk);
+  launch_calvel(h->stream, fd, 1, V.vs, V.v, dta, S.dy, ni * (nj + 1) * nk);
+  launch_calvel(h->stream, fd, 2, V.ws, V.w, dta, S.dz, ni * nj * (nk + 1));
+  return launch_calmas(h->stream, fd, V.u, V.v, V.w, V.su, 0, h->prm.dt, S.dx, S.dy, S.dz, parts,
+                       ni * nj * nk);
+}
+}  // namespace
+
 h3dmg_status h3dmg_project_device(h3dmg_handle *h, int b, const double *d_ustar,
                                   const double *d_vstar, const double *d_wstar, double *d_u,
                                   double *d_v, double *d_w, double *d_su, double alfapr,
@@ -2692,18 +2834,20 @@ h3dmg_status h3dmg_project_device(h3dmg_handle *h, int b, const double *d_ustar,
     return fail(H3DMG_ERR_UNSUPPORTED,
                 "differencing = 2: the projection of device arrays has no outer faces (use the "
                 "velocity loop with h3dmg_set_velocity)");
-  const FineDev &F = h->fine[b];
-  const BlockInfo &B = h->blk[b];
   const double dt = h->prm.dt;
   if (!(dt > 0)) return fail(H3DMG_ERR_ARG, "projection needs params.dt > 0");
-  const double dta = dt * alfapr;
-  const size_t ni = F.ni, nj = F.nj, nk = F.nk;
-  launch_calvel(h->stream, h->d_fine + b, 0, d_ustar, d_u, dta, B.spec.dx, (ni + 1) * nj * nk);
-  launch_calvel(h->stream, h->d_fine + b, 1, d_vstar, d_v, dta, B.spec.dy, ni * (nj + 1) * nk);
-  launch_calvel(h->stream, h->d_fine + b, 2, d_wstar, d_w, dta, B.spec.dz, ni * nj * (nk + 1));
   RedPartial *parts = h->d_proj + h->proj_begin[b];
-  const int groups = launch_calmas(h->stream, h->d_fine + b, d_u, d_v, d_w, d_su, 0, dt, B.spec.dx,
-                                   B.spec.dy, B.spec.dz, parts, ni * nj * nk);
+  const VelDev V{d_ustar, d_vstar, d_wstar, d_u, d_v, d_w, d_su};
+  int groups = 0;
+  if (project_one_overlaps(h, b, V)) {
+    groups = enqueue_project_axes(h, b, V, dt * alfapr, parts);
+  } else {
+    parts = h->d_pparts + (size_t)b * h->proj_groups;
+    groups = h->proj_groups;
+    const ProjLaunch a = project_shape(h);
+    launch_project(h->stream, a, h->d_fine, h->d_levs, nullptr, nullptr, nullptr, V,
+                   ProjDt{dt * alfapr, dt}, b, 1, parts);
+  }
   HIP_TRY(hipGetLastError());
   if (rmax) {
     std::vector<RedPartial> part(groups);
@@ -2711,7 +2855,7 @@ h3dmg_status h3dmg_project_device(h3dmg_handle *h, int b, const double *d_ustar,
                            hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(hipStreamSynchronize(h->stream));
     double m = 0.0;
-    for (const RedPartial &r : part) m = std::max(m, r.amax);
+    for (const RedPartial &q : part) m = std::max(m, q.amax);
     *rmax = m;
   } else {
     HIP_TRY(hipStreamSynchronize(h->stream));
@@ -2735,26 +2879,27 @@ h3dmg_status h3dmg_project_device_noalloc(h3dmg_handle *h, int b, const double *
     return fail(H3DMG_ERR_UNSUPPORTED,
                 "differencing = 2: the projection of device arrays has no outer faces (use the "
                 "velocity loop with h3dmg_set_velocity)");
-  const FineDev &F = h->fine[b];
-  const BlockInfo &B = h->blk[b];
   const double dt = h->prm.dt;
   if (!(dt > 0)) return fail(H3DMG_ERR_ARG, "projection needs params.dt > 0");
-  const size_t ni = F.ni, nj = F.nj, nk = F.nk;
-  const int groups = calmas_groups(ni * nj * nk);
-  if (groups > NOALLOC_PARTIALS)
-    return fail(H3DMG_ERR_ARG, "block %d: %d calmas partials exceed the %d the scratch holds", b,
-                groups, NOALLOC_PARTIALS);
   RedPartial *parts = nullptr;
   st = scratch_on(h->device, &parts);
   if (st) return st;
-  const double dta = dt * alfapr;
-  launch_calvel(h->stream, h->d_fine + b, 0, d_ustar, d_u, dta, B.spec.dx, (ni + 1) * nj * nk);
-  launch_calvel(h->stream, h->d_fine + b, 1, d_vstar, d_v, dta, B.spec.dy, ni * (nj + 1) * nk);
-  launch_calvel(h->stream, h->d_fine + b, 2, d_wstar, d_w, dta, B.spec.dz, ni * nj * (nk + 1));
   // every one of the `groups` partials is written before it is read: nothing
   // in the scratch needs clearing
-  launch_calmas(h->stream, h->d_fine + b, d_u, d_v, d_w, d_su, 0, dt, B.spec.dx, B.spec.dy,
-                B.spec.dz, parts, ni * nj * nk);
+  const VelDev V{d_ustar, d_vstar, d_wstar, d_u, d_v, d_w, d_su};
+  int groups = h->proj_groups;
+  static_assert(PROJ_MAX_GROUPS <= NOALLOC_PARTIALS, "k_project's partials fit the scratch");
+  if (project_one_overlaps(h, b, V)) {
+    const h3dmg_block &S = h->blk[b].spec;
+    groups = calmas_groups((size_t)S.ni * S.nj * S.nk);
+    if (groups > NOALLOC_PARTIALS)
+      return fail(H3DMG_ERR_ARG, "block %d: %d calmas partials exceed the %d the scratch holds", b,
+                  groups, NOALLOC_PARTIALS);
+    enqueue_project_axes(h, b, V, dt * alfapr, parts);
+  } else {
+    launch_project(h->stream, project_shape(h), h->d_fine, h->d_levs, nullptr, nullptr, nullptr, V,
+                   ProjDt{dt * alfapr, dt}, b, 1, parts);
+  }
   if (d_rmax) launch_partials_max(h->stream, parts, groups, d_rmax);
   HIP_TRY(hipGetLastError());
   return H3DMG_OK;
@@ -2982,9 +3127,6 @@ h3dmg_status enable_lsm(h3dmg_handle *h) {
   for (int b = 0; b < h->nb; ++b) {
     FineDev &F = h->fine[b];
     F.dens = h->lsm_store + h->lsm_dens[h->blk[b].desc[1]];
-    F.dx = h->blk[b].spec.dx;
-    F.dy = h->blk[b].spec.dy;
-    F.dz = h->blk[b].spec.dz;
   }
   HIP_TRY(hipMemcpy(h->d_fine, h->fine.data(), h->nb * sizeof(FineDev), hipMemcpyHostToDevice));
   h->lsm_set.assign(h->nb, 0);
@@ -3071,9 +3213,38 @@ h3dmg_status h3dmg_set_differencing(h3dmg_handle *h, int differencing) {
 h3dmg_status h3dmg_set_dt(h3dmg_handle *h, double dt) {
   if (!h) return fail(H3DMG_ERR_ARG, "null handle");
   if (!(dt > 0)) return fail(H3DMG_ERR_ARG, "dt must be > 0");
-  h->prm.dt = dt;  // the velocity step's graph is re-captured on the next begin
+  h->prm.dt = dt;  // the velocity step reads it from the next begin on
   return H3DMG_OK;
 }
+
+namespace {
+// k_project reads a face's u* while other workgroups write u, v, w: whether
+// a caller's arrays rule that out (u given as its own u*, say)
+bool velocity_overlap(const h3dmg_handle *h) {
+  Ranges in, out;
+  for (int b = 0; b < h->nb; ++b) {
+    if (!h->blk[b].enabled) continue;
+    const h3dmg_handle::VelBlock &V = h->vel[b];
+    const double *const i3[3] = {V.us, V.vs, V.ws}, *const o3[3] = {V.u, V.v, V.w};
+    face_ranges(h->blk[b].spec, i3, in);
+    face_ranges(h->blk[b].spec, o3, out);
+  }
+  return ranges_overlap(in, out);
+}
+
+// the blocks' arrays and the time step to the tables k_project reads
+h3dmg_status push_velocity(h3dmg_handle *h) {
+  std::vector<char> img(h->nb * sizeof(VelDev) + sizeof(ProjDt));
+  VelDev *t = (VelDev *)img.data();
+  for (int b = 0; b < h->nb; ++b) {
+    const h3dmg_handle::VelBlock &V = h->vel[b];
+    t[b] = VelDev{V.us, V.vs, V.ws, V.u, V.v, V.w, nullptr};
+  }
+  *(ProjDt *)(t + h->nb) = ProjDt{h->vel_dta, h->vel_dt};
+  HIP_TRY(hipMemcpyAsync(h->d_vel, img.data(), img.size(), hipMemcpyHostToDevice, h->stream));
+  return H3DMG_OK;
+}
+}  // namespace
 
 h3dmg_status h3dmg_velocity_begin(h3dmg_handle *h, const double *const *d_ustar,
                                   const double *const *d_vstar, const double *const *d_wstar,
@@ -3099,7 +3270,7 @@ h3dmg_status h3dmg_velocity_begin(h3dmg_handle *h, const double *const *d_ustar,
                     "block %d: differencing = 2 needs faces -1 and n+1 (host arrays with off >= 2)",
                     b);
   }
-  bool same = h->vel_ready && h->vel_dta == h->prm.dt * alfapr && h->vel_dt == h->prm.dt;
+  bool same = true;
   for (int b = 0; b < h->nb; ++b) {
     if (!h->blk[b].enabled) continue;
     h3dmg_handle::VelBlock V;
@@ -3119,6 +3290,14 @@ h3dmg_status h3dmg_velocity_begin(h3dmg_handle *h, const double *const *d_ustar,
            O.w == V.w;
     h->vel[b] = V;
   }
+  // the captured step reads the arrays and the time step from device memory,
+  // except in its per-axis form and the 4th-order calmas
+  const bool overlap = velocity_overlap(h);
+  const bool baked = overlap || h->differencing == 2;
+  same = overlap == h->vel_overlap &&
+         (!baked || (same && h->vel_ready && h->vel_dta == h->prm.dt * alfapr &&
+                     h->vel_dt == h->prm.dt));
+  h->vel_overlap = overlap;
   if (!same) {
     std::lock_guard<std::mutex> lock(g_device_mutex);
     HIP_TRY(hipStreamSynchronize(h->stream));
@@ -3133,6 +3312,8 @@ h3dmg_status h3dmg_velocity_begin(h3dmg_handle *h, const double *const *d_ustar,
   reset_active(h);
   h3dmg_status st = push_active(h);
   if (st) return st;
+  if ((st = push_velocity(h))) return st;
+  h->rhs_is_f = !h->vel_overlap && h->differencing == 1;
   enqueue_project(h);
   HIP_TRY(hipGetLastError());
   st = read_stats(h);
@@ -3223,6 +3404,7 @@ h3dmg_status h3dmg_dbg_put(h3dmg_handle *h, int b, int level, int which, const d
   if (level < 1 || level > h->blk[b].L || !d_src) return fail(H3DMG_ERR_ARG, "bad level/ptr");
   const int d = h->blk[b].desc[level];
   const LevelDev &L = h->levs[d];
+  if (level == 1 && which == 1) h->rhs_is_f = false;
   if (h->lev_is64[d])
     launch_pack_level<double>(h->stream, h->d_levs + d, which, 0, d_src, L.ni, L.nj, L.nk);
   else
