@@ -59,6 +59,9 @@ struct LevelDev {
   // (j-, i-, k-lines) and wall-state pair of the line (16), a(p) and
   // 1/(ap - alo*a(p-1)) at every position p of the line
   double *tdma;
+  // workspace of the two-launch line passes (tdma_ws_doubles; the block's,
+  // shared by its levels), or null
+  double *tdma_ws;
 };
 
 // Finest-level FP64 state of one block (pressure, right-hand side).
@@ -224,6 +227,18 @@ void launch_tdma_sweep(hipStream_t s, const Tile *tiles, int ntiles, const Level
 size_t tdma_sweep_lds_bytes(const LevelDev &L, bool pipelined);
 // permits `lds_bytes` of dynamic LDS for the whole-sweep TDMA kernel
 hipError_t tdma_sweep_allow_lds(size_t lds_bytes);
+// One pass of a constant-coefficient level whose axes have at most
+// TDMA_LINES_MAX cells, in two launches: everything known before the pass
+// over the natural tiles `nat`, then the lines, one workgroup per block
+// (`blocks`: Tile::lev).  maxlen: the pass's longest line over the blocks.
+constexpr int TDMA_LINES_MAX = 64;
+bool tdma_lines_fit(const LevelDev &L);
+size_t tdma_ws_doubles(const LevelDev &L);
+size_t tdma_lines_lds(int maxlen);  // dynamic LDS of the lines' launch
+hipError_t tdma_lines_allow_lds();
+void launch_tdma_pass(hipStream_t s, const Tile *nat, int nnat, const Tile *blocks, int nblocks,
+                      const LevelDev *levs, const int *active, int pass, int maxlen, int src,
+                      int zero);
 // fill LevelDev::tdma of every descriptor that has one (32*(ni+nj+nk) doubles)
 void launch_tdma_tables(hipStream_t s, const LevelDev *levs, int ndesc);
 

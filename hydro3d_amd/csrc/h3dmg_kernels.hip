@@ -3951,6 +3951,341 @@ __device__ __forceinline__ void tdma_pass_pipelined(const LevelDev &L, int src, 
   }
 }
 
+// One TDMA pass of a constant-coefficient level whose lines and lanes have at
+// most 64 cells, in two launches.
+//
+// A pass walks the diagonals u + v of its lines in order (line-wise GS); a
+// line needs the solution of its two neighbours on the previous diagonal.
+// The critical path is (lines' diagonals) x (forward + back substitution),
+// and everything else is moved off it:
+//   k_tdma_pre (the whole GPU, a thread per cell): everything known before
+//     the pass -- the rhs, the two not-yet-updated cross terms, ghosts --
+//     as t1 = r - x1*X1 and p3 = x3*X3 per cell, stored diagonal by
+//     diagonal, so that the pass reads whole rows of 16-byte entries;
+//   k_tdma_lines (one workgroup per block): wave 0 is the recurrence, a lane
+//     per line, the line in registers between the two substitutions.  The
+//     updated neighbours are the lane's own last solution and the next lower
+//     lane's, which the back substitution leaves in LDS.  The other waves
+//     load the next diagonal's entries while the forward substitution runs,
+//     put them into LDS during the back substitution, and store the
+//     solutions.
+// Lanes are the axis of the second cross term, steps the axis of the fourth:
+//   pass 0 (j-lines): lanes i, steps k;  ae*E, aw*W, at*T, ab*B
+//   pass 1 (i-lines): lanes j, steps k;  an*N, as*S, at*T, ab*B
+//   pass 2 (k-lines): lanes j, steps i;  an*N, as*S, ae*E, aw*W
+// The reference's left-to-right sum is kept: ((t1 - x2*X2) - p3) - x4*X4.
+// Where the second term's neighbour is a ghost (lane 0), the pass takes it
+// with t1 (the product is the next subtraction anyway); the fourth term's
+// ghost line (step 0) starts as the lane's "last solution".
+//
+// Bound by the dependent chain of FP64 operations, 3 per position forward
+// and 2 back: ~120 cycles per position and diagonal of the ~100 that five
+// dependent operations of 20 cycles take.  A 64^3 pass takes 415 us + 5 us of
+// k_tdma_pre where the one-workgroup pipelined sweep took 1.1 ms, a 32^3 one
+// 100 us where it took 350 us.
+// waves of the workgroup: the recurrence's and the ones that load and store.
+// Four leave each wave a SIMD's whole register file, which 64-cell lines need
+constexpr int tl_waves(int len) { return len > 56 ? 4 : 5; }
+constexpr int TL_ROW = 66;  // doubles per row of solutions in LDS
+
+// a pass's axes: lane, step and line coordinates of cell (i, j, k)
+struct TlAxes {
+  int nl, ns, len;  // lanes, steps, cells per line
+  int w;            // entries per diagonal: min(nl, ns)
+};
+__host__ __device__ inline TlAxes tl_axes(int pass, int ni, int nj, int nk) {
+  TlAxes a;
+  a.nl = pass == 0 ? ni : nj;
+  a.ns = pass == 2 ? ni : nk;
+  a.len = pass == 0 ? nj : pass == 1 ? ni : nk;
+  a.w = a.nl < a.ns ? a.nl : a.ns;
+  return a;
+}
+// workspace of one block (doubles): entries (t1, p3) at ((d*len + p)*w +
+// lane - first lane of d), line-end ghosts (2 per line) at (step*nl + lane),
+// ghost lines of step -1 at (p*nl + lane)
+__host__ __device__ inline size_t tl_entries(const TlAxes &a) {
+  return (size_t)2 * (a.nl + a.ns - 1) * a.len * a.w;
+}
+__host__ __device__ inline size_t tl_ends(const TlAxes &a) { return (size_t)2 * a.nl * a.ns; }
+
+// Tile: natural tiles (TILE_X x TILE_Y cells of one plane)
+template <int PASS>
+__global__ void __launch_bounds__(NTHREADS)
+    k_tdma_pre(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
+               const int *__restrict__ active, int src, int zero) {
+  const Tile t = tiles[blockIdx.x];
+  const LevelDev &L = levs[t.lev];
+  if (!active[L.blk]) return;
+  const int i = t.x0 + (int)threadIdx.x, j = t.y0 + (int)threadIdx.y, k = t.z0;
+  const int ni = L.ni, nj = L.nj, nk = L.nk, H = L.H;
+  if (i >= ni || j >= nj) return;
+  const TlAxes A = tl_axes(PASS, ni, nj, nk);
+  const int u = PASS == 0 ? i : j, v = PASS == 2 ? i : k, p = PASS == 0 ? j : PASS == 1 ? i : k;
+  const bool px = L.per & 1, py = L.per & 2, pz = L.per & 4;
+  const int dst = 1 - src;
+  const bool from_dst = PASS > 0;
+  // a not-yet-updated cross neighbour (interior: dst after the first pass,
+  // else src) or a ghost (its image in src); src reads are 0 when it holds
+  // zeros
+  auto val = [&](int x, int y, int z) -> double {
+    const bool ghost = (unsigned)x >= (unsigned)ni || (unsigned)y >= (unsigned)nj ||
+                       (unsigned)z >= (unsigned)nk;
+    const bool d = from_dst && !ghost;
+    x = image(x, ni, px);
+    y = image(y, nj, py);
+    z = image(z, nk, pz);
+    const double q = gload(L.phi[d ? dst : src][(x + y + z) & 1], cidx(H, nj, x, y, z));
+    return (zero && !d) ? 0.0 : q;
+  };
+  const Coef<double> c = cell_coef<double>(L, i, j, k);
+  const double r = gload(L.rhs[(i + j + k) & 1], cidx(H, nj, i, j, k));
+  double t1, p3;
+  if (PASS == 0) {
+    t1 = r - c.ae * val(i + 1, j, k);
+    p3 = c.at * val(i, j, k + 1);
+    if (u == 0) t1 = t1 - c.aw * val(-1, j, k);
+  } else if (PASS == 1) {
+    t1 = r - c.an * val(i, j + 1, k);
+    p3 = c.at * val(i, j, k + 1);
+    if (u == 0) t1 = t1 - c.as * val(i, -1, k);
+  } else {
+    t1 = r - c.an * val(i, j + 1, k);
+    p3 = c.ae * val(i + 1, j, k);
+    if (u == 0) t1 = t1 - c.as * val(i, -1, k);
+  }
+  gmem<double> *const ws = (gmem<double> *)L.tdma_ws;
+  const int d = u + v, ulo = max(0, d - A.ns + 1);
+  typedef double __attribute__((ext_vector_type(2))) d2;
+  *(gmem<d2> *)(ws + 2 * (((size_t)d * A.len + p) * A.w + (u - ulo))) = d2{t1, p3};
+  gmem<double> *const ends = ws + tl_entries(A), *const first = ends + tl_ends(A);
+  if (p == 0)
+    ends[2 * ((size_t)v * A.nl + u)] =
+        PASS == 0 ? val(i, -1, k) : PASS == 1 ? val(-1, j, k) : val(i, j, -1);
+  if (p == A.len - 1)
+    ends[2 * ((size_t)v * A.nl + u) + 1] =
+        PASS == 0 ? val(i, nj, k) : PASS == 1 ? val(ni, j, k) : val(i, j, nk);
+  if (v == 0) first[(size_t)p * A.nl + u] = PASS == 2 ? val(-1, j, k) : val(i, j, -1);
+}
+
+// LDS and barrier of k_tdma_lines: a barrier waits for the wave's LDS
+// accesses only (the loads and stores of global memory in flight stay so)
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// back substitution of k_tdma_lines: phi(p) = c(p) - a(p)*phi(p+1), the
+// operands a chunk ahead of the chain.  SHORT: any chunk may lie past the
+// line's end, not just part of the last one.
+template <int LEN, bool SHORT>
+__device__ __forceinline__ void tl_back(const double (&cv)[LEN], const lds<double> *a0,
+                                        lds<double> *out, int len, double next) {
+  constexpr int CH = 8;
+  double aq[LEN];
+#pragma unroll
+  for (int q = 0; q < CH; ++q) aq[LEN - CH + q] = a0[LEN - CH + q];
+#pragma unroll
+  for (int p1 = LEN - CH; p1 >= 0; p1 -= CH) {
+    if (p1 >= CH) {
+#pragma unroll
+      for (int q = 0; q < CH; ++q) aq[p1 - CH + q] = a0[p1 - CH + q];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = CH - 1; q >= 0; --q) {
+      const int p = p1 + q;
+      const double x = cv[p] - aq[p] * next;
+      next = (SHORT || p1 == LEN - CH) ? (p < len ? x : next) : x;
+      out[p * TL_ROW] = next;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// Tile::lev = the block's descriptor.  LEN: the longest line the kernel holds
+// in registers (a multiple of the chunk of 8 positions a line's end is looked
+// for at).  Dynamic LDS, doubles: entries 2*LEN*64, solutions LEN*TL_ROW (column 0 zeros,
+// the neighbour below lane 0; lane u in column u+1; the last column takes
+// what lanes whose line has not begun would write),
+// tables a(p) and 1/(ap - alo*a(p-1)) 16*LEN each, line-end ghosts 2*64.
+template <int LEN>
+__global__ void __launch_bounds__(64 * tl_waves(LEN))
+    k_tdma_lines(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
+                 const int *__restrict__ active, int pass, int src) {
+  typedef double __attribute__((ext_vector_type(2))) d2;
+  constexpr int CH = 8, AHEAD = 6, TL_WAVES = tl_waves(LEN);
+  constexpr int ROWS = (LEN + TL_WAVES - 2) / (TL_WAVES - 1);
+  static_assert(LEN % CH == 0 && LEN >= CH, "whole chunks");
+  extern __shared__ __align__(16) double tl_lds[];
+  const Tile t = tiles[blockIdx.x];
+  const LevelDev &L = levs[t.lev];
+  if (!active[L.blk]) return;
+  const int ni = L.ni, nj = L.nj, nk = L.nk, H = L.H, per = L.per;
+  const TlAxes A = tl_axes(pass, ni, nj, nk);
+  const int nl = A.nl, ns = A.ns, len = A.len, w = A.w;
+  const int lane = (int)threadIdx.x & 63,
+            wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  lds<d2> *const tb = (lds<d2> *)tl_lds;                    // [LEN][64]
+  lds<double> *const yb = (lds<double> *)(tl_lds + 2 * LEN * 64);  // [LEN][TL_ROW]
+  lds<double> *const ta = yb + LEN * TL_ROW, *const tr = ta + 16 * LEN;
+  lds<d2> *const eb = (lds<d2> *)(tr + 16 * LEN);        // [64]
+  const gmem<double> *const ws = (const gmem<double> *)L.tdma_ws;
+  const gmem<d2> *const en = (const gmem<d2> *)ws;
+  const gmem<d2> *const ends = (const gmem<d2> *)(ws + tl_entries(A));
+  const gmem<double> *const first = ws + tl_entries(A) + tl_ends(A);
+  const int nd = nl + ns - 1;
+  const bool pl = pass == 0 ? per & 1 : per & 2;           // lane axis periodic
+  const bool ps = pass == 2 ? per & 1 : per & 4;           // step axis
+  const bool pa = pass == 0 ? per & 2 : pass == 1 ? per & 1 : per & 4;  // line axis
+  const double cl = pass == 0 ? L.cx : L.cy, cs = pass == 2 ? L.cx : L.cz;
+  const double ca = pass == 0 ? L.cy : pass == 1 ? L.cx : L.cz;
+  // the pass's tables (both line coordinates' wall states, position)
+  const size_t toff = pass == 0 ? 0 : pass == 1 ? (size_t)32 * nj : (size_t)32 * (nj + ni);
+  for (int q = (int)threadIdx.x; q < 16 * len; q += 64 * TL_WAVES) {
+    const int var = q / len, p = q - var * len;
+    ta[var * LEN + p] = gload(L.tdma, toff + 2 * (size_t)q);
+    tr[var * LEN + p] = gload(L.tdma, toff + 2 * (size_t)q + 1);
+  }
+  // entries and line-end ghosts of a diagonal: rows of the helper waves
+  const int hw = wave - 1;
+  d2 hold[ROWS], hend = d2{0.0, 0.0};
+  auto fetch = [&](int d) {
+    const gmem<d2> *row = en + (size_t)d * len * w;
+#pragma unroll
+    for (int q = 0; q < ROWS; ++q) {
+      const int p = min(hw + q * (TL_WAVES - 1), len - 1);
+      hold[q] = row[(size_t)p * w + min(lane, w - 1)];
+    }
+    if (hw == 0) {
+      const int u = min(lane, nl - 1), v = min(max(d - u, 0), ns - 1);
+      hend = ends[(size_t)v * nl + u];
+    }
+  };
+  auto stage = [&]() {
+#pragma unroll
+    for (int q = 0; q < ROWS; ++q) {
+      const int p = hw + q * (TL_WAVES - 1);
+      if (p < len) tb[p * 64 + lane] = hold[q];
+    }
+    if (hw == 0) eb[lane] = hend;
+  };
+  // the solutions of diagonal d (in yb) to dst
+  gmem<double> *const out0 = (gmem<double> *)L.phi[1 - src][0];
+  gmem<double> *const out1 = (gmem<double> *)L.phi[1 - src][1];
+  auto store = [&](int d) {
+    const int u = lane, v = d - u;
+    if (u < nl && v >= 0 && v < ns) {
+      const int base = pass == 0 ? v * nj * H + (u >> 1) : pass == 1 ? (v * nj + u) * H
+                                                                     : u * H + (v >> 1);
+      const int step = pass == 0 ? H : pass == 1 ? 0 : nj * H;
+#pragma unroll 4
+      for (int q = 0; q < ROWS; ++q) {
+        const int p = hw + q * (TL_WAVES - 1);
+        if (p < len) {
+          const int e = pass == 1 ? base + (p >> 1) : base + p * step;
+          (((u + v + p) & 1) ? out1 : out0)[e] = yb[p * TL_ROW + 1 + lane];
+        }
+      }
+    }
+  };
+
+  // the ghost lines before step 0, and the zeros below lane 0
+  for (int q = (int)threadIdx.x; q < LEN * 64; q += 64 * TL_WAVES) {
+    const int p = q >> 6, u = q & 63;
+    yb[p * TL_ROW + 1 + u] = first[(size_t)min(p, len - 1) * nl + min(u, nl - 1)];
+    if (u == 0) yb[p * TL_ROW] = 0.0;
+  }
+  // each role in its own loop: the registers of one are not held by the
+  // other; both pass the same barriers
+  if (wave != 0) {
+    fetch(0);
+    stage();
+    lds_barrier();
+    for (int d = 0; d < nd; ++d) {
+      if (d + 1 < nd) fetch(d + 1);
+      if (d > 0) store(d - 1);
+      lds_barrier();  // the entries of d are read, the solutions of d-1 stored
+      if (d + 1 < nd) stage();
+      lds_barrier();  // the entries of d+1 and the solutions of d are in LDS
+    }
+    store(nd - 1);
+    return;
+  }
+  __builtin_amdgcn_s_setprio(3);
+  lds_barrier();
+  for (int d = 0; d < nd; ++d) {
+    const int u = lane, v = d - u;
+    const int ulo = max(0, d - ns + 1);
+    const int uc = min(u, nl - 1), vc = min(max(v, 0), ns - 1);
+    const int wl = wall_state(uc, nl, pl), wst = wall_state(vc, ns, ps);
+    // the tables' state pair is (i, k), (j, k) or (i, j)
+    const int var = pass == 2 ? wst | (wl << 2) : wl | (wst << 2);
+    const d2 end = eb[lane];
+    double cv[LEN];
+    // Forward substitution, software-pipelined by hand (the wave issues in
+    // order): while the chain m = alo*c, t = rs - m, c = t/(..) of position p
+    // waits for its operands, the right-hand sides of the next two positions
+    // advance a stage each: x2*X2; t1 - x2*X2, x4*X4; - p3; - x4*X4.  Lanes
+    // with no line on this diagonal work on values nobody reads.
+    {
+      const double x2 = u > 0 ? cl : 0.0, x4 = (v <= 0 && !ps) ? 0.0 : cs;
+      const lds<d2> *const e0 = tb + min(max(u - ulo, 0), w - 1);
+      const lds<double> *const r0 = tr + var * LEN;
+      const lds<double> *const y0 = yb + lane;
+      double c = end.x;
+      d2 en_[LEN];
+      double rr[LEN], X2[LEN], X4[LEN], rs[LEN];
+#pragma unroll
+      for (int p = 0; p < AHEAD; ++p) {
+        en_[p] = e0[p * 64];
+        rr[p] = r0[p];
+        X2[p] = y0[p * TL_ROW];
+        X4[p] = y0[p * TL_ROW + 1];
+      }
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        X4[p] = x4 * X4[p];
+        rs[p] = ((en_[p].x - x2 * X2[p]) - en_[p].y) - X4[p];
+      }
+#pragma unroll
+      for (int p = 0; p < LEN; ++p) {
+        const double m = ((p == 0 && !pa) ? 0.0 : ca) * c;
+        if (p + AHEAD < LEN) {
+          en_[p + AHEAD] = e0[(p + AHEAD) * 64];
+          rr[p + AHEAD] = r0[p + AHEAD];
+          X2[p + AHEAD] = y0[(p + AHEAD) * TL_ROW];
+          X4[p + AHEAD] = y0[(p + AHEAD) * TL_ROW + 1];
+        }
+        if (p + 2 < LEN) X2[p + 2] = x2 * X2[p + 2];
+        if (p + 1 < LEN && p > 0) rs[p + 1] = rs[p + 1] - en_[p + 1].y;
+        __builtin_amdgcn_sched_barrier(0);
+        const double t = rs[p] - m;
+        if (p + 2 < LEN) X4[p + 2] = x4 * X4[p + 2];
+        if (p + 1 < LEN && p > 0) rs[p + 1] = rs[p + 1] - X4[p + 1];
+        __builtin_amdgcn_sched_barrier(0);
+        c = t * rr[p];
+        if (p + 2 < LEN) rs[p + 2] = en_[p + 2].x - X2[p + 2];
+        cv[p] = c;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    lds_barrier();
+    {
+      const lds<double> *const a0 = ta + var * LEN;
+      lds<double> *const out = yb + (v >= 0 ? 1 + lane : TL_ROW - 1);
+      // positions past the line's end pass by: in the last chunk only, unless
+      // the block's lines are shorter than the launch's longest by more
+      if (len > LEN - CH)
+        tl_back<LEN, false>(cv, a0, out, len, end.y);
+      else
+        tl_back<LEN, true>(cv, a0, out, len, end.y);
+    }
+    lds_barrier();
+  }
+}
+
 __global__ void __launch_bounds__(TDMA_SWEEP_THREADS)
     k_tdma_sweep(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
                  const int *__restrict__ active, int src, int zero) {
@@ -4055,6 +4390,52 @@ hipError_t tdma_sweep_allow_lds(size_t lds_bytes) {
   if (e != hipSuccess) return e;
   return hipFuncSetAttribute((const void *)k_tdma_sweep_pipe,
                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+}
+
+size_t tdma_ws_doubles(const LevelDev &L) {
+  size_t most = 0;
+  for (int pass = 0; pass < 3; ++pass) {
+    const TlAxes a = tl_axes(pass, L.ni, L.nj, L.nk);
+    most = std::max(most, tl_entries(a) + tl_ends(a) + (size_t)a.len * a.nl);
+  }
+  return most;
+}
+
+bool tdma_lines_fit(const LevelDev &L) {
+  return std::max(L.ni, std::max(L.nj, L.nk)) <= TDMA_LINES_MAX;
+}
+
+// LEN of the kernel for lines of at most `len` cells
+static int tl_len(int len) { return (len + 7) & ~7; }
+
+size_t tdma_lines_lds(int maxlen) {
+  const size_t len = (size_t)tl_len(maxlen);
+  return sizeof(double) * (2 * len * 64 + len * TL_ROW + 32 * len + 128);
+}
+
+// by tl_len / 8 - 1
+static void (*const tl_kernels[8])(const Tile *, const LevelDev *, const int *, int, int) = {
+    k_tdma_lines<8>,  k_tdma_lines<16>, k_tdma_lines<24>, k_tdma_lines<32>,
+    k_tdma_lines<40>, k_tdma_lines<48>, k_tdma_lines<56>, k_tdma_lines<64>};
+
+hipError_t tdma_lines_allow_lds() {
+  const int most = (int)tdma_lines_lds(TDMA_LINES_MAX);
+  for (auto k : tl_kernels) {
+    hipError_t e = hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       most);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+void launch_tdma_pass(hipStream_t s, const Tile *nat, int nnat, const Tile *blocks, int nblocks,
+                      const LevelDev *levs, const int *active, int pass, int maxlen, int src,
+                      int zero) {
+  if (nblocks <= 0) return;
+  auto pre = pass == 0 ? k_tdma_pre<0> : pass == 1 ? k_tdma_pre<1> : k_tdma_pre<2>;
+  hipLaunchKernelGGL(pre, dim3(nnat), tile_block(), 0, s, nat, levs, active, src, zero);
+  hipLaunchKernelGGL(tl_kernels[tl_len(maxlen) / 8 - 1], dim3(nblocks), dim3(64 * tl_waves(tl_len(maxlen))), tdma_lines_lds(maxlen), s, blocks,
+                     levs, active, pass, src);
 }
 
 void launch_tdma_tables(hipStream_t s, const LevelDev *levs, int ndesc) {

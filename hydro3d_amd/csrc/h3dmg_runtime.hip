@@ -102,6 +102,8 @@ struct TileSet {
   int gs_tile = GS_TILE;             // GS sets: tile edge (GS_TILE or GS_BIG_TILE)
   size_t tdma_lds = 0;  // TDMA sets: > 0 = whole sweeps in one workgroup per block (LDS bytes)
   bool tdma_pipe = false;  // TDMA whole sweeps: the pipelined kernel (constant coefficients)
+  bool tdma_lines = false;  // TDMA passes in two launches (tiles: one per block)
+  int tdma_len[3] = {0, 0, 0};       // their longest line per pass
   OneDesc one;             // every tile on one descriptor: passed to the kernels
   int n() const { return (int)h.size(); }
 };
@@ -503,6 +505,10 @@ void relax_group(h3dmg_handle *h, const TileSet &ts, int nsweep, int &buf, bool 
       for (int d = 0; d + 1 < (int)ts.diag_begin.size(); ++d)
         launch_gs_tiles(h->stream, ts.d + ts.diag_begin[d], ts.diag_begin[d + 1] - ts.diag_begin[d],
                         h->d_levs, h->d_active, buf, zero ? 1 : 0, ts.gs_tile);
+    else if (h->prm.smoother == H3DMG_SMOOTH_TDMA && ts.tdma_lines)
+      for (int pass = 0; pass < 3; ++pass)
+        launch_tdma_pass(h->stream, ts.nat->d, ts.nat->n(), ts.d, ts.n(), h->d_levs, h->d_active,
+                         pass, ts.tdma_len[pass], buf, zero ? 1 : 0);
     else if (h->prm.smoother == H3DMG_SMOOTH_TDMA && ts.tdma_lds)  // small levels
       launch_tdma_sweep(h->stream, ts.d, ts.n(), h->d_levs, h->d_active, buf, zero ? 1 : 0,
                         ts.tdma_lds, ts.tdma_pipe);
@@ -1083,6 +1089,18 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
       tdma_off[d] = boff[L.blk];
       boff[L.blk] = align_up(boff[L.blk] + (size_t)32 * (L.ni + L.nj + L.nk) * 8, 256);
     }
+  // line passes in two launches: one workspace per block, as large as its
+  // largest level that takes them needs
+  std::vector<size_t> tws_off(nblocks, 0), tws_len(nblocks, 0);
+  if (h->prm.smoother == H3DMG_SMOOTH_TDMA)
+    for (int b = 0; b < nblocks; ++b) {
+      for (int g = 1; g <= h->blk[b].L; ++g) {
+        const LevelDev &L = h->levs[h->blk[b].desc[g]];
+        if (tdma_lines_fit(L)) tws_len[b] = std::max(tws_len[b], tdma_ws_doubles(L));
+      }
+      tws_off[b] = boff[b];
+      boff[b] = align_up(boff[b] + tws_len[b] * 8, 256);
+    }
   if (region_bytes) {
     for (int b = 0; b < nblocks; ++b) region_bytes[b] = boff[b];
     return H3DMG_OK;
@@ -1317,6 +1335,7 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
       for (int c = 0; c < 2; ++c) L.phi[bb][c] = R[P.b] + P.phi[bb][c];
     for (int c = 0; c < 2; ++c) L.rhs[c] = R[P.b] + P.rhs[c];
     if (h->prm.smoother == H3DMG_SMOOTH_TDMA) L.tdma = (double *)(R[P.b] + tdma_off[P.d]);
+    if (tws_len[P.b] && tdma_lines_fit(L)) L.tdma_ws = (double *)(R[P.b] + tws_off[P.b]);
   }
   h->fine.resize(nblocks);
   for (int b = 0; b < nblocks; ++b) {
@@ -1467,6 +1486,15 @@ bool tdma_sweep_ok(size_t budget) {
   return ok;
 }
 
+// whether the two-launch line passes may use their dynamic LDS (a process-wide
+// attribute of the kernels: set once, to the most they need)
+bool tdma_lines_ok() {
+  static std::once_flag once;
+  static bool ok = false;
+  std::call_once(once, []() { ok = tdma_lines_allow_lds() == hipSuccess; });
+  return ok;
+}
+
 // whether the 16^3 GS kernel may use its dynamic LDS (the attribute is
 // process-wide: set once, to what the kernel needs)
 bool gs_big_ok() {
@@ -1549,8 +1577,23 @@ h3dmg_status gen_relax(h3dmg_handle *h, int g) {
         }
         ts.diag_begin.push_back(ts.n());
       } else {
+        // every axis of every block within a wavefront's lanes: two launches
+        // per pass (constant coefficients)
+        bool lines = !h->lsm;
+        for (int pass = 0; pass < 3; ++pass) ts.tdma_len[pass] = 0;
+        for (const BlockInfo &B : h->blk)
+          if (member(B)) {
+            const LevelDev &L = h->levs[B.desc[g]];
+            lines = lines && tdma_lines_fit(L);
+            const int len[3] = {L.nj, L.ni, L.nk};
+            for (int pass = 0; pass < 3; ++pass)
+              ts.tdma_len[pass] = std::max(ts.tdma_len[pass], len[pass]);
+          }
+        for (int pass = 0; pass < 3; ++pass)
+          lines = lines && tdma_lines_lds(ts.tdma_len[pass]) <= h->lds_budget;
+        ts.tdma_lines = lines && tdma_lines_ok();
         // small levels: whole sweeps in one workgroup per block
-        bool small = true;
+        bool small = !ts.tdma_lines;
         size_t lds = 0;
         for (const BlockInfo &B : h->blk)
           if (member(B)) {
@@ -1565,10 +1608,10 @@ h3dmg_status gen_relax(h3dmg_handle *h, int g) {
         small = small && lds <= h->lds_budget && tdma_sweep_ok(h->lds_budget);
         ts.tdma_lds = small ? lds : 0;
         ts.tdma_pipe = !h->lsm;
-        if (small)
+        if (small || ts.tdma_lines)
           for (const BlockInfo &B : h->blk)
             if (member(B)) ts.h.push_back(Tile{B.desc[g], 0, 0, 0, 1, 7});
-        for (int pass = 0; pass < 3 && !small; ++pass) {
+        for (int pass = 0; pass < 3 && !small && !ts.tdma_lines; ++pass) {
           ts.pass_begin[pass] = ts.n();
           for (const BlockInfo &B : h->blk)
             if (member(B)) {
