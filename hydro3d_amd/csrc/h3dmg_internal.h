@@ -29,8 +29,10 @@ namespace h3dmg {
 constexpr int TILE_X = 64;  // one wavefront along the contiguous axis
 constexpr int TILE_Y = 4;   // four wavefronts per workgroup
 constexpr int NTHREADS = TILE_X * TILE_Y;
-constexpr int TAIL_THREADS = 512;  // V-cycle tail: one workgroup per block
-constexpr int TAIL_U = 4;           // cells per thread with loads in flight together
+constexpr int TAIL_THREADS = 1024;  // V-cycle tail: one workgroup per block
+// entries per colour of the largest level the tail runs with its addresses in
+// registers (two per thread and colour)
+constexpr int TAIL_FAST_ENTRIES = 2 * TAIL_THREADS;
 constexpr int TAIL_MAX_LEVELS = 16;
 
 struct LevelDev {
@@ -149,19 +151,31 @@ void launch_update(hipStream_t s, const Tile *tiles, int ntiles, const FineDev *
 void launch_finalize(hipStream_t s, const int *tile_begin, int nblocks, const RedPartial *partials,
                      RedPartial *out);
 // one workgroup per tile; Tile::lev = coarsest descriptor, Tile::x0 = block
-void launch_coarse_exact(hipStream_t s, const Tile *tiles, int ntiles, const LevelDev *levs,
-                         const int *active, const double *const *eig_q,
+// grid and LDS of the exact solve of a list of blocks (exact_grid_add of each)
+struct ExactGrid {
+  bool split = true;  // every block's planes and columns fit in LDS
+  size_t plane_lds = 0, cols_lds = 0;
+  int planes = 0, chunks = 0;
+  unsigned blocks = 0;
+};
+void exact_grid_add(ExactGrid &g, const LevelDev &L, size_t lds_budget);
+hipError_t exact_allow_lds(size_t lds_bytes);
+void launch_coarse_exact(hipStream_t s, const Tile *tiles, int ntiles, const ExactGrid &grid,
+                         const LevelDev *levs, const int *active, const double *const *eig_q,
                          const double *const *eig_l, double *const *scratch, int buf);
 
 // levels >= the tail level of every block in one launch, one workgroup per
 // block, every level in LDS (Tile::lev = the block's descriptor at the tail
-// level); every level ends in buffer (nu1+nu2)&1.  vtail_lds_bytes gives the
+// level, z1 = its levels from there down); every level ends in buffer (nu1+nu2)&1.  vtail_lds_bytes gives the
 // LDS a block needs from descriptor `top` down (host copies of the
 // descriptors).
 void launch_vtail(hipStream_t s, const Tile *tiles, int ntiles, const LevelDev *levs,
                   const int *active, const double *const *eig_q, const double *const *eig_l,
                   int nu1, int nu2, int exact, int mixed, size_t lds_bytes);
-size_t vtail_lds_bytes(const LevelDev *levs_host, int top, bool mixed, bool exact);
+// padded: with the alignment of the kernel's layout (at most
+// VTAIL_LDS_PAD more); the bound on a tail level counts the plain bytes
+size_t vtail_lds_bytes(const LevelDev *levs_host, int top, bool mixed, bool exact, bool padded);
+constexpr size_t VTAIL_LDS_PAD = 6 * 256 + 16 * TAIL_MAX_LEVELS;
 // permit `lds_bytes` of dynamic LDS for the tail kernel
 hipError_t vtail_allow_lds(size_t lds_bytes);
 

@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "h3dmg_internal.h"
 
@@ -194,6 +195,32 @@ __device__ __forceinline__ double div_ap(double num, double ap, double /*inv_ap*
 }
 __device__ __forceinline__ float div_ap(float num, float /*ap*/, float inv_ap) {
   return num * inv_ap;
+}
+
+// n / d, correctly rounded, by a divisor used many times: y = RN(1/d) once,
+// then q = RN(n*y) and two corrections q + RN(n - q*d)*y with fused
+// multiply-adds.  After the first q is within one ulp of n/d (each of RN(1/d)
+// and RN(n*y) is off by half an ulp at most, and the remainder of a q that
+// close is exact), and the second then rounds n/d correctly (P. Markstein,
+// IBM J. Res. Dev. 34(1), 1990: y correctly rounded, q faithful).  Six
+// operations, bitwise the quotient as written.  The remainders are exact only away from the ends of the
+// exponent range: a quotient whose numerator lies there is divided as
+// written, as is every quotient when the divisor does (fast = false).
+struct Divisor {
+  double d, y;
+  bool fast;
+};
+__device__ __forceinline__ bool divisor_fast(double d) {
+  return fabs(d) > 0x1p-300 && fabs(d) < 0x1p300;
+}
+__device__ __forceinline__ double div_by(double n, const Divisor &D) {
+  // biased exponent of n in [500, 1546]: |n| in [2^-523, 2^524), or n zero
+  const unsigned e = ((unsigned)(__double_as_longlong(n) >> 52)) & 0x7ffu;
+  if (__builtin_expect(!D.fast || (e - 500u > 1046u && n != 0.0), 0)) return n / D.d;
+  double q = n * D.y;
+  q = __builtin_fma(__builtin_fma(-q, D.d, n), D.y, q);
+  q = __builtin_fma(__builtin_fma(-q, D.d, n), D.y, q);
+  return __builtin_amdgcn_div_fixup(q, D.d, n);  // the sign of a zero quotient
 }
 
 // DPP wavefront shifts by one lane (GFX9 wave_shr:1 = 0x138, wave_shl:1 =
@@ -1955,134 +1982,327 @@ __global__ void __launch_bounds__(FIN_THREADS)
 // reference counterpart): A = Dx (+) Dy (+) Dz with Dx the 1-D Neumann or
 // periodic second difference; with Q_a the orthonormal eigenvectors of D_a
 // (columns) and l_a its eigenvalues, u = Q (Q^T f ./ (lx+ly+lz)) with the
-// zero (constant) mode dropped -- the null-space projection.  One workgroup
-// per block; scratch holds two n^3 arrays.  The body is shared by
-// k_coarse_exact (arrays in global memory) and the V-cycle tail kernel
-// (arrays in LDS, S = lds address space): the same arithmetic in the same
-// order.  Every thread of the workgroup calls it.
+// zero (constant) mode dropped -- the null-space projection.  The transforms
+// run along x, y, z forwards and z, y, x back, every sum in index order, on
+// one of three routes with the same arithmetic in the same order: inside the
+// V-cycle tail (coarse_exact_lds), in three launches over the chip
+// (k_exact_plane, k_exact_cols), or one launch per transform (k_exact_pass).
 template <class T>
 using lds = __attribute__((address_space(3))) T;
-
-template <bool IN_LDS>
-struct Space;
-template <>
-struct Space<false> {
-  template <class T>
-  using ptr = T *;
-  template <class T>
-  static __device__ __forceinline__ T *cast(void *p) {
-    return (T *)p;
-  }
-};
-template <>
-struct Space<true> {
-  template <class T>
-  using ptr = lds<T> *;
-  template <class T>
-  static __device__ __forceinline__ lds<T> *cast(void *p) {
-    return (lds<T> *)p;
-  }
-};
 
 __device__ __forceinline__ int cidx32(int H, int nj, int i, int j, int k) {
   return (k * nj + j) * H + (i >> 1);
 }
 
-template <bool IN_LDS>
-__device__ void coarse_exact_body(const LevelDev &L, const double *Q0g, const double *Q1g,
-                                  const double *Q2g, const double *l0g, const double *l1g,
-                                  const double *l2g, double *Ag, double *Bg, int buf) {
-  typedef Space<IN_LDS> S;
-  typedef typename S::template ptr<double> dp;
-  const dp Q0 = S::template cast<double>((void *)Q0g), Q1 = S::template cast<double>((void *)Q1g),
-           Q2 = S::template cast<double>((void *)Q2g);
-  const dp l0 = S::template cast<double>((void *)l0g), l1 = S::template cast<double>((void *)l1g),
-           l2 = S::template cast<double>((void *)l2g);
-  const dp A = S::template cast<double>(Ag), Bs = S::template cast<double>(Bg);
-  const dp R0 = S::template cast<double>(L.rhs[0]), R1 = S::template cast<double>(L.rhs[1]);
-  const dp P0 = S::template cast<double>(L.phi[buf][0]), P1 = S::template cast<double>(L.phi[buf][1]);
-  const int n0 = L.ni, n1 = L.nj, n2 = L.nk;
-  const int plane = n0 * n1;
-  const int n = plane * n2;
-  const int tid = (int)threadIdx.x;
-  const int nthr = (int)blockDim.x;
-  // gather rhs (colour split) into natural layout A[i + n0*(j + n1*k)]
-  for (int q = tid; q < n; q += nthr) {
-    const int i = q % n0, j = (q / n0) % n1, k = q / plane;
-    const int e = cidx32(L.H, L.nj, i, j, k);
-    A[q] = ((i + j + k) & 1) ? R1[e] : R0[e];
-  }
-  __syncthreads();
-  // forward transforms: B = Q0^T along i, A = Q1^T along j, B = Q2^T along k
-  for (int q = tid; q < n; q += nthr) {
-    const int i = q % n0;
-    const int base = q - i;
-    double s = 0.0;
-    for (int x = 0; x < n0; ++x) s += Q0[x * n0 + i] * A[base + x];
-    Bs[q] = s;
-  }
-  __syncthreads();
-  for (int q = tid; q < n; q += nthr) {
-    const int j = (q / n0) % n1;
-    const int base = q - j * n0;
-    double s = 0.0;
-    for (int y = 0; y < n1; ++y) s += Q1[y * n1 + j] * Bs[base + y * n0];
-    A[q] = s;
-  }
-  __syncthreads();
-  for (int q = tid; q < n; q += nthr) {
-    const int k = q / plane;
-    const int base = q - k * plane;
-    double s = 0.0;
-    for (int z = 0; z < n2; ++z) s += Q2[z * n2 + k] * A[base + z * plane];
-    const int i = q % n0, j = (q / n0) % n1;
-    const double lam = l0[i] + l1[j] + l2[k];
-    // mode (0,0,0) is the constant (null-space) mode of every axis
-    Bs[q] = ((i | j | k) == 0) ? 0.0 : s / lam;
-  }
-  __syncthreads();
-  // inverse transforms: A = Q2 along k, B = Q1 along j, phi = Q0 along i
-  for (int q = tid; q < n; q += nthr) {
-    const int k = q / plane;
-    const int base = q - k * plane;
-    double s = 0.0;
-    for (int z = 0; z < n2; ++z) s += Q2[k * n2 + z] * Bs[base + z * plane];
-    A[q] = s;
-  }
-  __syncthreads();
-  for (int q = tid; q < n; q += nthr) {
-    const int j = (q / n0) % n1;
-    const int base = q - j * n0;
-    double s = 0.0;
-    for (int y = 0; y < n1; ++y) s += Q1[j * n1 + y] * A[base + y * n0];
-    Bs[q] = s;
-  }
-  __syncthreads();
-  for (int q = tid; q < n; q += nthr) {
-    const int i = q % n0, j = (q / n0) % n1, k = q / plane;
-    const int base = q - i;
-    double s = 0.0;
-    for (int x = 0; x < n0; ++x) s += Q0[i * n0 + x] * Bs[base + x];
-    const int e = cidx32(L.H, L.nj, i, j, k);
-    if ((i + j + k) & 1)
-      P1[e] = s;
-    else
-      P0[e] = s;
-  }
-  __syncthreads();
+// q -> (i, j, k) of an n0 x n1 x . array, by float reciprocals with one exact
+// correction (q < 2^24)
+__device__ __forceinline__ void split3(int q, int n0, int n1, int &i, int &j, int &k) {
+  int r = (int)((float)q * (1.0f / (float)n0));
+  i = q - __mul24(r, n0);
+  const int a = i < 0 ? -1 : i >= n0 ? 1 : 0;
+  r += a;
+  i -= a * n0;
+  k = (int)((float)r * (1.0f / (float)n1));
+  j = r - __mul24(k, n1);
+  const int b = j < 0 ? -1 : j >= n1 ? 1 : 0;
+  k += b;
+  j -= b * n1;
 }
 
+// The six transforms, x y z forwards, then z y x back, one code for all (the
+// tail runs them once per launch: instruction fetches count).  Along an axis
+// of `len` points, for every row (the other two coordinates; points vs apart)
+// and index a,
+//   out(a) = sum over x, in order, of Q(x, a) * V(x),
+// Q(x, a) = Q[x*len + a] forwards, Q[a*len + x] back.  A thread forms RI
+// indexes x RR rows of outputs and reads RI + RR operands per term: one
+// output per thread reads two operands per product, and LDS reads bound the
+// transforms.  The sums run in the same order whatever RI and RR.
+typedef lds<double> *ldsd;
+template <int RI, int RR, class dp>
+__device__ __forceinline__ void coarse_exact_passes(int n0, int n1, int n2, int H, dp Q0, dp Q1,
+                                                    dp Q2, dp l0, dp l1, dp l2, dp A, dp Bs, dp P0,
+                                                    dp P1) {
+  const int plane = n0 * n1, n = plane * n2;
+  const int tid = (int)threadIdx.x, nthr = (int)blockDim.x;
+#pragma clang loop unroll(disable)
+  for (int p = 0; p < 6; ++p) {
+    const int ax = p < 3 ? p : 5 - p;
+    const bool fwd = p < 3;
+    const dp Q = ax == 0 ? Q0 : ax == 1 ? Q1 : Q2;
+    const dp V = (p & 1) ? Bs : A, O = (p & 1) ? A : Bs;
+    const int len = ax == 0 ? n0 : ax == 1 ? n1 : n2;
+    const int vs = ax == 0 ? 1 : ax == 1 ? n0 : plane;
+    const int qx = fwd ? len : 1, qa = fwd ? 1 : len;
+    const int nrow = n / len, nib = (len + RI - 1) / RI, nrb = (nrow + RR - 1) / RR;
+#pragma clang loop unroll(disable)
+    for (int t = tid; t < nib * nrb; t += nthr) {
+      int q, ib, dummy;
+      split3(t, nrb, nib, q, ib, dummy);
+      int at[RR], ix[RI];
+#pragma unroll
+      for (int r = 0; r < RR; ++r) {
+        // rows: (j,k) pairs, (i,k) pairs, (i,j) pairs
+        const int row = min(q + r * nrb, nrow - 1);
+        int i, k, z;
+        split3(row, n0, n2, i, k, z);
+        at[r] = ax == 0 ? row * n0 : ax == 1 ? k * plane + i : row;
+      }
+#pragma unroll
+      for (int a = 0; a < RI; ++a) ix[a] = min(ib * RI + a, len - 1) * qa;
+      double s[RI][RR];
+#pragma unroll
+      for (int a = 0; a < RI; ++a)
+#pragma unroll
+        for (int r = 0; r < RR; ++r) s[a][r] = 0.0;
+#pragma unroll 4
+      for (int x = 0; x < len; ++x) {
+        double qv[RI], vv[RR];
+#pragma unroll
+        for (int a = 0; a < RI; ++a) qv[a] = Q[x * qx + ix[a]];
+#pragma unroll
+        for (int r = 0; r < RR; ++r) vv[r] = V[at[r] + x * vs];
+#pragma unroll
+        for (int a = 0; a < RI; ++a)
+#pragma unroll
+          for (int r = 0; r < RR; ++r) s[a][r] += qv[a] * vv[r];
+      }
+#pragma unroll
+      for (int a = 0; a < RI; ++a)
+#pragma unroll
+        for (int r = 0; r < RR; ++r) {
+          const int ia = ib * RI + a, o = at[r] + ia * vs;
+          if (ia < len && q + r * nrb < nrow) {
+            if (p == 2 || p == 5) {
+              int i, j, k;
+              split3(o, n0, n1, i, j, k);
+              if (p == 2) {
+                // mode (0,0,0) is the constant (null-space) mode of every axis
+                O[o] = o == 0 ? 0.0 : s[a][r] / (l0[i] + l1[j] + l2[k]);
+              } else {
+                (((i + j + k) & 1) ? P1 : P0)[cidx32(H, n1, i, j, k)] = s[a][r];
+              }
+            } else {
+              O[o] = s[a][r];
+            }
+          }
+        }
+    }
+    __syncthreads();
+  }
+}
+
+// Every thread of the workgroup calls it; all arrays in LDS, rhs and phi
+// colour split, A and Bs scratch of n0*n1*n2.
+__device__ __forceinline__ void coarse_exact_lds(int n0, int n1, int n2, int H, ldsd R0, ldsd R1,
+                                                 ldsd P0, ldsd P1, ldsd Q0, ldsd Q1, ldsd Q2,
+                                                 ldsd l0, ldsd l1, ldsd l2, ldsd A, ldsd Bs) {
+  const int n = n0 * n1 * n2;
+  // gather rhs into natural layout A[i + n0*(j + n1*k)]
+  for (int q = (int)threadIdx.x; q < n; q += (int)blockDim.x) {
+    int i, j, k;
+    split3(q, n0, n1, i, j, k);
+    A[q] = (((i + j + k) & 1) ? R1 : R0)[cidx32(H, n1, i, j, k)];
+  }
+  __syncthreads();
+  if (n <= (int)blockDim.x)
+    coarse_exact_passes<1, 1, ldsd>(n0, n1, n2, H, Q0, Q1, Q2, l0, l1, l2, A, Bs, P0, P1);
+  else
+    coarse_exact_passes<2, 2, ldsd>(n0, n1, n2, H, Q0, Q1, Q2, l0, l1, l2, A, Bs, P0, P1);
+}
+
+// One axis of a transform in LDS: for every row r < nrow (points rs apart)
+// and index a < len, out(r, a, sum over x, in order, of Q[x*qx + a*qa] *
+// V[r*rs + x*vs]).
+template <int RI, int RR, class F>
+__device__ __forceinline__ void exact_axis(int len, int nrow, int rs, int vs, ldsd Q, int qx,
+                                           int qa, ldsd V, F &&out) {
+  const int nib = (len + RI - 1) / RI, nrb = (nrow + RR - 1) / RR;
+#pragma clang loop unroll(disable)
+  for (int t = (int)threadIdx.x; t < nib * nrb; t += (int)blockDim.x) {
+    int q, ib, dummy;
+    split3(t, nrb, nib, q, ib, dummy);
+    int at[RR], ix[RI];
+#pragma unroll
+    for (int r = 0; r < RR; ++r) at[r] = min(q + r * nrb, nrow - 1) * rs;
+#pragma unroll
+    for (int a = 0; a < RI; ++a) ix[a] = min(ib * RI + a, len - 1) * qa;
+    double s[RI][RR];
+#pragma unroll
+    for (int a = 0; a < RI; ++a)
+#pragma unroll
+      for (int r = 0; r < RR; ++r) s[a][r] = 0.0;
+#pragma unroll 4
+    for (int x = 0; x < len; ++x) {
+      double qv[RI], vv[RR];
+#pragma unroll
+      for (int a = 0; a < RI; ++a) qv[a] = Q[x * qx + ix[a]];
+#pragma unroll
+      for (int r = 0; r < RR; ++r) vv[r] = V[at[r] + x * vs];
+#pragma unroll
+      for (int a = 0; a < RI; ++a)
+#pragma unroll
+        for (int r = 0; r < RR; ++r) s[a][r] += qv[a] * vv[r];
+    }
+#pragma unroll
+    for (int a = 0; a < RI; ++a)
+#pragma unroll
+      for (int r = 0; r < RR; ++r)
+        if (ib * RI + a < len && q + r * nrb < nrow) out(q + r * nrb, ib * RI + a, s[a][r]);
+  }
+}
+
+// Odd row pitch: rows of doubles then start in different LDS banks.
+__host__ __device__ inline int exact_pitch(int n) { return n | 1; }
+constexpr int EXACT_COLS = 16;     // z-columns per workgroup of k_exact_cols
+constexpr int EXACT_SMALL = 512;   // plane cells up to which a thread forms single outputs
+
+// x and y transforms of plane blockIdx.y of block tiles[blockIdx.x]: rhs to
+// scratch 0 (FWD), or back from scratch 1 to phi.  One workgroup per block is
+// bound by its LDS reads (two per product): a two-level cycle of 52x28x20 took
+// 215 us, of 64^3 2783; the planes and columns over the CUs 63 and 70,
+// and 4 us a launch.  Output tiles (RI x RI) read RI operands per product
+// less; below EXACT_SMALL cells there are not enough of them for the threads.
+template <bool FWD>
 __global__ void __launch_bounds__(256)
-    k_coarse_exact(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
-                   const int *__restrict__ active, const double *const *__restrict__ eig_q,
-                   const double *const *__restrict__ eig_l, double *const *__restrict__ scratch,
-                   int buf) {
+    k_exact_plane(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
+                  const int *__restrict__ active, const double *const *__restrict__ eig_q,
+                  double *const *__restrict__ scratch, int buf) {
+  extern __shared__ __align__(16) char smem[];
   const Tile t = tiles[blockIdx.x];  // lev = coarsest descriptor, x0 = block
-  if (!active[t.x0]) return;
+  const int b = t.x0, k = (int)blockIdx.y;
+  const LevelDev &L = levs[t.lev];
+  const int n0 = L.ni, n1 = L.nj;
+  if (!active[b] || k >= L.nk) return;
+  const int p0 = exact_pitch(n0), p1 = exact_pitch(n1), plane = n0 * n1;
+  const ldsd Q0 = (ldsd)smem, Q1 = Q0 + n0 * p0, V = Q1 + n1 * p1, W = V + p0 * n1;
+  const int tid = (int)threadIdx.x;
+  auto table = [&](ldsd Q, const double *g, int n, int p) {
+    for (int e = tid; e < n * n; e += 256) {
+      int i, j, z;
+      split3(e, n, n, i, j, z);
+      Q[j * p + i] = g[e];
+    }
+  };
+  table(Q0, eig_q[3 * b], n0, p0);
+  table(Q1, eig_q[3 * b + 1], n1, p1);
+  const double *R[2] = {(const double *)L.rhs[0], (const double *)L.rhs[1]};
+  double *P[2] = {(double *)L.phi[buf][0], (double *)L.phi[buf][1]};
+  double *const A = scratch[2 * b] + (size_t)k * plane;
+  const double *const B = scratch[2 * b + 1] + (size_t)k * plane;
+  const size_t row0 = (size_t)k * n1;
+  auto cell = [&](int i, int j) { return (row0 + j) * L.H + (i >> 1); };
+  for (int e = tid; e < plane; e += 256) {
+    int i, j, z;
+    split3(e, n0, n1, i, j, z);
+    V[j * p0 + i] = FWD ? (((i + j + k) & 1) ? R[1] : R[0])[cell(i, j)] : B[e];
+  }
+  __syncthreads();
+  auto mid = [&](int r, int a, double s) { W[FWD ? r * p0 + a : a * p0 + r] = s; };
+  auto end = [&](int r, int a, double s) {
+    if (FWD)
+      A[a * n0 + r] = s;
+    else
+      (((r + a + k) & 1) ? P[1] : P[0])[cell(a, r)] = s;
+  };
+  auto run = [&](auto ri) __attribute__((always_inline)) {
+    constexpr int RI = decltype(ri)::value;
+    if (FWD) {
+      exact_axis<RI, RI>(n0, n1, p0, 1, Q0, p0, 1, V, mid);  // rows j
+      __syncthreads();
+      exact_axis<RI, RI>(n1, n0, 1, p0, Q1, p1, 1, W, end);  // rows i
+    } else {
+      exact_axis<RI, RI>(n1, n0, 1, p0, Q1, 1, p1, V, mid);
+      __syncthreads();
+      exact_axis<RI, RI>(n0, n1, p0, 1, Q0, 1, p0, W, end);
+    }
+  };
+  if (plane <= EXACT_SMALL)
+    run(std::integral_constant<int, 1>());
+  else
+    run(std::integral_constant<int, 2>());
+}
+
+// z transform, division by the eigenvalues and z transform back of
+// EXACT_COLS columns: scratch 0 to scratch 1
+__global__ void __launch_bounds__(256)
+    k_exact_cols(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
+                 const int *__restrict__ active, const double *const *__restrict__ eig_q,
+                 const double *const *__restrict__ eig_l, double *const *__restrict__ scratch) {
+  extern __shared__ __align__(16) char smem[];
+  const Tile t = tiles[blockIdx.x];
   const int b = t.x0;
-  coarse_exact_body<false>(levs[t.lev], eig_q[3 * b], eig_q[3 * b + 1], eig_q[3 * b + 2],
-                           eig_l[3 * b], eig_l[3 * b + 1], eig_l[3 * b + 2], scratch[2 * b],
-                           scratch[2 * b + 1], buf);
+  const LevelDev &L = levs[t.lev];
+  const int n0 = L.ni, n2 = L.nk, plane = n0 * L.nj, c0 = (int)blockIdx.y * EXACT_COLS;
+  if (!active[b] || c0 >= plane) return;
+  const int p2 = exact_pitch(n2), nc = min(EXACT_COLS, plane - c0);
+  const ldsd Q2 = (ldsd)smem, V = Q2 + n2 * p2, W = V + n2 * EXACT_COLS,
+             lxy = W + n2 * EXACT_COLS, lz = lxy + EXACT_COLS;
+  const int tid = (int)threadIdx.x;
+  for (int e = tid; e < n2 * n2; e += 256) {
+    int i, j, z;
+    split3(e, n2, n2, i, j, z);
+    Q2[j * p2 + i] = eig_q[3 * b + 2][e];
+  }
+  const double *const A = scratch[2 * b] + c0;
+  for (int e = tid; e < n2 * EXACT_COLS; e += 256) {
+    const int k = e / EXACT_COLS, c = e % EXACT_COLS;
+    if (c < nc) V[e] = A[(size_t)k * plane + c];
+  }
+  if (tid < nc) {
+    const int j = (c0 + tid) / n0, i = (c0 + tid) - j * n0;
+    lxy[tid] = eig_l[3 * b][i] + eig_l[3 * b + 1][j];
+  }
+  for (int e = tid; e < n2; e += 256) lz[e] = eig_l[3 * b + 2][e];
+  __syncthreads();
+  exact_axis<1, 1>(n2, nc, 1, EXACT_COLS, Q2, p2, 1, V, [&](int r, int a, double s) {
+    // mode (0,0,0) is the constant (null-space) mode of every axis
+    W[a * EXACT_COLS + r] = (c0 + r == 0 && a == 0) ? 0.0 : s / (lxy[r] + lz[a]);
+  });
+  __syncthreads();
+  double *const B = scratch[2 * b + 1] + c0;
+  exact_axis<1, 1>(n2, nc, 1, EXACT_COLS, Q2, 1, p2, W,
+                   [&](int r, int a, double s) { B[(size_t)a * plane + r] = s; });
+}
+
+// Any size: transform `pass` of the six, a thread per output.
+__global__ void __launch_bounds__(256)
+    k_exact_pass(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
+                 const int *__restrict__ active, const double *const *__restrict__ eig_q,
+                 const double *const *__restrict__ eig_l, double *const *__restrict__ scratch,
+                 int buf, int pass) {
+  const Tile t = tiles[blockIdx.x];
+  const int b = t.x0;
+  if (!active[b]) return;
+  const LevelDev &L = levs[t.lev];
+  const int ax = pass < 3 ? pass : 5 - pass;
+  const bool fwd = pass < 3;
+  const int n0 = L.ni, n1 = L.nj, n2 = L.nk, len = ax == 0 ? n0 : ax == 1 ? n1 : n2;
+  const size_t plane = (size_t)n0 * n1, n = plane * n2;
+  const size_t vs = ax == 0 ? 1 : ax == 1 ? (size_t)n0 : plane;
+  const double *const Q = eig_q[3 * b + ax];
+  const double *const V = scratch[2 * b + (pass & 1)];
+  double *const O = scratch[2 * b + 1 - (pass & 1)];
+  for (size_t q = (size_t)blockIdx.y * 256 + threadIdx.x; q < n; q += (size_t)gridDim.y * 256) {
+    const int i = (int)(q % n0), j = (int)((q / n0) % n1), k = (int)(q / plane);
+    const int a = ax == 0 ? i : ax == 1 ? j : k;
+    const size_t base = q - a * vs;
+    double s = 0.0;
+    if (pass == 0) {
+      const size_t row = ((size_t)k * n1 + j) * L.H;
+      for (int x = 0; x < len; ++x)
+        s += Q[(size_t)x * len + a] * ((const double *)L.rhs[(x + j + k) & 1])[row + (x >> 1)];
+    } else {
+      const size_t qx = fwd ? len : 1, qa = fwd ? 1 : len;
+      for (int x = 0; x < len; ++x) s += Q[x * qx + a * qa] * V[base + x * vs];
+    }
+    if (pass == 2)
+      O[q] = q == 0 ? 0.0 : s / (eig_l[3 * b][i] + eig_l[3 * b + 1][j] + eig_l[3 * b + 2][k]);
+    else if (pass == 5)
+      ((double *)L.phi[buf][(i + j + k) & 1])[((size_t)k * n1 + j) * L.H + (i >> 1)] = s;
+    else
+      O[q] = s;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2093,209 +2313,381 @@ __global__ void __launch_bounds__(256)
 // workgroup barriers.  Small levels are latency-bound: one launch, LDS
 // latency and on-chip barriers replace ~3 full-chip launches per level.
 //
-// The tail levels are copied into LDS with their global layout (colour
-// split, pitch H); descriptors whose pointers point into LDS feed per-cell
-// functions that compute every cell with the same expression, in the same
-// order, as the per-level kernels (bitwise-identical results).  In: the top
-// level's rhs (global).  Out: the top level's phi in buffer (nu1+nu2)&1
-// (global), the buffer every level ends in on the host side.  The tile's
-// `lev` is the block's level-Lt descriptor.  Levels are float in a
-// mixed-precision handle except the coarsest (double).
+// Every cell's value is the expression of the per-level kernels, in the same
+// order (a wall's term is the product with zero).  The tail's one CU is bound
+// by instruction issue and, since it runs every piece of code a few times
+// only, by instruction fetches: a thread sets up its entries once per visit
+// of a level (TailCells) and the neighbours then lie constant steps away; no
+// piece is unrolled over levels, sweeps or colours.
+//
+// LDS per level: four phi arrays [buffer][colour] and two rhs arrays in the
+// global layout (colour split, pitch H), and between them a zero, the value
+// behind every wall.  In: the top level's rhs (global).
+// Out: the top level's phi in buffer (nu1+nu2)&1 (global), the buffer every
+// level ends in on the host side.  The tile's `lev` is the block's level-Lt
+// descriptor.  Levels are float in a mixed-precision handle except the
+// coarsest (double).
+constexpr int TAIL_U = TAIL_FAST_ENTRIES / TAIL_THREADS;  // entries a thread keeps per colour
 
-// value of cell (x,y,z) in [-1, n] of an LDS-resident level, buffer `buf`,
-// ghosts resolved to their image
-template <class T>
-__device__ __forceinline__ T lds_value(const LevelDev &L, int buf, int x, int y, int z) {
-  x = image(x, L.ni, L.per & 1);
-  y = image(y, L.nj, L.per & 2);
-  z = image(z, L.nk, L.per & 4);
-  const lds<T> *a = (const lds<T> *)L.phi[buf][(x + y + z) & 1];
-  return a[cidx32(L.H, L.nj, x, y, z)];
+// bytes of one array of a level in LDS
+__host__ __device__ inline size_t tail_phi_bytes(size_t entries, size_t word) {
+  return (entries * word + 15) & ~(size_t)15;
 }
 
-// One colour half-sweep over a whole level, cell-parallel; the loads of
-// TAIL_U cells per thread are issued before any of their stores.  A red cell
-// reads its black neighbours before the sweep (buffer src), a black cell its
-// red neighbours after it (buffer 1-src); ghosts read their image in buffer
-// src; with zero != 0 buffer src holds zeros.  Coefficients and arithmetic
-// are cell_coef's and the per-level kernels'.  Only the coordinate a
-// neighbour differs in can leave the level, so each neighbour resolves one
-// image and tests one ghost condition, and entries are split into (entry,
-// row, plane) by float reciprocals with one exact correction (n < 2^24).
+// a level's geometry and its arrays' byte offsets in dynamic LDS
+struct TailLev {
+  int ni, nj, nk, H, per, n;  // n: entries per colour array
+  unsigned phi, ps, rhs, rs;  // first phi / rhs array and the step between arrays
+  double cx, cy, cz;
+};
+
+// Level q (of nl) of the tail of a block whose top level is G, in scalar
+// registers: cells halve from level to level, and 1/h^2 with h doubled is a
+// quarter, exactly (a power of two).  The levels' arrays follow one another.
+__device__ __forceinline__ double uniform(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(b & 0xffffffffll));
+  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <bool MIXED>
+__device__ __forceinline__ TailLev tail_level(const LevelDev &G, int q, int nl) {
+  unsigned off = 0;
+  TailLev L;
+  for (int p = 0; p <= q; ++p) {
+    const unsigned word = !MIXED || p == nl - 1 ? 8u : 4u;
+    L.ni = G.ni >> p;
+    L.nj = G.nj >> p;
+    L.nk = G.nk >> p;
+    L.H = (((L.ni + 1) / 2) + 1) & ~1;
+    L.n = L.H * L.nj * L.nk;
+    L.phi = off;
+    L.ps = (unsigned)tail_phi_bytes((size_t)L.n, word);
+    L.rhs = L.phi + 4 * L.ps + 16;  // (a zero slot after the phi arrays)
+    L.rs = ((unsigned)L.n * word + 15u) & ~15u;
+    off = L.rhs + 2 * L.rs;
+  }
+  const double s = 1.0 / (double)(1ull << (2 * q));
+  L.per = G.per;
+  L.cx = uniform(G.cx * s);
+  L.cy = uniform(G.cy * s);
+  L.cz = uniform(G.cz * s);
+  return L;
+}
+// the first byte after a level's arrays
+__device__ __forceinline__ unsigned tail_end(const TailLev &L) { return L.rhs + 2 * L.rs; }
+
+// entry e -> (pair m, row j, plane k), by float reciprocals with one exact
+// correction (n < 2^24)
+struct TailSplit {
+  int H, nj;
+  float iH, iJ;
+  __device__ explicit TailSplit(const TailLev &L)
+      : H(L.H), nj(L.nj), iH(1.0f / (float)L.H), iJ(1.0f / (float)L.nj) {}
+  __device__ __forceinline__ void operator()(int e, int &m, int &j, int &k) const {
+    int r = (int)((float)e * iH);
+    m = e - __mul24(r, H);
+    const int a = m < 0 ? -1 : m >= H ? 1 : 0;
+    r += a;
+    m -= a * H;
+    k = (int)((float)r * iJ);
+    j = r - __mul24(k, nj);
+    const int b = j < 0 ? -1 : j >= nj ? 1 : 0;
+    k += b;
+    j -= b * nj;
+  }
+};
+
 template <class T>
-__device__ __forceinline__ void tail_half_sweep(const LevelDev &Ls, int colour, int src, int zero) {
-  // the descriptor lives in LDS: its fields once, in registers
-  const int H = Ls.H, nj = Ls.nj, nk = Ls.nk, ni = Ls.ni, per = Ls.per;
-  const bool px = per & 1, py = per & 2, pz = per & 4;
-  const bool wx0 = wall_face(Ls, 0), wx1 = wall_face(Ls, 1), wy0 = wall_face(Ls, 2),
-             wy1 = wall_face(Ls, 3), wz0 = wall_face(Ls, 4), wz1 = wall_face(Ls, 5);
-  const T cx = (T)Ls.cx, cy = (T)Ls.cy, cz = (T)Ls.cz;
-  const int n = H * nj * nk, plane = H * nj;
-  const lds<T> *nb_int =
-      colour == 0 ? (const lds<T> *)Ls.phi[src][1] : (const lds<T> *)Ls.phi[1 - src][0];
-  const lds<T> *g0 = (const lds<T> *)Ls.phi[src][0], *g1 = (const lds<T> *)Ls.phi[src][1];
-  const lds<T> *R = (const lds<T> *)Ls.rhs[colour];
-  lds<T> *D = (lds<T> *)Ls.phi[1 - src][colour];
-  const bool zero_int = zero && colour == 0, zero_ghost = zero != 0;
-  const float invH = 1.0f / (float)H, invJ = 1.0f / (float)nj;
-  // a neighbour: interior from nb_int, a ghost from its image in buffer src
-  // (colour array by the image's parity); zeros in the zero state
-  auto nbv = [&](bool ghost, int par, int entry) -> T {
-    const lds<T> *a = ghost ? ((par & 1) ? g1 : g0) : nb_int;
-    const T v = a[entry];
-    return (ghost ? zero_ghost : zero_int) ? T(0) : v;
-  };
-  for (int base = (int)threadIdx.x; base < n; base += TAIL_THREADS * TAIL_U) {
-    T v[TAIL_U][7];
-    int ci[TAIL_U], cj[TAIL_U], ck[TAIL_U];
-    bool ok[TAIL_U];
+__device__ __forceinline__ T tail_ld(unsigned off) {
+  extern __shared__ __align__(16) char smem[];
+  return *(const lds<T> *)((const lds<char> *)smem + off);
+}
+template <class T>
+__device__ __forceinline__ void tail_st(unsigned off, T v) {
+  extern __shared__ __align__(16) char smem[];
+  *(lds<T> *)((lds<char> *)smem + off) = v;
+}
+
+// What a thread keeps of its entries tid + u*TAIL_THREADS of a level (from
+// `first` on) while the level is swept: the entry's byte offset, the faces its
+// cells touch, and each colour's ap and divisor.
+template <class T>
+struct TailDiv;
+template <>
+struct TailDiv<float> {  // FP32 multiplies by 1/ap (div_ap)
+  float a, inv;
+  __device__ __forceinline__ void set(float ap) {
+    a = ap;
+    inv = 1.0f / ap;
+  }
+  __device__ __forceinline__ float operator()(float num) const { return num * inv; }
+};
+template <>
+struct TailDiv<double> {  // FP64 divides by ap, correctly rounded (div_by)
+  double a, inv;
+  __device__ __forceinline__ void set(double ap) {
+    a = ap;
+    inv = 1.0 / ap;
+  }
+  __device__ __forceinline__ double operator()(double num) const {
+    return div_by(num, Divisor{a, inv, divisor_fast(a)});
+  }
+};
+
+template <class T>
+struct TailCells {
+  // Byte offsets of the six neighbours while buffer 0 / 1 is being swept.
+  // Inside the level they lie a constant step away in the other colour
+  // (before the sweep for a red cell, after it for a black one); across a
+  // periodic face their image does in the swept buffer, its colour fixed by
+  // the axis' parity; across a wall it is the level's zero slot.
+  unsigned a[TAIL_U][2][2][6];
+  unsigned o[TAIL_U];  // entry * sizeof(T)
+  bool in[TAIL_U];     // a valid entry
+  bool wave, two;      // (uniform) the wave has entries; the second ones exist
+  TailDiv<T> div[TAIL_U][2];
+
+  __device__ __forceinline__ void set(const TailLev &L, int first) {
+    constexpr unsigned SZ = sizeof(T);
+    const TailSplit split(L);
+    const bool px = L.per & 1, py = L.per & 2, pz = L.per & 4;
+    const unsigned row = (unsigned)L.H * SZ, plane = row * (unsigned)L.nj;
+    const unsigned span = plane * (unsigned)(L.nk - 1), zero = L.phi + 4 * L.ps;
+    const unsigned xl = (unsigned)((L.ni - 1) >> 1) * SZ;  // entry of cell ni-1 in its row
+    const T cx = (T)L.cx, cy = (T)L.cy, cz = (T)L.cz;
+    const int w0 = __builtin_amdgcn_readfirstlane(first + (int)threadIdx.x);
+    wave = w0 < L.n;
+    two = w0 + TAIL_THREADS < L.n;
+    static_assert(TAIL_U == 2, "two entries per thread");
 #pragma unroll
     for (int u = 0; u < TAIL_U; ++u) {
-      const int e0 = base + u * TAIL_THREADS;
-      const int e = min(e0, n - 1);  // lanes past the end read a valid entry
-      int r = (int)((float)e * invH);
-      int m = e - r * H;
-      if (m < 0) {
-        --r;
-        m += H;
-      } else if (m >= H) {
-        ++r;
-        m -= H;
+      const int e0 = first + (int)threadIdx.x + u * TAIL_THREADS;
+      in[u] = e0 < L.n;
+      if (u ? !two : !wave) continue;
+      const int q = min(e0, L.n - 1);  // lanes past the end read a valid entry
+      int m, j, k;
+      split(q, m, j, k);
+      o[u] = (unsigned)q * SZ;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int sx = (c + j + k) & 1, i = 2 * m + sx;
+        const bool fw = i == 0, fe = i == L.ni - 1, fs = j == 0, fn = j == L.nj - 1, fb = k == 0,
+                   ft = k == L.nk - 1;
+        const T aw = (!px && fw) ? T(0) : cx, ae = (!px && fe) ? T(0) : cx;
+        const T as = (!py && fs) ? T(0) : cy, an = (!py && fn) ? T(0) : cy;
+        const T ab = (!pz && fb) ? T(0) : cz, at = (!pz && ft) ? T(0) : cz;
+        div[u][c].set(T(-1) * (aw + ae + as + an + ab + at));
+        const unsigned gx = o[u] + L.phi + (unsigned)((c + L.ni - 1) & 1) * L.ps,
+                       gy = o[u] + L.phi + (unsigned)((c + L.nj - 1) & 1) * L.ps,
+                       gz = o[u] + L.phi + (unsigned)((c + L.nk - 1) & 1) * L.ps;
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const unsigned g = (unsigned)(2 * b) * L.ps;
+          const unsigned in0 =
+              o[u] + L.phi + (unsigned)(2 * (c ? 1 - b : b) + (1 - c)) * L.ps;
+          unsigned(&x)[6] = a[u][c][b];
+          x[0] = fw ? (px ? gx + g + xl : zero) : in0 - (sx ? 0u : SZ);
+          x[1] = fe ? (px ? gx + g - xl : zero) : in0 + (sx ? SZ : 0u);
+          x[2] = fs ? (py ? gy + g + (plane - row) : zero) : in0 - row;
+          x[3] = fn ? (py ? gy + g - (plane - row) : zero) : in0 + row;
+          x[4] = fb ? (pz ? gz + g + span : zero) : in0 - plane;
+          x[5] = ft ? (pz ? gz + g - span : zero) : in0 + plane;
+        }
       }
-      int k = (int)((float)r * invJ);
-      int j = r - k * nj;
-      if (j < 0) {
-        --k;
-        j += nj;
-      } else if (j >= nj) {
-        ++k;
-        j -= nj;
-      }
-      const int i0 = 2 * m + ((colour + j + k) & 1);
-      const int i = min(i0, ni - 1);
-      ok[u] = e0 < n && i0 < ni;
-      ci[u] = i;
-      cj[u] = j;
-      ck[u] = k;
-      const int rb = (k * nj + j) * H;  // the row's first entry
-      const int xw = image(i - 1, ni, px), xe = image(i + 1, ni, px);
-      const int ys = image(j - 1, nj, py), yn = image(j + 1, nj, py);
-      const int zb = image(k - 1, nk, pz), zt = image(k + 1, nk, pz);
-      v[u][0] = nbv(i == 0, xw + j + k, rb + (xw >> 1));
-      v[u][1] = nbv(i == ni - 1, xe + j + k, rb + (xe >> 1));
-      v[u][2] = nbv(j == 0, i + ys + k, rb + (ys - j) * H + (i >> 1));
-      v[u][3] = nbv(j == nj - 1, i + yn + k, rb + (yn - j) * H + (i >> 1));
-      v[u][4] = nbv(k == 0, i + j + zb, rb + (zb - k) * plane + (i >> 1));
-      v[u][5] = nbv(k == nk - 1, i + j + zt, rb + (zt - k) * plane + (i >> 1));
-      v[u][6] = R[e];
     }
+  }
+
+  // One colour half-sweep from buffer SRC; skip: every neighbour is zero.
+  template <int C, int SRC>
+  __device__ __forceinline__ void half(const TailLev &L, bool skip) const {
+    const T cx = (T)L.cx, cy = (T)L.cy, cz = (T)L.cz;
+    const unsigned rb = L.rhs + (unsigned)C * L.rs,
+                   ob = L.phi + (unsigned)(2 * (1 - SRC) + C) * L.ps;
+    auto one = [&](int u) __attribute__((always_inline)) {
+      T v[6];
+#pragma unroll
+      for (int f = 0; f < 6; ++f) v[f] = tail_ld<T>(a[u][C][SRC][f]);
+      const T r = tail_ld<T>(rb + o[u]);
+      const T q = cx * v[0] + cx * v[1] + cy * v[2] + cy * v[3] + cz * v[4] + cz * v[5];
+      return div[u][C](r - (C == 0 && skip ? T(0) : q));
+    };
+    if (two) {
+      const T x0 = one(0), x1 = one(1);
+      tail_st<T>(ob + o[0], x0);
+      if (in[1]) tail_st<T>(ob + o[1], x1);
+    } else if (wave) {
+      const T x0 = one(0);
+      if (in[0]) tail_st<T>(ob + o[0], x0);
+    }
+    __syncthreads();
+  }
+
+  // the residual of both colours' cells from buffer `buf` into the other (a
+  // black cell's interior neighbours in `buf` are those of a sweep from the
+  // other buffer)
+  __device__ __forceinline__ void residual(const TailLev &L, int buf) const {
+    const T cx = (T)L.cx, cy = (T)L.cy, cz = (T)L.cz;
+    const unsigned border = L.phi + 2 * L.ps, zero = L.phi + 4 * L.ps;
 #pragma unroll
     for (int u = 0; u < TAIL_U; ++u) {
-      if (!ok[u]) continue;
-      const int i = ci[u], j = cj[u], k = ck[u];
-      // cell_coef's coefficients: zero towards a wall
-      const T aw = (i == 0 && wx0) ? T(0) : cx, ae = (i == ni - 1 && wx1) ? T(0) : cx;
-      const T as = (j == 0 && wy0) ? T(0) : cy, an = (j == nj - 1 && wy1) ? T(0) : cy;
-      const T ab = (k == 0 && wz0) ? T(0) : cz, at = (k == nk - 1 && wz1) ? T(0) : cz;
-      const T ap = T(-1) * (aw + ae + as + an + ab + at);
-      const T sum = aw * v[u][0] + ae * v[u][1] + as * v[u][2] + an * v[u][3] + ab * v[u][4] +
-                    at * v[u][5];
-      D[base + u * TAIL_THREADS] = div_ap(v[u][6] - sum, ap, T(1) / ap);
-    }
-  }
-  __syncthreads();
-}
-
-template <class T>
-__device__ __forceinline__ void tail_fill_zero(const LevelDev &L, int buf) {
-  const int n = L.H * L.nj * L.nk;
-  lds<T> *a = (lds<T> *)L.phi[buf][0], *b = (lds<T> *)L.phi[buf][1];
-  for (int e = (int)threadIdx.x; e < n; e += TAIL_THREADS) {
-    a[e] = T(0);
-    b[e] = T(0);
-  }
-  __syncthreads();
-}
-
-// nsweep sweeps from buffer `buf` (flag `zero`: buffer holds zeros)
-template <class T>
-__device__ __forceinline__ void tail_relax(const LevelDev &L, int nsweep, int &buf, bool &zero) {
-  for (int sw = 0; sw < nsweep; ++sw) {
-    tail_half_sweep<T>(L, 0, buf, zero ? 1 : 0);
-    tail_half_sweep<T>(L, 1, buf, zero ? 1 : 0);
-    buf ^= 1;
-    zero = false;
-  }
-}
-
-// mgrestr for one coarse cell per thread (the arithmetic of restrict_tile)
-template <class Tf, class Tc>
-__device__ __forceinline__ void tail_restrict(const LevelDev &F, const LevelDev &C, int src_f) {
-  const int n = C.ni * C.nj * C.nk;
-  const lds<Tf> *P0 = (const lds<Tf> *)F.phi[src_f][0], *P1 = (const lds<Tf> *)F.phi[src_f][1];
-  const lds<Tf> *F0 = (const lds<Tf> *)F.rhs[0], *F1 = (const lds<Tf> *)F.rhs[1];
-  lds<Tc> *C0 = (lds<Tc> *)C.rhs[0], *C1 = (lds<Tc> *)C.rhs[1];
-  for (int q0 = (int)threadIdx.x; q0 < n; q0 += TAIL_THREADS) {
-    const int ic = q0 % C.ni, jc = (q0 / C.ni) % C.nj, kc = q0 / (C.ni * C.nj);
-    Tc acc = Tc(0);
+      if (u ? !two : !wave) continue;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int i = 2 * ic + (q & 1), j = 2 * jc + ((q >> 1) & 1), k = 2 * kc + (q >> 2);
-      const Coef<Tf> c = cell_coef<Tf>(F, i, j, k);
-      const Tf W = lds_value<Tf>(F, src_f, i - 1, j, k);
-      const Tf E = lds_value<Tf>(F, src_f, i + 1, j, k);
-      const Tf S = lds_value<Tf>(F, src_f, i, j - 1, k);
-      const Tf N = lds_value<Tf>(F, src_f, i, j + 1, k);
-      const Tf B = lds_value<Tf>(F, src_f, i, j, k - 1);
-      const Tf Tt = lds_value<Tf>(F, src_f, i, j, k + 1);
-      const int fq = cidx32(F.H, F.nj, i, j, k);
-      const bool fc = (i + j + k) & 1;
-      const Tf P = fc ? P1[fq] : P0[fq];
-      const Tf r = fc ? F1[fq] : F0[fq];
-      const Tf res =
-          r - (c.aw * W + c.ae * E + c.as * S + c.an * N + c.ab * B + c.at * Tt + c.ap * P);
-      acc = q == 0 ? (Tc)res : acc + (Tc)res;
+      for (int c = 0; c < 2; ++c) {
+        const unsigned p = L.phi + (unsigned)(2 * buf + c) * L.ps + o[u];
+        T v[6];
+#pragma unroll
+        for (int f = 0; f < 6; ++f) {
+          const unsigned x0 = a[u][c][0][f], x1 = a[u][c][1][f];
+          v[f] = tail_ld<T>((x0 >= border) == (buf != 0) || x0 == zero ? x0 : x1);
+        }
+        const T P = tail_ld<T>(p), r = tail_ld<T>(L.rhs + (unsigned)c * L.rs + o[u]);
+        const T res = r - (cx * v[0] + cx * v[1] + cy * v[2] + cy * v[3] + cz * v[4] +
+                           cz * v[5] + div[u][c].a * P);
+        if (in[u]) tail_st<T>(L.phi + (unsigned)(2 * (1 - buf) + c) * L.ps + o[u], res);
+      }
     }
-    const int cq = cidx32(C.H, C.nj, ic, jc, kc);
-    if ((ic + jc + kc) & 1)
-      C1[cq] = Tc(0.125) * acc;
-    else
-      C0[cq] = Tc(0.125) * acc;
+    __syncthreads();
+  }
+
+  __device__ __forceinline__ void half_any(const TailLev &L, int c, int src, bool skip) const {
+    if (src == 0) {
+      if (c == 0)
+        half<0, 0>(L, skip);
+      else
+        half<1, 0>(L, false);
+    } else {
+      if (c == 0)
+        half<0, 1>(L, skip);
+      else
+        half<1, 1>(L, false);
+    }
+  }
+};
+
+template <class T>
+__device__ __forceinline__ void tail_fill_zero(const TailLev &L, int buf) {
+  for (int e = (int)threadIdx.x; e < L.n; e += TAIL_THREADS)
+    for (int c = 0; c < 2; ++c)
+      tail_st<T>(L.phi + (unsigned)(2 * buf + c) * L.ps + (unsigned)e * (unsigned)sizeof(T), T(0));
+  __syncthreads();
+}
+
+// nsweep sweeps of a level from buffer `buf` (zero: it starts from zeros,
+// filled in here) and, with resid, the residual into the free buffer.  Levels
+// of more than TAIL_U*TAIL_THREADS entries set their cells anew in every
+// pass.
+template <class T>
+__device__ __forceinline__ void tail_relax(const TailLev &L, int nsweep, int &buf, bool zero,
+                                           bool resid) {
+  if (threadIdx.x == 0) tail_st<T>(L.phi + 4 * L.ps, T(0));  // the zero slot
+  if (zero) tail_fill_zero<T>(L, buf);
+  else
+    __syncthreads();
+  TailCells<T> W;
+  if (L.n <= TAIL_U * TAIL_THREADS) {
+    W.set(L, 0);
+#pragma clang loop unroll(disable)
+    for (int h = 0; h < 2 * nsweep; ++h) {
+      W.half_any(L, h & 1, buf, zero && h == 0);
+      buf ^= h & 1;
+    }
+    if (resid) W.residual(L, buf);
+    return;
+  }
+#pragma clang loop unroll(disable)
+  for (int h = 0; h < 2 * nsweep + (resid ? 1 : 0); ++h) {
+#pragma clang loop unroll(disable)
+    for (int q = 0; q < L.n; q += TAIL_U * TAIL_THREADS) {
+      W.set(L, q);
+      if (h < 2 * nsweep)
+        W.half_any(L, h & 1, buf, zero && h == 0);
+      else
+        W.residual(L, buf);
+    }
+    if (h < 2 * nsweep) buf ^= h & 1;
+  }
+}
+
+// mgrestr: the 8-child sums (i fastest, then j, then k) of the residual in
+// buffer 1-buf, times 0.125
+template <class Tf, class Tc>
+__device__ __forceinline__ void tail_sum8(const TailLev &F, const TailLev &C, int buf) {
+  const TailSplit split(C);
+  constexpr unsigned SZ = sizeof(Tf);
+  const unsigned row = (unsigned)F.H * SZ, plane = row * (unsigned)F.nj;
+  const unsigned base = F.phi + (unsigned)(2 * (1 - buf)) * F.ps;
+  for (int q0 = (int)threadIdx.x; q0 < 2 * C.n; q0 += TAIL_THREADS) {
+    const int c = q0 >= C.n, e = q0 - (c ? C.n : 0);
+    int m, j, k;
+    split(e, m, j, k);
+    const int i = 2 * m + ((c + j + k) & 1);
+    if (i >= C.ni) continue;
+    // child (2i + q0, 2j + q1, 2k + q2): entry i of its row, colour the
+    // parity of q0 + q1 + q2
+    const unsigned o = base + __umul24(2 * k, plane) + __umul24(2 * j, row) + (unsigned)i * SZ;
+    Tf r[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      r[q] = tail_ld<Tf>(o + ((q >> 1) & 1 ? row : 0u) + (q >> 2 ? plane : 0u) +
+                         (((q & 1) + ((q >> 1) & 1) + (q >> 2)) & 1 ? F.ps : 0u));
+    Tc acc = (Tc)r[0];
+#pragma unroll
+    for (int q = 1; q < 8; ++q) acc = acc + (Tc)r[q];
+    tail_st<Tc>(C.rhs + (unsigned)c * C.rs + (unsigned)e * (unsigned)sizeof(Tc), Tc(0.125) * acc);
   }
   __syncthreads();
 }
 
-// mgcorr for one fine cell per thread (the arithmetic of k_prolong): fine
-// cell (i,j,k) is cell e = i&1 of entry l = i>>1, coarse row/plane pair
-// m = (j+1)>>1, n = (k+1)>>1 with offsets dj = (j+1)&1, dk = (k+1)&1
+// mgcorr for the two cells 2m, 2m+1 of an entry (the arithmetic of
+// k_prolong): they share the coarse corners x = m-1, m, m+1 of coarse row
+// pair (j+1)>>1 and plane pair (k+1)>>1
 template <class Tf, class Tc>
-__device__ __forceinline__ void tail_prolong(const LevelDev &F, const LevelDev &C, int src_f,
+__device__ __forceinline__ void tail_prolong(const TailLev &F, const TailLev &C, int src_f,
                                              int src_c) {
-  const int n = F.ni * F.nj * F.nk;
+  const TailSplit split(F);
   const bool px = C.per & 1, py = C.per & 2, pz = C.per & 4;
-  const lds<Tc> *V0 = (const lds<Tc> *)C.phi[src_c][0], *V1 = (const lds<Tc> *)C.phi[src_c][1];
-  lds<Tf> *D0 = (lds<Tf> *)F.phi[src_f][0], *D1 = (lds<Tf> *)F.phi[src_f][1];
-  for (int q0 = (int)threadIdx.x; q0 < n; q0 += TAIL_THREADS) {
-    const int i = q0 % F.ni, j = (q0 / F.ni) % F.nj, k = q0 / (F.ni * F.nj);
-    const int l = i >> 1, e = i & 1, di = 1 - e;
-    const int m = (j + 1) >> 1, dj = (j + 1) & 1;
-    const int nn = (k + 1) >> 1, dk = (k + 1) & 1;
-    Tc s = Tc(0);
+  for (int e = (int)threadIdx.x; e < F.n; e += TAIL_THREADS) {
+    int m, j, k;
+    split(e, m, j, k);
+    if (2 * m >= F.ni) continue;
+    const int mj = (j + 1) >> 1, dj = (j + 1) & 1, mk = (k + 1) >> 1, dk = (k + 1) & 1;
+    int xc[3], yc[2], zc[2];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int oi = q >> 2, oj = q & 1, ok = (q >> 1) & 1;
-      const int x = image(l - 1 + e + oi, C.ni, px);
-      const int y = image(m - 1 + oj, C.nj, py);
-      const int z = image(nn - 1 + ok, C.nk, pz);
-      const Tc w = (oi == di ? Tc(3) : Tc(1)) * (oj == dj ? Tc(3) : Tc(1)) *
-                   (ok == dk ? Tc(3) : Tc(1));
-      const int cq = cidx32(C.H, C.nj, x, y, z);
-      const Tc v = ((x + y + z) & 1) ? V1[cq] : V0[cq];
-      s = (q == 0) ? w * v : s + w * v;
+    for (int a = 0; a < 3; ++a) xc[a] = image(m - 1 + a, C.ni, px);
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      yc[a] = image(mj - 1 + a, C.nj, py);
+      zc[a] = image(mk - 1 + a, C.nk, pz);
     }
-    lds<Tf> *fa = ((i + j + k) & 1) ? D1 : D0;
-    const int fq = cidx32(F.H, F.nj, i, j, k);
-    fa[fq] = fa[fq] + (Tf)(s / Tc(64));
+    Tc cv[3][2][2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int row = __mul24(__mul24(zc[c], C.nj) + yc[b], C.H);
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+          cv[a][b][c] = tail_ld<Tc>(C.phi +
+                                    (unsigned)(2 * src_c + ((xc[a] + yc[b] + zc[c]) & 1)) * C.ps +
+                                    (unsigned)(row + (xc[a] >> 1)) * (unsigned)sizeof(Tc));
+      }
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {  // cell 2m+d; ni is even above the coarsest level
+      const int di = 1 - d;
+      Tc s = Tc(0);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int oi = q >> 2, oj = q & 1, ok = (q >> 1) & 1;
+        const Tc w = (oi == di ? Tc(3) : Tc(1)) * (oj == dj ? Tc(3) : Tc(1)) *
+                     (ok == dk ? Tc(3) : Tc(1));
+        const Tc v = cv[d + oi][oj][ok];
+        s = (q == 0) ? w * v : s + w * v;
+      }
+      const unsigned o = F.phi + (unsigned)(2 * src_f + ((d + j + k) & 1)) * F.ps +
+                         (unsigned)e * (unsigned)sizeof(Tf);
+      tail_st<Tf>(o, tail_ld<Tf>(o) + (Tf)(s / Tc(64)));
+    }
   }
   __syncthreads();
 }
@@ -2305,138 +2697,106 @@ __device__ __forceinline__ void tail_copy(D *dst, const S *src, int n) {
   for (int e = (int)threadIdx.x; e < n; e += TAIL_THREADS) dst[e] = src[e];
 }
 
+// the exact solve's tables as the block's region holds them: per axis of n
+// points Q (n x n) and lambda (n), each 256-byte aligned
+__host__ __device__ inline unsigned tail_eig_q(int n) {
+  return ((unsigned)(n * n) * 8u + 255u) & ~255u;
+}
+__host__ __device__ inline unsigned tail_eig_axis(int n) {
+  return tail_eig_q(n) + (((unsigned)n * 8u + 255u) & ~255u);
+}
+__host__ __device__ inline unsigned tail_eig_bytes(int ni, int nj, int nk) {
+  return tail_eig_axis(ni) + tail_eig_axis(nj) + tail_eig_axis(nk);
+}
+
 template <bool MIXED>
 __global__ void __launch_bounds__(TAIL_THREADS)
     k_vtail(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
             const int *__restrict__ active, const double *const *__restrict__ eig_q,
             const double *const *__restrict__ eig_l, int nu1, int nu2, int exact) {
   extern __shared__ __align__(16) char smem[];
-  // descriptors of the tail's levels with their arrays in LDS: level q of the
-  // tail is lv[q] (written by thread 0, read by all)
-  __shared__ LevelDev lv[TAIL_MAX_LEVELS];
-  __shared__ int s_nl;
-  __shared__ size_t s_off;
   const Tile t = tiles[blockIdx.x];
-  const int top = t.lev;
-  const int blk = levs[top].blk;
+  const int nl = t.z1;  // the block's levels from the tail level down
+  const LevelDev &G = levs[t.lev];
+  const int blk = G.blk;
   if (!active[blk]) return;
+  typedef typename std::conditional<MIXED, float, double>::type T;  // above the coarsest level
   const int fin = (nu1 + nu2) & 1;
-  if (threadIdx.x == 0) {
-    int nl = 0;
-    size_t off = 0;
-    for (int d = top; d >= 0 && nl < TAIL_MAX_LEVELS; d = levs[d].coarser) {
-      LevelDev L = levs[d];
-      const bool w8 = !MIXED || L.coarser < 0;
-      const size_t half = (size_t)L.H * L.nj * L.nk * (w8 ? 8 : 4);
-      for (int bb = 0; bb < 2; ++bb)
-        for (int c = 0; c < 2; ++c) {
-          L.phi[bb][c] = smem + off;
-          off += (half + 15) & ~(size_t)15;
-        }
-      for (int c = 0; c < 2; ++c) {
-        L.rhs[c] = smem + off;
-        off += (half + 15) & ~(size_t)15;
-      }
-      lv[nl++] = L;
-    }
-    s_nl = nl;
-    s_off = off;
+  const int last = nl - 1;
+  const int tid = (int)threadIdx.x;
+  const TailLev L0 = tail_level<MIXED>(G, 0, nl), Z = tail_level<MIXED>(G, last, nl);
+  const bool do_exact = exact && (nl > 1 || G.finer >= 0);  // as the host: not for a 1-level block
+  // the exact solve's tables (Q and lambda of each axis, one contiguous image
+  // in the block's region, each part 256-byte aligned) and scratch follow the
+  // levels
+  unsigned eo = tail_end(Z);
+  const gmem<char> *const eg = (const gmem<char> *)(do_exact ? eig_q[3 * blk] : nullptr);
+  if (do_exact) {
+    const unsigned bytes = tail_eig_bytes(Z.ni, Z.nj, Z.nk);
+    for (unsigned e = (unsigned)tid * 8u; e < bytes; e += TAIL_THREADS * 8u)
+      tail_st<double>(eo + e, *(const gmem<double> *)(eg + e));
+  }
+  // the top level's rhs into LDS; its phi starts from zero
+  const bool top64 = !MIXED || nl == 1;
+  for (int c = 0; c < 2; ++c) {
+    if (top64)
+      tail_copy((lds<double> *)(smem + L0.rhs + c * L0.rs), (const gmem<double> *)G.rhs[c], L0.n);
+    else
+      tail_copy((lds<float> *)(smem + L0.rhs + c * L0.rs), (const gmem<float> *)G.rhs[c], L0.n);
   }
   __syncthreads();
-  const int last = s_nl - 1;
-  size_t off = s_off;
-  auto is64 = [&](int q) { return !MIXED || lv[q].coarser < 0; };
-  const bool do_exact = exact && lv[last].finer >= 0;  // as the host: not for a 1-level block
-  // the exact solve's tables and scratch follow the levels
-  const double *Q[3], *lam[3];
-  double *A = nullptr, *Bs = nullptr;
-  if (do_exact) {
-    const LevelDev &L = lv[last];
-    const int na[3] = {L.ni, L.nj, L.nk};
-    for (int a = 0; a < 3; ++a) {
-      double *q = (double *)(smem + off);
-      off += (size_t)na[a] * na[a] * 8;
-      double *l = (double *)(smem + off);
-      off += ((size_t)na[a] * 8 + 15) & ~(size_t)15;
-      tail_copy((lds<double> *)q, eig_q[3 * blk + a], na[a] * na[a]);
-      tail_copy((lds<double> *)l, eig_l[3 * blk + a], na[a]);
-      Q[a] = q;
-      lam[a] = l;
-    }
-    const size_t n3 = (size_t)na[0] * na[1] * na[2];
-    A = (double *)(smem + off);
-    off += n3 * 8;
-    Bs = (double *)(smem + off);
-  }
-  // top level's rhs into LDS
-  {
-    const LevelDev &G = levs[top];
-    const int n = G.H * G.nj * G.nk;
-    for (int c = 0; c < 2; ++c) {
-      if (is64(0))
-        tail_copy((lds<double> *)lv[0].rhs[c], (const double *)G.rhs[c], n);
-      else
-        tail_copy((lds<float> *)lv[0].rhs[c], (const float *)G.rhs[c], n);
-    }
-    __syncthreads();
-  }
-  // down: pre-smoothing and restriction
-  for (int q = 0; q < last; ++q) {
-    const LevelDev &L = lv[q];
-    const LevelDev &C = lv[q + 1];
-    int buf = 0;
-    bool zero = true;
-    if (is64(q)) {
-      tail_relax<double>(L, nu1, buf, zero);
-      if (zero) tail_fill_zero<double>(L, buf);
-      tail_restrict<double, double>(L, C, buf);
-    } else {
-      tail_relax<float>(L, nu1, buf, zero);
-      if (zero) tail_fill_zero<float>(L, buf);
-      if (is64(q + 1))
-        tail_restrict<float, double>(L, C, buf);
-      else
-        tail_restrict<float, float>(L, C, buf);
-    }
-  }
   // coarsest level of the block (always FP64)
-  if (do_exact) {
-    coarse_exact_body<true>(lv[last], Q[0], Q[1], Q[2], lam[0], lam[1], lam[2], A, Bs, fin);
-  } else {
+  auto coarsest = [&]() __attribute__((always_inline)) {
+    const TailLev &L = Z;
+    if (do_exact) {
+      const unsigned q1 = eo + tail_eig_axis(L.ni), q2 = q1 + tail_eig_axis(L.nj),
+                     sc = q2 + tail_eig_axis(L.nk), n3 = (unsigned)(L.ni * L.nj * L.nk) * 8u;
+      auto at = [&](unsigned o) { return (ldsd)((lds<char> *)smem + o); };
+      coarse_exact_lds(L.ni, L.nj, L.nk, L.H, at(L.rhs), at(L.rhs + L.rs),
+                       at(L.phi + (unsigned)(2 * fin) * L.ps),
+                       at(L.phi + (unsigned)(2 * fin + 1) * L.ps), at(eo), at(q1), at(q2),
+                       at(eo + tail_eig_q(L.ni)), at(q1 + tail_eig_q(L.nj)),
+                       at(q2 + tail_eig_q(L.nk)), at(sc), at(sc + n3));
+      return;
+    }
     int buf = 0;
-    bool zero = true;
-    tail_relax<double>(lv[last], nu1, buf, zero);
-    tail_relax<double>(lv[last], nu2, buf, zero);
-    if (zero) tail_fill_zero<double>(lv[last], buf);
-  }
-  // up: prolongation and post-smoothing
-  for (int q = last - 1; q >= 0; --q) {
-    const LevelDev &F = lv[q];
-    const LevelDev &C = lv[q + 1];
-    const int fb = nu1 & 1;
-    int buf = fb;
-    bool zero = false;
-    if (is64(q)) {
-      tail_prolong<double, double>(F, C, fb, fin);
-      tail_relax<double>(F, nu2, buf, zero);
-    } else {
-      if (is64(q + 1))
-        tail_prolong<float, double>(F, C, fb, fin);
+    tail_relax<double>(L, nu1 + nu2, buf, true, false);
+  };
+  // One copy of every piece of code, run level by level: the kernel runs each
+  // only a few times per launch, and its instruction fetches count (a cold
+  // kilobyte of code costs ~0.8 us here).
+#pragma clang loop unroll(disable)
+  for (int q = 0, up = 0; q >= 0; up ? --q : ++q) {
+    // one level on the way down (up = 0) or up; the coarsest turns around
+    if (q == last) {
+      coarsest();
+      up = 1;
+      continue;
+    }
+    const TailLev L = tail_level<MIXED>(G, q, nl), C = tail_level<MIXED>(G, q + 1, nl);
+    const bool c64 = !MIXED || q + 1 == last;
+    int buf = up ? nu1 & 1 : 0;
+    if (up) {
+      if (c64)
+        tail_prolong<T, double>(L, C, buf, fin);
       else
-        tail_prolong<float, float>(F, C, fb, fin);
-      tail_relax<float>(F, nu2, buf, zero);
+        tail_prolong<T, T>(L, C, buf, fin);
+    }
+    tail_relax<T>(L, up ? nu2 : nu1, buf, !up, !up);
+    if (!up) {
+      if (c64)
+        tail_sum8<T, double>(L, C, buf);
+      else
+        tail_sum8<T, T>(L, C, buf);
     }
   }
   // top level's phi (buffer fin) back to global
-  {
-    const LevelDev &G = levs[top];
-    const int n = G.H * G.nj * G.nk;
-    for (int c = 0; c < 2; ++c) {
-      if (is64(0))
-        tail_copy((double *)G.phi[fin][c], (const lds<double> *)lv[0].phi[fin][c], n);
-      else
-        tail_copy((float *)G.phi[fin][c], (const lds<float> *)lv[0].phi[fin][c], n);
-    }
+  for (int c = 0; c < 2; ++c) {
+    const unsigned o = L0.phi + (unsigned)(2 * fin + c) * L0.ps;
+    if (top64)
+      tail_copy((gmem<double> *)G.phi[fin][c], (const lds<double> *)(smem + o), L0.n);
+    else
+      tail_copy((gmem<float> *)G.phi[fin][c], (const lds<float> *)(smem + o), L0.n);
   }
 }
 
@@ -4561,12 +4921,46 @@ void launch_finalize(hipStream_t s, const int *tile_begin, int nblocks, const Re
   hipLaunchKernelGGL(k_finalize, dim3(nblocks), dim3(FIN_THREADS), 0, s, tile_begin, partials, out);
 }
 
-void launch_coarse_exact(hipStream_t s, const Tile *tiles, int ntiles, const LevelDev *levs,
-                         const int *active, const double *const *eig_q,
+void launch_coarse_exact(hipStream_t s, const Tile *tiles, int ntiles, const ExactGrid &grid,
+                         const LevelDev *levs, const int *active, const double *const *eig_q,
                          const double *const *eig_l, double *const *scratch, int buf) {
   if (ntiles <= 0) return;
-  hipLaunchKernelGGL(k_coarse_exact, dim3(ntiles), dim3(256), 0, s, tiles, levs, active, eig_q,
-                     eig_l, scratch, buf);
+  if (grid.plane_lds) {
+    const dim3 gp(ntiles, grid.planes), gc(ntiles, grid.chunks);
+    hipLaunchKernelGGL(k_exact_plane<true>, gp, dim3(256), grid.plane_lds, s, tiles, levs, active,
+                       eig_q, scratch, buf);
+    hipLaunchKernelGGL(k_exact_cols, gc, dim3(256), grid.cols_lds, s, tiles, levs, active, eig_q,
+                       eig_l, scratch);
+    hipLaunchKernelGGL(k_exact_plane<false>, gp, dim3(256), grid.plane_lds, s, tiles, levs, active,
+                       eig_q, scratch, buf);
+    return;
+  }
+  for (int p = 0; p < 6; ++p)
+    hipLaunchKernelGGL(k_exact_pass, dim3(ntiles, grid.blocks), dim3(256), 0, s, tiles, levs,
+                       active, eig_q, eig_l, scratch, buf, p);
+}
+
+void exact_grid_add(ExactGrid &g, const LevelDev &L, size_t lds_budget) {
+  const size_t p0 = exact_pitch(L.ni), p1 = exact_pitch(L.nj), p2 = exact_pitch(L.nk);
+  const size_t plane = 8 * (L.ni * p0 + L.nj * p1 + 2 * p0 * L.nj);
+  const size_t cols = 8 * (L.nk * p2 + (2 * (size_t)L.nk + 1) * EXACT_COLS + L.nk);
+  const size_t n = (size_t)L.ni * L.nj * L.nk;
+  g.split = g.split && plane <= lds_budget && cols <= lds_budget;
+  g.plane_lds = g.split ? std::max(g.plane_lds, plane) : 0;
+  g.cols_lds = g.split ? std::max(g.cols_lds, cols) : 0;
+  g.planes = std::max(g.planes, L.nk);
+  g.chunks = std::max(g.chunks, (L.ni * L.nj + EXACT_COLS - 1) / EXACT_COLS);
+  g.blocks = std::max<unsigned>(g.blocks, (unsigned)std::min<size_t>((n + 255) / 256, 4096));
+}
+
+hipError_t exact_allow_lds(size_t lds_bytes) {
+  for (const void *f : {(const void *)k_exact_plane<true>, (const void *)k_exact_plane<false>,
+                        (const void *)k_exact_cols}) {
+    const hipError_t e =
+        hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 void launch_vtail(hipStream_t s, const Tile *tiles, int ntiles, const LevelDev *levs,
@@ -4589,21 +4983,23 @@ hipError_t vtail_allow_lds(size_t lds_bytes) {
                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
 }
 
-size_t vtail_lds_bytes(const LevelDev *levs_host, int top, bool mixed, bool exact) {
+size_t vtail_lds_bytes(const LevelDev *levs_host, int top, bool mixed, bool exact, bool padded) {
   size_t off = 0;
   int last = top, nl = 0;
   for (int d = top; d >= 0 && nl < TAIL_MAX_LEVELS; d = levs_host[d].coarser, ++nl) {
     const LevelDev &L = levs_host[d];
     const bool is64 = !mixed || L.coarser < 0;
     const size_t half = (size_t)L.H * L.nj * L.nk * (is64 ? 8 : 4);
-    off += 6 * ((half + 15) & ~(size_t)15);
+    off += 6 * ((half + 15) & ~(size_t)15) + (padded ? 16 : 0);
     last = d;
   }
   const LevelDev &C = levs_host[last];
   if (exact && C.finer >= 0) {
     const int na[3] = {C.ni, C.nj, C.nk};
-    for (int a = 0; a < 3; ++a) off += (size_t)na[a] * na[a] * 8 + (((size_t)na[a] * 8 + 15) & ~(size_t)15);
-    off += 2 * (size_t)na[0] * na[1] * na[2] * 8;
+    for (int a = 0; a < 3; ++a)
+      off += padded ? tail_eig_axis(na[a])
+                    : (size_t)na[a] * na[a] * 8 + (((size_t)na[a] * 8 + 15) & ~(size_t)15);
+    off += 2 * (size_t)C.ni * C.nj * C.nk * 8;
   }
   return off;
 }

@@ -277,6 +277,7 @@ struct h3dmg_handle {
   std::vector<TileSet> prol_nc, prol_c;     // fine natural at g; L_b > g+1 / == g+1
   std::vector<TileSet> nat_nc, nat_c;       // natural at g (zero fill)
   std::vector<TileSet> coarse_list;         // blocks whose coarsest level is g
+  std::vector<ExactGrid> coarse_grid;       // the exact solve's grid over them
   TileSet fine_tiles;                       // residual tiles of level 1, lev = block
   TileSet update_tiles;                     // p += pp tiles, lev = block
   std::vector<int> tile_begin;              // per block range in fine_tiles
@@ -658,8 +659,8 @@ void enqueue_vcycle(h3dmg_handle *h, bool red1 = false) {
       int b = 0;
       if (exact && g > 1) {
         const int out = (nu1 + nu2) & 1;
-        launch_coarse_exact(h->stream, h->coarse_list[g].d, h->coarse_list[g].n(), h->d_levs,
-                            h->d_active, (const double *const *)h->d_eig_q,
+        launch_coarse_exact(h->stream, h->coarse_list[g].d, h->coarse_list[g].n(),
+                            h->coarse_grid[g], h->d_levs, h->d_active, (const double *const *)h->d_eig_q,
                             (const double *const *)h->d_eig_l, h->d_scratch, out);
         b = out;
         z = false;
@@ -950,6 +951,16 @@ h3dmg_status validate_blocks(const h3dmg_block *blocks, int nblocks, const h3dmg
   return validate_neighbours(blocks, nblocks, P);
 }
 
+// dynamic LDS the exact solve's kernels may use (a process-wide attribute of
+// the kernels: set once, to the device's budget)
+size_t exact_lds_budget(const h3dmg_handle *h) {
+  static std::once_flag once;
+  static bool ok = false;
+  const size_t budget = h->lds_budget;
+  std::call_once(once, [budget]() { ok = exact_allow_lds(budget) == hipSuccess; });
+  return ok ? budget : std::min<size_t>(budget, 65536);
+}
+
 // Lays out and uploads a handle over `blocks`.  `fresh` (pooled handles):
 // blocks whose region starts new (zero p and f, the exact solve's tables
 // uploaded); the others carry theirs over.  With `region_bytes` set, only
@@ -1127,8 +1138,13 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
   h->nat_nc.assign(Lm + 2, {});
   h->nat_c.assign(Lm + 2, {});
   h->coarse_list.assign(Lm + 2, {});
-  for (int b = 0; b < nblocks; ++b)
-    h->coarse_list[h->blk[b].L].h.push_back(Tile{h->blk[b].desc[h->blk[b].L], b, 0, 0});
+  h->coarse_grid.assign(Lm + 2, {});
+  for (int b = 0; b < nblocks; ++b) {
+    const int g = h->blk[b].L, d = h->blk[b].desc[g];
+    h->coarse_list[g].h.push_back(Tile{d, b, 0, 0});
+    if (h->prm.coarse == H3DMG_COARSE_EXACT)
+      exact_grid_add(h->coarse_grid[g], h->levs[d], exact_lds_budget(h));
+  }
   for (int g = 1; g <= Lm; ++g)
     for (int b = 0; b < nblocks; ++b) {
       const BlockInfo &B = h->blk[b];
@@ -1678,31 +1694,42 @@ h3dmg_status upload_relax(h3dmg_handle *h, int g, bool sync) {
 }
 
 // LDS the tail needs when it starts at level g (max over the blocks that
-// reach g; 0 when none does)
-size_t tail_lds_at(const h3dmg_handle *h, int g) {
+// reach g; 0 when none does); padded: as the kernel lays it out
+size_t tail_lds_at(const h3dmg_handle *h, int g, bool padded) {
   size_t need = 0;
   for (const BlockInfo &B : h->blk)
     if (B.L >= g)
       need = std::max(need, vtail_lds_bytes(h->levs.data(), B.desc[g], is_mixed(h),
-                                            h->prm.coarse == H3DMG_COARSE_EXACT));
+                                            h->prm.coarse == H3DMG_COARSE_EXACT, padded));
   return need;
 }
 
-// Automatic tail level: the first level from which every block's remaining
-// levels fit in one workgroup's LDS; none when no level does.
-// The tail's one workgroup per block is bound by its CU's VALU issue, so it
-// pays for the exact solves of the blocks' coarsest levels (all of them in
-// one launch, without their levels' global round trips), not for levels
-// above them, and not for a smoothed coarsest level: with the exact solve,
-// the first level from the shallowest block's coarsest down whose tail fits
-// in LDS; otherwise off.  Measured on MI355X (single 32^3 to 256^3 blocks
-// and batches of 2 to 48 blocks of mixed sizes, both precisions).
+// Automatic tail level, 0 < g < the coarsest: the first level from which every
+// block's remaining levels fit in one workgroup's LDS and whose cells the tail
+// kernel keeps in registers (TAIL_FAST_ENTRIES per colour: 16^3), for handles
+// whose blocks all have the same number of levels.  Measured per cycle, tail
+// from 16^3 | every level its own launches, us: one 64^3 of 4 levels, mixed,
+// exact coarsest 122 | 135, FP64 smoothed 119 | 137; 48 of them 458 | 489 and
+// 653 | 677; 96 of 32^3, FP64 300 | 351.  The coarsest level alone is left to
+// its launches: an exact solve there takes 62 (16^3 blocks) to 74 (28^3) us a
+// two-level cycle in the tail's one workgroup, 55 to 59 spread over the chip,
+// a smoothed one as long either way.  Handles of unequal depths: with the
+// exact solve the first level from the shallowest block's coarsest down that
+// fits (the deeper blocks' levels and all exact solves in one launch).
 int auto_tail_level(const h3dmg_handle *h) {
-  if (h->prm.coarse != H3DMG_COARSE_EXACT) return h->Lmax + 1;
+  const bool exact = h->prm.coarse == H3DMG_COARSE_EXACT;
   int t0 = h->Lmax;
   for (const BlockInfo &B : h->blk) t0 = std::min(t0, B.L);
-  for (int g = std::max(t0, 1); g <= h->Lmax; ++g) {
-    const size_t need = tail_lds_at(h, g);
+  const bool equal = t0 == h->Lmax;
+  for (int g = 1; g <= h->Lmax; ++g) {
+    bool want = equal ? g < h->Lmax : exact && g >= t0;
+    if (equal)
+      for (const BlockInfo &B : h->blk) {
+        const LevelDev &L = h->levs[B.desc[g]];
+        want = want && (long)L.H * L.nj * L.nk <= TAIL_FAST_ENTRIES;
+      }
+    if (!want) continue;
+    const size_t need = tail_lds_at(h, g, false);
     if (need > 0 && need <= h->lds_budget) return g;
   }
   return h->Lmax + 1;
@@ -1710,14 +1737,14 @@ int auto_tail_level(const h3dmg_handle *h) {
 
 h3dmg_status gen_tail(h3dmg_handle *h) {
   h->tail_lt = h->tail_req > 0 ? h->tail_req : auto_tail_level(h);
-  h->tail_lds = h->tail_lt <= h->Lmax ? tail_lds_at(h, h->tail_lt) : 0;
-  if (h->tail_lds > h->lds_budget) {
+  h->tail_lds = h->tail_lt <= h->Lmax ? tail_lds_at(h, h->tail_lt, true) : 0;
+  if (h->tail_lds > 0 && tail_lds_at(h, h->tail_lt, false) > h->lds_budget) {
     const int lt = h->tail_lt;
     h->tail_req = 0;
     h->tail_lt = h->Lmax + 1;
     h->tail_lds = 0;
     return fail(H3DMG_ERR_ARG, "tail level %d needs %zu bytes of LDS (at most %zu here)", lt,
-                tail_lds_at(h, lt), h->lds_budget);
+                tail_lds_at(h, lt, false), h->lds_budget);
   }
   // The permitted LDS is a process-wide attribute of the kernel: set once,
   // to the device's whole budget, so that handles of different tail sizes
@@ -1725,7 +1752,7 @@ h3dmg_status gen_tail(h3dmg_handle *h) {
   if (h->tail_lds > 65536) {
     static std::once_flag once;
     static hipError_t once_err = hipSuccess;
-    const size_t budget = h->lds_budget;
+    const size_t budget = h->lds_budget + VTAIL_LDS_PAD;
     std::call_once(once, [budget]() { once_err = vtail_allow_lds(budget); });
     HIP_TRY(once_err);
   }
@@ -1733,7 +1760,9 @@ h3dmg_status gen_tail(h3dmg_handle *h) {
   ts.h.clear();
   if (h->tail_lt <= h->Lmax)
     for (int b = 0; b < h->nb; ++b)
-      if (h->blk[b].L >= h->tail_lt) ts.h.push_back(Tile{h->blk[b].desc[h->tail_lt], b, 0, 0, 0, 0});
+      if (h->blk[b].L >= h->tail_lt) 
+        ts.h.push_back(
+            Tile{h->blk[b].desc[h->tail_lt], b, 0, 0, h->blk[b].L - h->tail_lt + 1, 0});
   return H3DMG_OK;
 }
 
@@ -2091,7 +2120,7 @@ h3dmg_status create_locked(const h3dmg_block *blocks, int nblocks, const h3dmg_p
   int lds = 0;
   if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
     lds = 65536;
-  // the tail kernel's static LDS (its level descriptors) comes on top
+  // (the tail kernel's alignment, VTAIL_LDS_PAD, comes on top)
   h->lds_budget = lds > 8192 ? (size_t)lds - 8192 : 0;
   if (stream) {
     h->stream = (hipStream_t)stream;
