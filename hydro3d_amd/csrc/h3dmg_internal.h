@@ -97,8 +97,8 @@ struct RedPartial {
 // T = storage type of the level (double or float).
 // one colour half-sweep of the red-black smoother over a tile list whose
 // tiles are all `depth` (1, 2 or 4) planes deep: kinds 0 (march tile, y/z
-// interior), 3 (march tile touching a y/z face), or, on levels one cell wide
-// in x (depth 1 only), 1 (general boundary march) and 2 (x faces)
+// interior), 3 (march tile touching a y/z face); depth 0: natural tiles, cell
+// by cell (blocks with neighbours, levels one cell wide in x)
 // A launch whose tiles all belong to one descriptor (lev; lev2: its finer
 // level for a restriction, its coarser for a prolongation; blk its block):
 // the kernel then reads the tile, the descriptors and the block's flag at

@@ -153,10 +153,9 @@ __device__ __forceinline__ double fine_value(const FineDev *__restrict__ fine, i
 // zero != 0: the level holds zeros in buffer src (the first sweep after
 // mgrestr zeroed phi, mgsolver.for:655-662, or pp = 0 at the finest level).
 //
-// Three tile kinds share a half-sweep (one launch, k_rb_sweep): march tiles
-// whose cells have all y/z neighbours inside the block (no ghost logic at
-// all), the other march tiles, and x-face tiles for the cells on the two x
-// faces (i = 0, ni-1), which the march tiles skip.
+// Two tile kinds share a half-sweep (one launch, k_rb_sweep): tiles whose
+// cells have all y/z neighbours inside the block, and the others; blocks with
+// neighbours and levels one cell wide in x go cell by cell (k_cell_sweep).
 //
 // Work layout of the march kernels.  A lane owns two adjacent entries m0,
 // m0+1 of one row of the colour arrays; L.lpr lanes cover a row segment and a
@@ -245,113 +244,6 @@ __device__ __forceinline__ double wave_shift(double v, int shr) {
 // scalar base and a 32-bit lane offset).
 template <class T>
 using gmem = __attribute__((address_space(1))) T;
-
-template <class T, bool INNER>
-__device__ __forceinline__ void march_tile(const Tile &t, const LevelDev *__restrict__ levs,
-                                           int colour, int src, int zero) {
-  const LevelDev &L = levs[t.lev];
-  typedef typename Vec2<T>::type v2;
-  const int lpr = L.lpr;
-  const int lane = (int)threadIdx.x;
-  const int rl = lane & (lpr - 1);
-  const int m0 = t.x0 + 2 * rl;
-  const int j = t.y0 + (int)threadIdx.y * (64 / lpr) + lane / lpr;
-  const int ni = L.ni, nj = L.nj, nk = L.nk, H = L.H;
-  const bool col_ok = m0 < H && j < nj;  // H even: m0 + 1 < H as well
-  const unsigned row = (unsigned)H, plane = (unsigned)H * (unsigned)nj;
-  const gmem<T> *O = (const gmem<T> *)(colour == 0 ? L.phi[src][1] : L.phi[1 - src][0]);
-  const gmem<T> *R = (const gmem<T> *)L.rhs[colour];
-  gmem<T> *D = (gmem<T> *)L.phi[1 - src][colour];
-  const bool zero_int = zero && colour == 0;  // uniform
-  const bool zero_ghost = zero != 0;
-  // lanes outside the level read a valid entry (clamped) and store nothing
-  const int jc = min(j, nj - 1);
-  const unsigned cbase = (unsigned)jc * row + (unsigned)min(m0, H - 2);
-  const v2 vz = {T(0), T(0)};
-  // tiles that do not start/end a row: the end lanes fetch entries m0-1 and
-  // m0+2 from the neighbouring tile's range (uniform test, then one lane)
-  const bool tile_left = t.x0 > 0, tile_right = t.x0 + 2 * lpr < H;
-  const T cx = (T)L.cx, cy = (T)L.cy, cz = (T)L.cz;
-  const T ap_in = T(-1) * (cx + cx + cy + cy + cz + cz);
-  const T inv_in = T(1) / ap_in;
-
-  // byte offsets in 32 bits (arrays < 4 GiB): scalar base + lane offset
-  auto ld2 = [&](const gmem<T> *a, unsigned off) -> v2 {
-    return *(const gmem<v2> *)((const gmem<char> *)a + off * (unsigned)sizeof(T));
-  };
-  auto ld1 = [&](const gmem<T> *a, unsigned off) -> T {
-    return *(const gmem<T> *)((const gmem<char> *)a + off * (unsigned)sizeof(T));
-  };
-  auto own = [&](int k) -> v2 {
-    if (zero_int || (!INNER && (unsigned)k >= (unsigned)nk)) return vz;
-    return ld2(O, (unsigned)k * plane + cbase);
-  };
-  auto ghost = [&](int x, int y, int z) -> T {
-    return zero_ghost ? T(0) : level_value<T>(levs, t.lev, src, x, y, z);
-  };
-
-  int k = t.z0;
-  const int k1 = t.z1;
-  v2 o_m = own(k - 1), o_c = own(k);
-  for (; k < k1; ++k) {
-    const v2 o_p = own(k + 1);
-    const unsigned q = (unsigned)k * plane + cbase;
-    v2 S2 = vz, N2 = vz;
-    if (!zero_int) {
-      // jc: the lane's row, clamped like cbase (lanes beyond the level load
-      // in-bounds rows; their results are not stored)
-      if (INNER || jc > 0) S2 = ld2(O, q - row);
-      if (INNER || jc + 1 < nj) N2 = ld2(O, q + row);
-    }
-    const v2 R2 = ld2(R, q);
-    T lf = wave_shift(o_c.y, 1);  // entry m0-1: lane-1's second entry
-    T rt = wave_shift(o_c.x, 0);  // entry m0+2: lane+1's first entry
-    if (tile_left && !zero_int && rl == 0) lf = ld1(O, q - 1);
-    if (tile_right && !zero_int && rl == lpr - 1) rt = ld1(O, q + 2);
-    const int s = (colour + j + k) & 1;
-    // x-neighbours of the cells i0 = 2*m0 + s and i1 = i0 + 2
-    const T W0 = s ? o_c.x : lf;
-    const T E0 = s ? o_c.y : o_c.x;
-    const T W1 = s ? o_c.y : o_c.x;
-    const T E1 = s ? rt : o_c.y;
-    const int i0 = 2 * m0 + s, i1 = i0 + 2;
-    T out0, out1;
-    if (INNER) {
-      const T sum0 = cx * W0 + cx * E0 + cy * S2.x + cy * N2.x + cz * o_m.x + cz * o_p.x;
-      const T sum1 = cx * W1 + cx * E1 + cy * S2.y + cy * N2.y + cz * o_m.y + cz * o_p.y;
-      out0 = div_ap(R2.x - sum0, ap_in, inv_in);
-      out1 = div_ap(R2.y - sum1, ap_in, inv_in);
-    } else {
-      const T Wv[2] = {W0, W1}, Ev[2] = {E0, E1};
-      T o[2];
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const int i = e ? i1 : i0;
-        const T S = (jc > 0) ? (e ? S2.y : S2.x) : ghost(i, -1, k);
-        const T N = (jc + 1 < nj) ? (e ? N2.y : N2.x) : ghost(i, nj, k);
-        const T B = (k > 0) ? (e ? o_m.y : o_m.x) : ghost(i, jc, -1);
-        const T Tt = (k + 1 < nk) ? (e ? o_p.y : o_p.x) : ghost(i, jc, nk);
-        const Coef<T> c = cell_coef<T>(L, i, jc, k);
-        const T sum = c.aw * Wv[e] + c.ae * Ev[e] + c.as * S + c.an * N + c.ab * B + c.at * Tt;
-        o[e] = div_ap((e ? R2.y : R2.x) - sum, c.ap, T(1) / c.ap);
-      }
-      out0 = o[0];
-      out1 = o[1];
-    }
-    // cells on the x faces belong to the x-face tiles of the same launch
-    const bool w0 = col_ok && i0 > 0 && i0 < ni - 1, w1 = col_ok && i1 < ni - 1;
-    gmem<char> *dq = (gmem<char> *)D + q * (unsigned)sizeof(T);
-    if (w0 && w1) {
-      const v2 o = {out0, out1};
-      *(gmem<v2> *)dq = o;
-    } else {
-      if (w0) *(gmem<T> *)dq = out0;
-      if (w1) *(gmem<T> *)(dq + sizeof(T)) = out1;
-    }
-    o_m = o_c;
-    o_c = o_p;
-  }
-}
 
 // March tile of KB planes with every load issued up front (one memory round
 // trip per tile): the own-column window (KB+2 planes), rows j-1 and j+1, the
@@ -547,49 +439,177 @@ __device__ __forceinline__ void march_tile_fast(const Tile &t, const LevelDev &L
   }
 }
 
-// The cells of colour `colour` on the two x faces (i = 0 and i = ni-1), with
-// the full ghost treatment.  The tile covers 256 rows j = t.x0 + ... of plane
-// k = t.y0; one thread per row does both faces.
+// Cell-parallel kernels for blocks with neighbours, blocks one cell wide in
+// x, and the variable-density operator.  The value across each face of the
+// block lies in the block itself (a wall, a periodic wrap) or in the
+// neighbour; which arrays and how they are laid out is the same for the whole
+// workgroup (scalar registers), so a cell selects each neighbour's address
+// instead of branching and its loads are all in flight together: a kernel
+// with a branch per ghost read them one memory latency after the other.
 template <class T>
-__device__ __forceinline__ void xface_tile(const Tile &t, const LevelDev *__restrict__ levs,
-                                           int colour, int src, int zero) {
-  const LevelDev &L = levs[t.lev];
-  const int j = t.x0 + (int)threadIdx.x + TILE_X * (int)threadIdx.y;
-  const int k = t.y0;
-  if (j >= L.nj || k >= L.nk) return;
-  const T *nb_int = colour == 0 ? (const T *)L.phi[src][1] : (const T *)L.phi[1 - src][0];
-  const bool zero_int = zero && colour == 0;
-  const bool zero_ghost = zero != 0;
-  auto nb = [&](int x, int y, int z) -> T {
-    const bool ghost = (unsigned)x >= (unsigned)L.ni || (unsigned)y >= (unsigned)L.nj ||
-                       (unsigned)z >= (unsigned)L.nk;
-    if (!ghost) return zero_int ? T(0) : nb_int[cidx(L.H, L.nj, x, y, z)];
-    return zero_ghost ? T(0) : level_value<T>(levs, t.lev, src, x, y, z);
-  };
-  for (int side = 0; side < 2; ++side) {
-    const int i = side ? L.ni - 1 : 0;
-    if (side && i == 0) break;
-    if (((i + j + k) & 1) != colour) continue;
-    const Coef<T> c = cell_coef<T>(L, i, j, k);
-    const T W = nb(i - 1, j, k), E = nb(i + 1, j, k);
-    const T S = nb(i, j - 1, k), N = nb(i, j + 1, k);
-    const T B = nb(i, j, k - 1), Tt = nb(i, j, k + 1);
-    const size_t q = cidx(L.H, L.nj, i, j, k);
-    const T r = ((const T *)L.rhs[colour])[q];
-    const T sum = c.aw * W + c.ae * E + c.as * S + c.an * N + c.ab * B + c.at * Tt;
-    ((T *)L.phi[1 - src][colour])[q] = div_ap(r - sum, c.ap, T(1) / c.ap);
+struct FaceSrc {
+  const gmem<T> *p[6][2];  // face f, by the colour of the cell at the face
+  unsigned wH, wx, eH, ex;  // x neighbours: row pitch and the cell's entry
+  unsigned sn, sy, nn, ny;  // y neighbours: rows per plane and the row
+  unsigned bz, tz;          // z neighbours: the plane
+};
+
+template <class T>
+__device__ __forceinline__ FaceSrc<T> face_src(const LevelDev *__restrict__ levs,
+                                               const LevelDev &L, int src) {
+  FaceSrc<T> S;
+  const int nl[3] = {L.ni, L.nj, L.nk};
+  int at[6];
+  const LevelDev *P[6];
+#pragma unroll
+  for (int f = 0; f < 6; ++f) {
+    const int a = f >> 1;
+    P[f] = L.nbr[f] >= 0 ? &levs[L.nbr[f]] : &L;
+    const int np = a == 0 ? P[f]->ni : a == 1 ? P[f]->nj : P[f]->nk;
+    const bool wall = wall_face(L, f), low = (f & 1) == 0;
+    // a wall mirrors the cell itself; else the far cell of the block across
+    at[f] = wall ? (low ? 0 : nl[a] - 1) : low ? np - 1 : 0;
+    const int flip = wall ? 0 : ((low ? np : nl[a]) - 1) & 1;
+    S.p[f][0] = (const gmem<T> *)P[f]->phi[src][flip];
+    S.p[f][1] = (const gmem<T> *)P[f]->phi[src][1 - flip];
+  }
+  S.wH = (unsigned)P[0]->H;
+  S.wx = (unsigned)at[0] >> 1;
+  S.eH = (unsigned)P[1]->H;
+  S.ex = (unsigned)at[1] >> 1;
+  S.sn = (unsigned)P[2]->nj;
+  S.sy = (unsigned)at[2];
+  S.nn = (unsigned)P[3]->nj;
+  S.ny = (unsigned)at[3];
+  S.bz = (unsigned)at[4];
+  S.tz = (unsigned)at[5];
+  return S;
+}
+
+// The six neighbours of cell (i, j, k) of colour c: O the other colour's
+// array inside the block; zg: ghosts hold zero.  e: the cell's entry.
+template <class T>
+__device__ __forceinline__ void cell_neighbours(const FaceSrc<T> &S, const LevelDev &L,
+                                                const gmem<T> *O, int c, int i, int j, int k,
+                                                unsigned e, bool zg, T (&v)[6]) {
+  const int s = i & 1;
+  const unsigned H = (unsigned)L.H, nj = (unsigned)L.nj, plane = H * nj, m = (unsigned)i >> 1;
+  const unsigned uj = (unsigned)j, uk = (unsigned)k;
+  const bool g[6] = {i == 0, i >= L.ni - 1, j == 0, j == L.nj - 1, k == 0, k == L.nk - 1};
+  const unsigned in[6] = {s ? e : e - 1, s ? e + 1 : e, e - H, e + H, e - plane, e + plane};
+  const unsigned gh[6] = {(uk * nj + uj) * S.wH + S.wx,    (uk * nj + uj) * S.eH + S.ex,
+                          (uk * S.sn + S.sy) * H + m,      (uk * S.nn + S.ny) * H + m,
+                          (S.bz * nj + uj) * H + m,        (S.tz * nj + uj) * H + m};
+#pragma unroll
+  for (int f = 0; f < 6; ++f) {
+    const gmem<T> *const b = g[f] ? (c ? S.p[f][1] : S.p[f][0]) : O;
+    v[f] = b[g[f] ? gh[f] : in[f]];
+  }
+#pragma unroll
+  for (int f = 0; f < 6; ++f)
+    if (zg && g[f]) v[f] = T(0);
+}
+
+// the coefficients of entry e of colour c: aw, ae, as, an, ab, at, ap
+template <class T, bool LSM>
+__device__ __forceinline__ void cell_coefs(const LevelDev &L, int c, int i, int j, int k,
+                                           unsigned e, T (&a)[7]) {
+  if constexpr (LSM) {
+#pragma unroll
+    for (int q = 0; q < 7; ++q)
+      a[q] = ((const gmem<double> *)L.lsm)[(size_t)(2 * q + c) * L.lsm_half + e];
+  } else {
+    const Coef<T> C = cell_coef<T>(L, i, j, k);
+    a[0] = C.aw, a[1] = C.ae, a[2] = C.as, a[3] = C.an, a[4] = C.ab, a[5] = C.at, a[6] = C.ap;
   }
 }
 
+// One colour half-sweep (mgsolver.for:553-605; LSM: with per-cell
+// coefficients) over natural tiles (TILE_X x TILE_Y cells of one plane): 128
+// threads, one per cell of the colour.  The buffer rules are k_rb_sweep's.
+// Bound by the launch and one round of loads.  Averages over four levels, us,
+// with a branch per ghost | now: 64 joined blocks of 64x8x64, 18.3 | 5.9
+// (restriction 74 | 11, prolongation 33 | 15); 96x64x80 with variable density
+// 6.1 | 3.9 (restriction 70 | 6.3).
+template <class T, bool LSM>
+__global__ void __launch_bounds__(128)
+    k_cell_sweep(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
+                 const int *__restrict__ active, int colour, int src, int zero, int ntiles) {
+  const Tile t = tiles[xcd_remap((int)blockIdx.x, ntiles)];
+  const LevelDev &L = levs[t.lev];
+  if (!active[L.blk]) return;
+  const FaceSrc<T> S = face_src<T>(levs, L, src);
+  const int q = (int)threadIdx.x + TILE_X * (int)threadIdx.y;
+  const int jt = t.y0 + q / (TILE_X / 2), k = t.z0;
+  const int mt = (t.x0 >> 1) + q % (TILE_X / 2);
+  // lanes beyond the level read a valid cell and store nothing
+  const int j = min(jt, L.nj - 1), m = min(mt, (L.ni - 1) >> 1);
+  const int i = 2 * m + ((colour + j + k) & 1);
+  const unsigned e = (unsigned)cidx(L.H, L.nj, i, j, k);
+  T v[6], a[7];
+  const T r = ((const gmem<T> *)L.rhs[colour])[e];
+  cell_coefs<T, LSM>(L, colour, i, j, k, e, a);
+  if (zero && colour == 0) {  // every neighbour is zero
+#pragma unroll
+    for (int f = 0; f < 6; ++f) v[f] = T(0);
+  } else {
+    cell_neighbours<T>(S, L,
+                       (const gmem<T> *)(colour == 0 ? L.phi[src][1] : L.phi[1 - src][0]), colour,
+                       i, j, k, e, zero != 0, v);
+  }
+  const T sum =
+      a[0] * v[0] + a[1] * v[1] + a[2] * v[2] + a[3] * v[3] + a[4] * v[4] + a[5] * v[5];
+  if (jt < L.nj && mt == m && i < L.ni)
+    ((gmem<T> *)L.phi[1 - src][colour])[e] = div_ap(r - sum, a[6], T(1) / a[6]);
+}
+
+// Restriction (mgrestr, mgsolver.for:693-756) over natural tiles of the coarse
+// level: grid.y is the tile's row; wavefront y of a workgroup forms, for 64
+// coarse cells, the two fine residuals r = f - (aw*W + ae*E + as*S + an*N +
+// ab*B + at*T + ap*P) of row y & 1, plane y >> 1 of the children, and
+// wavefront 0 sums the eight i fastest, then j, then k, times 0.125.  (A
+// thread per coarse cell walked its children one after the other, and a level
+// had too few threads.)
+template <class Tf, class Tc, bool LSM>
+__global__ void __launch_bounds__(NTHREADS)
+    k_cell_restrict(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
+                    const int *__restrict__ active, int src_f, int ntiles) {
+  __shared__ Tf res[8][TILE_X];
+  const Tile t = tiles[xcd_remap((int)blockIdx.x, ntiles)];
+  const LevelDev &C = levs[t.lev];
+  const int jc = t.y0 + (int)blockIdx.y, kc = t.z0;
+  if (!active[C.blk] || jc >= C.nj) return;
+  const LevelDev &F = levs[C.finer];
+  const FaceSrc<Tf> S = face_src<Tf>(levs, F, src_f);
+  const int lane = (int)threadIdx.x, ch = (int)threadIdx.y;
+  const int lt = t.x0 + lane, l = min(lt, C.ni - 1);
+  const int j = 2 * jc + (ch & 1), k = 2 * kc + (ch >> 1);
+#pragma unroll
+  for (int d = 0; d < 2; ++d) {
+    const int i = 2 * l + d, c = (i + j + k) & 1;
+    const unsigned e = (unsigned)cidx(F.H, F.nj, i, j, k);
+    Tf v[6], a[7];
+    const Tf f = ((const gmem<Tf> *)F.rhs[c])[e];
+    const Tf P = ((const gmem<Tf> *)F.phi[src_f][c])[e];
+    cell_coefs<Tf, LSM>(F, c, i, j, k, e, a);
+    cell_neighbours<Tf>(S, F, (const gmem<Tf> *)F.phi[src_f][1 - c], c, i, j, k, e, false, v);
+    res[2 * ch + d][lane] = f - (a[0] * v[0] + a[1] * v[1] + a[2] * v[2] + a[3] * v[3] +
+                                 a[4] * v[4] + a[5] * v[5] + a[6] * P);
+  }
+  __syncthreads();
+  if (ch != 0 || lt >= C.ni) return;
+  Tc acc = (Tc)res[0][lane];
+#pragma unroll
+  for (int q = 1; q < 8; ++q) acc = acc + (Tc)res[q][lane];
+  ((gmem<Tc> *)C.rhs[(l + jc + kc) & 1])[cidx(C.H, C.nj, l, jc, kc)] = Tc(0.125) * acc;
+}
+
 // One launch per colour half-sweep over a level.  Every tile of the list is
-// KB planes deep: a march tile (kind 0: y/z interior, kind 3: touching a y/z
-// face) or, on levels one cell wide in x (KB = 1 launches only), a general
-// boundary march tile (kind 1) or an x-face tile (kind 2); the tiles write
-// disjoint cells.  One instantiation per depth keeps each one's register
+// KB planes deep: kind 0 has every y/z neighbour inside the block, kind 3
+// touches a y/z face; the tiles write disjoint cells.  One instantiation per depth keeps each one's register
 // count to what its own tiles need.
 template <class T, int KB>
-__device__ __forceinline__ void rb_dispatch(const Tile &t, const LevelDev &L,
-                                            const LevelDev *__restrict__ levs, int colour, int src,
+__device__ __forceinline__ void rb_dispatch(const Tile &t, const LevelDev &L, int colour, int src,
                                             int zero, bool on);
 
 // In the one-descriptor kernels, one empty asm statement takes the tile,
@@ -618,31 +638,25 @@ __global__ void __launch_bounds__(NTHREADS)
                  "s"(L.nk), "s"(L.H), "s"(L.per), "s"(L.lpr), "s"(L.cx), "s"(L.cy), "s"(L.cz),
                  "s"(L.phi[0][0]), "s"(L.phi[0][1]), "s"(L.phi[1][0]), "s"(L.phi[1][1]),
                  "s"(L.rhs[0]), "s"(L.rhs[1]));
-    rb_dispatch<T, KB>(t, L, levs, colour, src, zero, on != 0);
+    rb_dispatch<T, KB>(t, L, colour, src, zero, on != 0);
   } else {
     const LevelDev &L = levs[t.lev];
     if (!active[L.blk]) return;
-    rb_dispatch<T, KB>(t, L, levs, colour, src, zero, true);
+    rb_dispatch<T, KB>(t, L, colour, src, zero, true);
   }
 }
 
 template <class T, int KB>
-__device__ __forceinline__ void rb_dispatch(const Tile &t, const LevelDev &L,
-                                            const LevelDev *__restrict__ levs, int colour, int src,
+__device__ __forceinline__ void rb_dispatch(const Tile &t, const LevelDev &L, int colour, int src,
                                             int zero, bool on) {
   // the interior neighbours are zeros in the red half of a zero-state sweep
   const bool zint = zero && colour == 0;
   if (t.kind == 0) {
     zint ? march_tile_fast<T, KB, true, false>(t, L, colour, src, zero, on)
          : march_tile_fast<T, KB, false, false>(t, L, colour, src, zero, on);
-  } else if (t.kind == 3) {
+  } else {
     zint ? march_tile_fast<T, KB, true, true>(t, L, colour, src, zero, on)
          : march_tile_fast<T, KB, false, true>(t, L, colour, src, zero, on);
-  } else if (KB == 1 && on) {
-    if (t.kind == 1)
-      march_tile<T, false>(t, levs, colour, src, zero);
-    else
-      xface_tile<T>(t, levs, colour, src, zero);
   }
 }
 
@@ -1252,43 +1266,6 @@ __global__ void __launch_bounds__(NTHREADS)
     restrict_tile_fast<Tf, Tc, KBC, true>(t, C, F, src_f, true, zbuf);
 }
 
-// Restriction for blocks with neighbours: one thread per coarse cell of
-// natural tiles (TILE_X x TILE_Y cells of one coarse plane); the fine
-// residual of each of the eight children, its neighbours read through
-// resolve_cell where they are ghosts, in restrict_tile_fast's arithmetic:
-// r = f - (aw*W + ae*E + as*S + an*N + ab*B + at*T + ap*P), the children
-// summed i fastest, then j, then k, times 0.125 (mgsolver.for:693-756).
-template <class Tf, class Tc>
-__global__ void __launch_bounds__(NTHREADS)
-    k_restrict_gen(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
-                   const int *__restrict__ active, int src_f) {
-  const Tile t = tiles[blockIdx.x];
-  const LevelDev &C = levs[t.lev];
-  if (!active[C.blk]) return;
-  const int l = t.x0 + (int)threadIdx.x, jc = t.y0 + (int)threadIdx.y, kc = t.z0;
-  if (l >= C.ni || jc >= C.nj || kc >= C.nk) return;
-  const int fd = C.finer;
-  const LevelDev &F = levs[fd];
-  auto val = [&](int x, int y, int z) -> Tf {
-    if ((unsigned)x < (unsigned)F.ni && (unsigned)y < (unsigned)F.nj &&
-        (unsigned)z < (unsigned)F.nk)
-      return ((const Tf *)F.phi[src_f][(x + y + z) & 1])[cidx(F.H, F.nj, x, y, z)];
-    return level_value<Tf>(levs, fd, src_f, x, y, z);
-  };
-  Tc acc = Tc(0);
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int i = 2 * l + (q & 1), j = 2 * jc + ((q >> 1) & 1), k = 2 * kc + (q >> 2);
-    const Coef<Tf> c = cell_coef<Tf>(F, i, j, k);
-    const Tf f = ((const Tf *)F.rhs[(i + j + k) & 1])[cidx(F.H, F.nj, i, j, k)];
-    const Tf r = f - (c.aw * val(i - 1, j, k) + c.ae * val(i + 1, j, k) + c.as * val(i, j - 1, k) +
-                      c.an * val(i, j + 1, k) + c.ab * val(i, j, k - 1) + c.at * val(i, j, k + 1) +
-                      c.ap * val(i, j, k));
-    acc = q == 0 ? (Tc)r : acc + (Tc)r;
-  }
-  ((Tc *)C.rhs[(l + jc + kc) & 1])[cidx(C.H, C.nj, l, jc, kc)] = Tc(0.125) * acc;
-}
-
 // ---------------------------------------------------------------------------
 // mgcorr (mgsolver.for:828-896): fine += trilinear interpolation of coarse.
 // Fine padded index ip = 2*icp + d with icp the coarse padded index; the
@@ -1303,7 +1280,11 @@ __global__ void __launch_bounds__(NTHREADS)
 // Tile::x0 = first l, y0 = first m (TILE_Y per tile), z0 = n.  The fine
 // level is updated in place (each fine cell by exactly one thread).
 // GEN: blocks with neighbours -- the coarse ghost corners (edges and corners
-// included) are read through resolve_cell, possibly in another block.
+// included) may lie in another block.  A wavefront's corner rows and planes
+// are the same for all its lanes, and in x a corner is inside the row or
+// across one of its two ends: twelve lanes resolve the rows and their ends
+// (resolve_cell) into LDS and every lane picks, instead of following the
+// neighbour table for sixteen corners, one after the other.
 // ONE, scalar arguments: as k_rb_sweep (one_lev the fine descriptor,
 // one_lev2 its coarser level).
 template <class Tf, class Tc, bool GEN, bool ONE>
@@ -1327,6 +1308,28 @@ __global__ void __launch_bounds__(NTHREADS)
   const int l = t.x0 + 2 * (int)threadIdx.x;
   const int m = t.y0 + (int)threadIdx.y;
   const int n = t.z0;
+  // GEN: the wavefront's corner rows (y, z), inside the block's x range,
+  // before it and after it: the row's arrays by the parity of x, and the x of
+  // the end cell
+  struct RowSrc {
+    const gmem<Tc> *p[2];
+    int x;
+  };
+  __shared__ RowSrc rows[GEN ? TILE_Y : 1][12];
+  if (GEN) {
+    const int q = (int)threadIdx.x;
+    if (q < 12) {
+      int x = q % 3 == 0 ? 0 : q % 3 == 1 ? -1 : C.ni;
+      int y = min(m, C.nj) - 1 + (q / 3) % 2, z = min(n, C.nk) - 1 + q / 6;
+      const LevelDev &P = levs[resolve_cell(levs, F.coarser, x, y, z)];
+      const size_t row = ((size_t)z * P.nj + y) * P.H;
+      RowSrc &r = rows[threadIdx.y][q];
+      r.p[0] = (const gmem<Tc> *)P.phi[src_c][(y + z) & 1] + row;
+      r.p[1] = (const gmem<Tc> *)P.phi[src_c][(y + z + 1) & 1] + row;
+      r.x = x;
+    }
+    __syncthreads();
+  }
   if (2 * l >= F.ni || m > C.nj || n > C.nk) return;
   const bool two = 2 * l + 2 < F.ni;  // entry l+1 holds cells (F.ni is even)
   const bool px = C.per & 1, py = C.per & 2, pz = C.per & 4;
@@ -1348,8 +1351,11 @@ __global__ void __launch_bounds__(NTHREADS)
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         if (GEN) {
-          cv[a][b][c] = level_value<Tc>(levs, F.coarser, src_c, min(l - 1 + a, two ? l + 2 : l + 1),
-                                        m - 1 + b, n - 1 + c);
+          const int x = min(l - 1 + a, two ? l + 2 : l + 1);
+          const int at = x < 0 ? 1 : x >= C.ni ? 2 : 0;
+          const RowSrc r = rows[threadIdx.y][at + 3 * (b + 2 * c)];
+          const int xx = at == 0 ? x : r.x;
+          cv[a][b][c] = ((xx & 1) ? r.p[1] : r.p[0])[xx >> 1];
         } else {
           const unsigned off = ((unsigned)zc[c] * (unsigned)C.nj + (unsigned)yc[b]) *
                                    (unsigned)C.H + (unsigned)(xc[a] >> 1);
@@ -2871,36 +2877,6 @@ __global__ void k_lsm_coef(const LevelDev *__restrict__ lev_dev, const double *_
   for (int a = 0; a < 7; ++a) L.lsm[(size_t)(2 * a + colour) * L.lsm_half + e] = c[a];
 }
 
-// one colour half-sweep (mgsolver.for:553-605 with per-cell coefficients):
-// natural tiles (TILE_X x TILE_Y cells of one plane), threads of the other
-// colour idle; ghosts and the stale-ghost buffer rule as in march_tile
-__global__ void __launch_bounds__(NTHREADS)
-    k_lsm_sweep(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
-                const int *__restrict__ active, int colour, int src, int zero) {
-  const Tile t = tiles[blockIdx.x];
-  const LevelDev &L = levs[t.lev];
-  if (!active[L.blk]) return;
-  const int i = t.x0 + (int)threadIdx.x, j = t.y0 + (int)threadIdx.y, k = t.z0;
-  if (i >= L.ni || j >= L.nj || k >= L.nk || ((i + j + k) & 1) != colour) return;
-  const double *O = (const double *)(colour == 0 ? L.phi[src][1] : L.phi[1 - src][0]);
-  const bool zero_int = zero && colour == 0, zero_ghost = zero != 0;
-  auto nb = [&](int x, int y, int z) -> double {
-    const bool ghost = (unsigned)x >= (unsigned)L.ni || (unsigned)y >= (unsigned)L.nj ||
-                       (unsigned)z >= (unsigned)L.nk;
-    if (!ghost) return zero_int ? 0.0 : O[cidx(L.H, L.nj, x, y, z)];
-    return zero_ghost ? 0.0 : level_value<double>(levs, t.lev, src, x, y, z);
-  };
-  const size_t e = cidx(L.H, L.nj, i, j, k);
-  double c[7];
-  for (int a = 0; a < 7; ++a) c[a] = lsm_coef(L, a, colour)[e];
-  const double W = nb(i - 1, j, k), E = nb(i + 1, j, k);
-  const double S = nb(i, j - 1, k), N = nb(i, j + 1, k);
-  const double B = nb(i, j, k - 1), T = nb(i, j, k + 1);
-  const double r = ((const double *)L.rhs[colour])[e];
-  const double sum = c[0] * W + c[1] * E + c[2] * S + c[3] * N + c[4] * B + c[5] * T;
-  ((double *)L.phi[1 - src][colour])[e] = (r - sum) / c[6];
-}
-
 // finest-level residual r = f - A p with per-cell coefficients into the
 // level-1 rhs, with per-tile partial sum of r^2 and max |r| (the residual
 // tiles' work layout: lane l holds cells 2l and 2l+1 of one row)
@@ -2941,49 +2917,6 @@ __global__ void __launch_bounds__(NTHREADS)
   }
   block_reduce(ss, am);
   if (threadIdx.x == 0 && threadIdx.y == 0) partials[ti] = RedPartial{ss, am};
-}
-
-// restriction (mgrestr, mgsolver.for:693-756) with per-cell coefficients:
-// a thread per coarse cell of the restriction tile's layout; the eight fine
-// residuals summed i fastest, then j, k, times 0.125
-__global__ void __launch_bounds__(NTHREADS)
-    k_lsm_restrict(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
-                   const int *__restrict__ active, int src_f) {
-  const Tile t = tiles[xcd_remap((int)blockIdx.x, (int)gridDim.x)];
-  const LevelDev &C = levs[t.lev];
-  if (!active[C.blk]) return;
-  const LevelDev &F = levs[C.finer];
-  const int lpr = C.lpr1;
-  const int lane = (int)threadIdx.x;
-  const int jc = t.y0 + (int)threadIdx.y * (64 / lpr) + lane / lpr;
-  auto res = [&](int i, int j, int k) -> double {
-    const int c = (i + j + k) & 1;
-    const size_t e = cidx(F.H, F.nj, i, j, k);
-    double cf[7];
-    for (int a = 0; a < 7; ++a) cf[a] = lsm_coef(F, a, c)[e];
-    auto nb = [&](int x, int y, int z) { return level_value<double>(levs, C.finer, src_f, x, y, z); };
-    return ((const double *)F.rhs[c])[e] -
-           (cf[0] * nb(i - 1, j, k) + cf[1] * nb(i + 1, j, k) + cf[2] * nb(i, j - 1, k) +
-            cf[3] * nb(i, j + 1, k) + cf[4] * nb(i, j, k - 1) + cf[5] * nb(i, j, k + 1) +
-            cf[6] * nb(i, j, k));
-  };
-  // the tile's two halves of lpr coarse cells, one cell per lane
-  for (int half = 0; half < 2; ++half) {
-  const int l = t.x0 + half * lpr + (lane & (lpr - 1));
-  if (l >= C.ni || jc >= C.nj) continue;
-  for (int kc = t.z0; kc < t.z1; ++kc) {
-    const int i0 = 2 * l, j0 = 2 * jc, k0 = 2 * kc;
-    double acc = res(i0, j0, k0);
-    acc = acc + res(i0 + 1, j0, k0);
-    acc = acc + res(i0, j0 + 1, k0);
-    acc = acc + res(i0 + 1, j0 + 1, k0);
-    acc = acc + res(i0, j0, k0 + 1);
-    acc = acc + res(i0 + 1, j0, k0 + 1);
-    acc = acc + res(i0, j0 + 1, k0 + 1);
-    acc = acc + res(i0 + 1, j0 + 1, k0 + 1);
-    ((double *)C.rhs[(l + jc + kc) & 1])[cidx(C.H, C.nj, l, jc, kc)] = 0.125 * acc;
-  }
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -4681,6 +4614,11 @@ template <class T>
 void launch_rb_sweep(hipStream_t s, const Tile *tiles, int ntiles, int depth, const LevelDev *levs,
                      const int *active, int colour, int src, int zero, OneDesc one) {
   if (ntiles <= 0) return;
+  if (depth == 0) {  // natural tiles, cell by cell
+    hipLaunchKernelGGL((k_cell_sweep<T, false>), dim3(ntiles), dim3(TILE_X, TILE_Y / 2), 0, s, tiles,
+                       levs, active, colour, src, zero, ntiles);
+    return;
+  }
   auto k = one.lev >= 0 ? (depth == 4   ? k_rb_sweep<T, 4, true>
                            : depth == 2 ? k_rb_sweep<T, 2, true>
                                         : k_rb_sweep<T, 1, true>)
@@ -4709,8 +4647,8 @@ void launch_lsm_coef(hipStream_t s, const LevelDev *lev_dev, const double *dens,
 void launch_lsm_sweep(hipStream_t s, const Tile *tiles, int ntiles, const LevelDev *levs,
                       const int *active, int colour, int src, int zero) {
   if (ntiles <= 0) return;
-  hipLaunchKernelGGL(k_lsm_sweep, dim3(ntiles), tile_block(), 0, s, tiles, levs, active, colour,
-                     src, zero);
+  hipLaunchKernelGGL((k_cell_sweep<double, true>), dim3(ntiles), dim3(TILE_X, TILE_Y / 2), 0, s,
+                     tiles, levs, active, colour, src, zero, ntiles);
 }
 
 void launch_gs_tiles(hipStream_t s, const Tile *tiles, int ntiles, const LevelDev *levs,
@@ -4830,7 +4768,8 @@ void launch_lsm_residual(hipStream_t s, const Tile *tiles, int ntiles, const Fin
 void launch_lsm_restrict(hipStream_t s, const Tile *tiles, int ntiles, const LevelDev *levs,
                          const int *active, int src_f) {
   if (ntiles <= 0) return;
-  hipLaunchKernelGGL(k_lsm_restrict, dim3(ntiles), tile_block(), 0, s, tiles, levs, active, src_f);
+  hipLaunchKernelGGL((k_cell_restrict<double, double, true>), dim3(ntiles, TILE_Y), tile_block(), 0,
+                     s, tiles, levs, active, src_f, ntiles);
 }
 
 template <class T>
@@ -4846,8 +4785,8 @@ void launch_restrict(hipStream_t s, const Tile *tiles, int ntiles, int depth, co
                      const int *active, int src_f, OneDesc one, int zbuf) {
   if (ntiles <= 0) return;
   if (depth == 0) {  // natural tiles of the coarse level, blocks with neighbours
-    hipLaunchKernelGGL((k_restrict_gen<Tf, Tc>), dim3(ntiles), tile_block(), 0, s, tiles, levs,
-                       active, src_f);
+    hipLaunchKernelGGL((k_cell_restrict<Tf, Tc, false>), dim3(ntiles, TILE_Y), tile_block(), 0, s,
+                       tiles, levs, active, src_f, ntiles);
     return;
   }
   auto k = one.lev >= 0 ? (depth == 4   ? k_restrict<Tf, Tc, 4, true>

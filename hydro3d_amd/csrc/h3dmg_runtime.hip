@@ -156,30 +156,22 @@ int launch_depth(long cols, long target, int want, int cap, const std::vector<in
 // remap then hands every XCD a contiguous slab): per chunk of kb planes the
 // march tiles (2*lpr entries x 4*(64/lpr) rows x kb planes), kind 0 when
 // every y/z neighbour of the tile is inside the block, kind 3 otherwise; both
-// update the x-face cells of their rows.  Levels one cell wide in x use the
-// general boundary tiles (kind 1) and separate x-face tiles (kind 2, 256
-// rows of one plane each).
+// update the x-face cells of their rows.
 int march_tiles_xy(const LevelDev &L) {
   const int xs = 2 * L.lpr, ys = TILE_Y * (64 / L.lpr);
   return ((L.H + xs - 1) / xs) * ((L.nj + ys - 1) / ys);
 }
 
-// kb planes per tile; kb divides L.nk; `general`: kinds 1 and 2 (every
-// ghost through the neighbour table: blocks with neighbours)
-void add_tiles_march(TileSet &ts, int lev, const LevelDev &L, int kb, bool general) {
+// kb planes per tile; kb divides L.nk
+void add_tiles_march(TileSet &ts, int lev, const LevelDev &L, int kb) {
   const int xs = 2 * L.lpr, ys = TILE_Y * (64 / L.lpr);
   const int nx = L.H, ny = L.nj, nz = L.nk;
-  const bool faces_in_tiles = L.ni >= 2 && !general;
   for (int z = 0; z < nz; z += kb) {
     const int z1 = std::min(z + kb, nz);
-    if (!faces_in_tiles)
-      for (int zz = z; zz < z1; ++zz)
-        for (int y = 0; y < ny; y += NTHREADS) ts.h.push_back(Tile{lev, y, zz, 0, 0, 2});
     for (int y = 0; y < ny; y += ys)
       for (int x = 0; x < nx; x += xs) {
         const bool inner = y >= 1 && y + ys <= ny - 1 && z >= 1 && z1 <= nz - 1;
-        const int kind = faces_in_tiles ? (inner ? 0 : 3) : 1;
-        ts.h.push_back(Tile{lev, x, y, z, z1, kind});
+        ts.h.push_back(Tile{lev, x, y, z, z1, inner ? 0 : 3});
       }
   }
 }
@@ -620,7 +612,7 @@ void enqueue_vcycle(h3dmg_handle *h, bool red1 = false) {
         z_nc[g - 1] = 0;
       }
       if (h->lsm) {
-        for (const TileSet *ts : {&h->restr_nc[g], &h->restr_c[g]})
+        for (const TileSet *ts : {&h->nat_nc[g], &h->nat_c[g]})
           launch_lsm_restrict(h->stream, ts->d, ts->n(), h->d_levs, h->d_active, buf_nc[g - 1]);
       } else if (h->restr_nc[g].n()) {
         const int zbuf = red_by_restr ? 1 - buf_nc[g] : -1;
@@ -1528,7 +1520,8 @@ h3dmg_status gen_relax(h3dmg_handle *h, int g) {
     ts.nat = grp == 0 ? &h->nat_nc[g] : &h->nat_c[g];
     // one depth for the whole launch: the requested planes, or enough for
     // ~4096 workgroups over the group's blocks; at most 4, a power of two
-    // dividing every block's nk; 1 where a level is one cell wide in x
+    // dividing every block's nk; 0 (cell by cell) for blocks with neighbours
+    // and where a level is one cell wide in x
     auto member = [&](const BlockInfo &B) { return B.L >= g && (grp == 1) == (B.L == g); };
     long cols = 0;
     bool general = false;
@@ -1652,17 +1645,20 @@ h3dmg_status gen_relax(h3dmg_handle *h, int g) {
               for (int x = 0; x < L.ni; x += FUSED_X)
                 ts.h.push_back(Tile{B.desc[g], x, y, z, std::min(z + FUSED_Z, L.nk), 4});
         }
+    } else if (general) {
+      ts.depth = 0;
+      ts.h = ts.nat->h;
     } else {
-      const int kb = general ? 1 : launch_depth(cols, 4096, h->march_kb[g], 4, nks);
+      const int kb = launch_depth(cols, 4096, h->march_kb[g], 4, nks);
       ts.depth = kb;
       for (int b = 0; b < h->nb; ++b) {
         const BlockInfo &B = h->blk[b];
         if (!member(B)) continue;
-        add_tiles_march(ts, B.desc[g], h->levs[B.desc[g]], kb, h->connected);
+        add_tiles_march(ts, B.desc[g], h->levs[B.desc[g]], kb);
       }
     }
     for (const Tile &t : ts.h)
-      if (t.kind != 2 && t.kind != 4 && t.z1 - t.z0 != ts.depth)
+      if (ts.depth && t.kind != 4 && t.z1 - t.z0 != ts.depth)
         return fail(H3DMG_ERR_ARG, "internal: tile depth");
     set_one(ts, h->levs, 0);
   }
@@ -3541,7 +3537,7 @@ h3dmg_status h3dmg_dbg_restrict(h3dmg_handle *h, int level) {
   if (st) return st;
   const bool f64 = !is_mixed(h);
   if (h->lsm) {
-    for (const TileSet *ts : {&h->restr_nc[level], &h->restr_c[level]})
+    for (const TileSet *ts : {&h->nat_nc[level], &h->nat_c[level]})
       launch_lsm_restrict(h->stream, ts->d, ts->n(), h->d_levs, h->d_active, 0);
   } else if (h->restr_nc[level].n()) {
     if (f64)
