@@ -145,6 +145,11 @@ template <class T>
 void launch_residual(hipStream_t s, const Tile *tiles, int ntiles, int depth, const FineDev *fine,
                      const LevelDev *levs, const int *active, RedPartial *partials, int use_p,
                      int zbuf = -1);
+// f, level-1 rhs and ||f||'s partials of one block (its tiles, `planes` deep,
+// and partials) from a dense array
+template <class T>
+void launch_set_rhs(hipStream_t s, const Tile *tiles, int ntiles, int planes, const FineDev *fine,
+                    const LevelDev *levs, const double *src, RedPartial *partials);
 template <class T>
 void launch_update(hipStream_t s, const Tile *tiles, int ntiles, const FineDev *fine,
                    const LevelDev *levs, const int *active, int buf);

@@ -1833,6 +1833,69 @@ __global__ void __launch_bounds__(NTHREADS)
   if (threadIdx.x == 0 && threadIdx.y == 0) partials[ti] = RedPartial{ss, am};
 }
 
+// A block's right-hand side from a dense array: f, the level-1 rhs, and the
+// partial sums of ||f||, tile by tile in k_residual_gen's layout and order.
+// One pass over memory: a pack and a pass over every block's tiles took 59 +
+// 54 us at 256^3 (float level 1), now 63; for each of 48 blocks 4 + 16, now
+// 8.5.
+template <class T, int KB>
+__global__ void __launch_bounds__(NTHREADS)
+    k_set_rhs(const Tile *__restrict__ tiles, const FineDev *__restrict__ fine,
+              const LevelDev *__restrict__ levs, const double *__restrict__ src,
+              RedPartial *__restrict__ partials) {
+  const int ti = xcd_remap((int)blockIdx.x, (int)gridDim.x);
+  const Tile t = tiles[ti];
+  const FineDev &F = fine[t.lev];
+  const LevelDev &L = levs[t.lev];
+  const int lpr = F.lpr, lane = (int)threadIdx.x;
+  const int j = t.y0 + (int)threadIdx.y * (64 / lpr) + lane / lpr;
+  const int ni = F.ni, nj = F.nj;
+  gmem<double> *const F0 = (gmem<double> *)F.f[0], *const F1 = (gmem<double> *)F.f[1];
+  gmem<T> *const R0 = (gmem<T> *)L.rhs[0], *const R1 = (gmem<T> *)L.rhs[1];
+  const gmem<double> *const A = (const gmem<double> *)src;
+  double ss = 0.0, am = 0.0;
+  // every load first: a small block has few workgroups (lanes and planes
+  // outside the block read a cell of it and store nothing)
+  const int jc = min(j, nj - 1);
+  double fa[2][KB], fb[2][KB];
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    const int l = min(t.x0 + half * lpr + (lane & (lpr - 1)), (ni - 1) >> 1);
+#pragma unroll
+    for (int p = 0; p < KB; ++p) {
+      const size_t row = (size_t)((unsigned)(t.z0 + p) * (unsigned)nj + (unsigned)jc) * ni;
+      fa[half][p] = A[row + 2 * l];
+      fb[half][p] = A[row + min(2 * l + 1, ni - 1)];
+    }
+  }
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    const int l = t.x0 + half * lpr + (lane & (lpr - 1));
+    const bool ok = 2 * l < ni && j < nj, b_ok = 2 * l + 1 < ni && j < nj;
+#pragma unroll
+    for (int p = 0; p < KB; ++p) {
+      const int k = t.z0 + p;
+      const unsigned q = ((unsigned)k * (unsigned)nj + (unsigned)j) * (unsigned)F.H + (unsigned)l;
+      const double a = fa[half][p], b = fb[half][p];
+      const bool ca = (j + k) & 1;
+      if (ok) {
+        (ca ? F1 : F0)[q] = a;
+        (ca ? R1 : R0)[q] = (T)a;
+        ss += a * a;
+        am = fmax(am, fabs(a));
+      }
+      if (b_ok) {
+        (ca ? F0 : F1)[q] = b;
+        (ca ? R0 : R1)[q] = (T)b;
+        ss += b * b;
+        am = fmax(am, fabs(b));
+      }
+    }
+  }
+  block_reduce(ss, am);
+  if (threadIdx.x == 0 && threadIdx.y == 0) partials[ti] = RedPartial{ss, am};
+}
+
 // p = p + (pp - ppref) with ppref = 0 (newsolv_mg.for:39-49), streamed over
 // the colour arrays of one block (pad entries included: they are never read
 // as cells); pp is the level-1 correction in buffer `buf`.  Tile::x0 is the
@@ -1902,65 +1965,87 @@ __global__ void __launch_bounds__(FIN_THREADS)
 // in the same order and IEEE operations: per block ||r|| = sqrt(ss), rel =
 // ||r|| / ||f|| (one global rel for blocks joined by faces), rmax = amax *
 // rfac * vol; done when (REF) it >= max(min_cycles, 2) and the global rmax <
-// tol, else it >= min_cycles and rel <= the block's tolerance.  One thread:
-// a handful of blocks, serial in block order like the host's sums.
-__device__ void decide_body(const DecideBlock *__restrict__ blocks, DecideState *__restrict__ state,
-                            DecideCtl *__restrict__ ctl, const RedPartial *__restrict__ stats,
-                            int *__restrict__ active, char *__restrict__ ring,
-                            const DecideParams *__restrict__ prm_in) {
+// tol, else it >= min_cycles and rel <= the block's tolerance.  One wavefront,
+// a lane per block (one thread for all of them waits for memory block after
+// block: 48 blocks took 54 us, now 7.6); sums are taken in block order
+// like the host's, the maxima do not depend on it.
+__device__ __forceinline__ void decide_body(const DecideBlock *__restrict__ blocks,
+                                            DecideState *__restrict__ state,
+                                            DecideCtl *__restrict__ ctl,
+                                            const RedPartial *__restrict__ stats,
+                                            int *__restrict__ active, char *__restrict__ ring,
+                                            const DecideParams *__restrict__ prm_in) {
   const DecideParams prm = *prm_in;
-  const int nb = prm.nb;
+  const int nb = prm.nb, lane = (int)threadIdx.x;
   const int it = ctl->it + 1;
   double grel = 0.0;
   if (prm.connected) {
     double ss = 0.0, ff = 0.0;
-    for (int b = 0; b < nb; ++b)
-      if (blocks[b].enabled) {
-        ss += stats[b].ss;
-        ff += blocks[b].fnorm * blocks[b].fnorm;
+    for (int b0 = 0; b0 < nb; b0 += 64) {
+      const int b = b0 + lane;
+      const bool on = b < nb && blocks[b].enabled;
+      const double s = on ? stats[b].ss : 0.0, f = on ? blocks[b].fnorm * blocks[b].fnorm : 0.0;
+      for (int q = 0; q < min(64, nb - b0); ++q) {
+        ss += __shfl(s, q);
+        ff += __shfl(f, q);
       }
+    }
     grel = ff > 0 ? sqrt(ss) / sqrt(ff) : sqrt(ss);
   }
   double worst = 0.0, gmax = 0.0;
-  int bad = 0;
-  for (int b = 0; b < nb; ++b) {
-    const DecideBlock &B = blocks[b];
+  bool bad = false;
+  for (int b = lane; b < nb; b += 64) {
+    const DecideBlock B = blocks[b];
+    const RedPartial r = stats[b];
+    DecideState s = state[b];
+    const int a = active[b];
     if (!B.enabled) continue;
-    const double nrm = sqrt(stats[b].ss);
-    if (active[b]) {
-      state[b].rel = prm.connected ? grel : B.fnorm > 0 ? nrm / B.fnorm : nrm;
-      state[b].rmax = stats[b].amax * prm.rfac * B.vol;
+    const double nrm = sqrt(r.ss);
+    if (a) {
+      s.rel = prm.connected ? grel : B.fnorm > 0 ? nrm / B.fnorm : nrm;
+      s.rmax = r.amax * prm.rfac * B.vol;
+      state[b] = s;
     }
-    if (!isfinite(nrm)) bad = 1;
-    worst = worst < state[b].rel ? state[b].rel : worst;
-    gmax = gmax < state[b].rmax ? state[b].rmax : gmax;
+    if (!isfinite(nrm)) bad = true;
+    worst = worst < s.rel ? s.rel : worst;
+    gmax = gmax < s.rmax ? s.rmax : gmax;
   }
-  int all_done = 1;
-  for (int b = 0; b < nb; ++b) {
-    const DecideBlock &B = blocks[b];
+  bad = __any(bad);
+  for (int w = 32; w > 0; w >>= 1) {
+    const double x = __shfl_xor(worst, w), g = __shfl_xor(gmax, w);
+    worst = worst < x ? x : worst;
+    gmax = gmax < g ? g : gmax;
+  }
+  char *slot = ring + (size_t)(it & 1) * decide_slot_bytes(nb);
+  DecideState *rs = (DecideState *)(slot + sizeof(DecideCtl));
+  RedPartial *rp = (RedPartial *)(rs + nb);
+  int *ra = (int *)(rp + nb);
+  bool going = false;
+  for (int b = lane; b < nb; b += 64) {
+    const DecideBlock B = blocks[b];
+    const RedPartial r = stats[b];
+    const DecideState s = state[b];
+    int a = active[b];
     bool done;
     if (!B.enabled)
       done = true;
     else if (prm.ref)
       done = it >= max(prm.min_cycles, 2) && gmax < prm.tol;
     else
-      done = it >= prm.min_cycles && state[b].rel <= B.tol;
+      done = it >= prm.min_cycles && s.rel <= B.tol;
     // a non-finite norm ends the loop: a cycle queued behind this one does
     // nothing
-    if (done || bad) active[b] = 0;
-    if (active[b]) all_done = 0;
+    if (done || bad) active[b] = a = 0;
+    if (a) going = true;
+    rs[b] = s;
+    rp[b] = r;
+    ra[b] = a;
   }
-  const DecideCtl c{it, all_done, bad, 0, prm.ref ? gmax : worst};
-  *ctl = c;
-  char *slot = ring + (size_t)(it & 1) * decide_slot_bytes(nb);
-  *(DecideCtl *)slot = c;
-  DecideState *rs = (DecideState *)(slot + sizeof(DecideCtl));
-  RedPartial *rp = (RedPartial *)(rs + nb);
-  int *ra = (int *)(rp + nb);
-  for (int b = 0; b < nb; ++b) {
-    rs[b] = state[b];
-    rp[b] = stats[b];
-    ra[b] = active[b];
+  going = __any(going);
+  if (lane == 0) {
+    const DecideCtl c{it, going ? 0 : 1, bad ? 1 : 0, 0, prm.ref ? gmax : worst};
+    *ctl = c;
+    *(DecideCtl *)slot = c;
   }
 }
 
@@ -1975,12 +2060,15 @@ __global__ void __launch_bounds__(FIN_THREADS)
                       int *__restrict__ active, char *__restrict__ ring,
                       const DecideParams *__restrict__ prm, unsigned *__restrict__ arrived) {
   finalize_body(tile_begin, partials, out);
-  if (threadIdx.x != 0) return;
-  __threadfence();  // this block's statistics before the count
-  const unsigned n = gridDim.x;
-  if (atomicAdd(arrived, 1u) != n - 1) return;
+  if (threadIdx.x >= 64) return;
+  int last = 0;
+  if (threadIdx.x == 0) {
+    __threadfence();  // this block's statistics before the count
+    last = atomicAdd(arrived, 1u) == gridDim.x - 1;
+    if (last) *arrived = 0u;
+  }
+  if (!__builtin_amdgcn_readfirstlane(last)) return;
   __threadfence();  // every block's statistics after it
-  *arrived = 0u;
   decide_body(blocks, state, ctl, out, active, ring, prm);
 }
 // ---------------------------------------------------------------------------
@@ -3386,26 +3474,37 @@ __global__ void __launch_bounds__(256)
 }
 
 // ---- layout conversion ---------------------------------------------------
-__global__ void k_pack_fine(const FineDev *__restrict__ fd, int which,
-                            const double *__restrict__ src, int ni, int nj, int nk) {
-  const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t n = (size_t)ni * nj * nk;
-  if (q >= n) return;
-  const int i = (int)(q % ni), j = (int)((q / ni) % nj), k = (int)(q / ((size_t)ni * nj));
+// p (which 0) or f of a block to and from a dense array: a thread per entry of
+// both colours in a row of lp lanes (a power of two), 32-bit row arithmetic.
+// (A thread per cell divided 64-bit indexes: 59 in and 69 us out at 256^3, now
+// 53 and 44.)
+template <bool PACK>
+__global__ void __launch_bounds__(256)
+    k_copy_fine(const FineDev *__restrict__ fd, int which, double *__restrict__ dense, int lp,
+                int xb) {
   const FineDev &F = *fd;
-  double *dst = which == 0 ? F.p[(i + j + k) & 1] : F.f[(i + j + k) & 1];
-  dst[cidx(F.H, F.nj, i, j, k)] = src[q];
-}
-
-__global__ void k_unpack_fine(const FineDev *__restrict__ fd, int which, double *__restrict__ dst,
-                              int ni, int nj, int nk) {
-  const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t n = (size_t)ni * nj * nk;
-  if (q >= n) return;
-  const int i = (int)(q % ni), j = (int)((q / ni) % nj), k = (int)(q / ((size_t)ni * nj));
-  const FineDev &F = *fd;
-  const double *src = which == 0 ? F.p[(i + j + k) & 1] : F.f[(i + j + k) & 1];
-  dst[q] = src[cidx(F.H, F.nj, i, j, k)];
+  const unsigned rb = blockIdx.x / (unsigned)xb, xt = blockIdx.x - rb * (unsigned)xb;
+  const int tid = (int)threadIdx.x, rl = tid & (lp - 1);
+  const unsigned row = rb * (unsigned)(256 / lp) + (unsigned)(tid / lp);
+  const int l = (int)(xt * (unsigned)lp) + rl, ni = F.ni;
+  if (row >= (unsigned)F.nj * (unsigned)F.nk || 2 * l >= ni) return;
+  const unsigned k = row / (unsigned)F.nj, j = row - k * (unsigned)F.nj;
+  double *const *const a = which == 0 ? F.p : F.f;
+  gmem<double> *const a0 = (gmem<double> *)a[0], *const a1 = (gmem<double> *)a[1];
+  const bool c = (j + k) & 1;
+  gmem<double> *const pa = (c ? a1 : a0) + (row * (unsigned)F.H + (unsigned)l),
+                *const pb = (c ? a0 : a1) + (row * (unsigned)F.H + (unsigned)l);
+  gmem<double> *const d = (gmem<double> *)dense + ((size_t)row * ni + 2 * l);
+  const bool two = 2 * l + 1 < ni;
+  if (PACK) {
+    const double va = d[0], vb = two ? d[1] : 0.0;
+    *pa = va;
+    if (two) *pb = vb;
+  } else {
+    const double va = *pa, vb = two ? *pb : 0.0;
+    d[0] = va;
+    if (two) d[1] = vb;
+  }
 }
 
 // p of block b with its one-cell ghost layer, dense (nk+2, nj+2, ni+2), i
@@ -4840,6 +4939,18 @@ void launch_residual(hipStream_t s, const Tile *tiles, int ntiles, int depth, co
 }
 
 template <class T>
+void launch_set_rhs(hipStream_t s, const Tile *tiles, int ntiles, int planes, const FineDev *fine,
+                    const LevelDev *levs, const double *src, RedPartial *partials) {
+  if (ntiles <= 0) return;
+  auto k = planes == 8   ? k_set_rhs<T, 8>
+           : planes == 4 ? k_set_rhs<T, 4>
+           : planes == 2 ? k_set_rhs<T, 2>
+                         : k_set_rhs<T, 1>;
+  hipLaunchKernelGGL(k, dim3(ntiles), tile_block(), 0, s, tiles, fine, levs, src,
+                     partials);
+}
+
+template <class T>
 void launch_update(hipStream_t s, const Tile *tiles, int ntiles, const FineDev *fine,
                    const LevelDev *levs, const int *active, int buf) {
   if (ntiles <= 0) return;
@@ -5004,18 +5115,29 @@ int launch_calmas4(hipStream_t s, const FineDev *fd, const double *u, const doub
   return grid;
 }
 
+static void copy_fine_grid(int ni, int nj, int nk, int &lp, int &xb, unsigned &grid) {
+  const int half = (ni + 1) / 2;
+  lp = 1;
+  while (lp < 256 && lp < half) lp *= 2;
+  xb = (half + lp - 1) / lp;
+  grid = (unsigned)xb * (unsigned)(((size_t)nj * nk + 256 / lp - 1) / (256 / lp));
+}
+
 void launch_pack_fine(hipStream_t s, const FineDev *fd, int which, const double *src, int ni,
                       int nj, int nk) {
-  const size_t n = (size_t)ni * nj * nk;
-  hipLaunchKernelGGL(k_pack_fine, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, fd, which,
-                     src, ni, nj, nk);
+  int lp, xb;
+  unsigned grid;
+  copy_fine_grid(ni, nj, nk, lp, xb, grid);
+  hipLaunchKernelGGL(k_copy_fine<true>, dim3(grid), dim3(256), 0, s, fd, which,
+                     const_cast<double *>(src), lp, xb);
 }
 
 void launch_unpack_fine(hipStream_t s, const FineDev *fd, int which, double *dst, int ni, int nj,
                         int nk) {
-  const size_t n = (size_t)ni * nj * nk;
-  hipLaunchKernelGGL(k_unpack_fine, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, fd,
-                     which, dst, ni, nj, nk);
+  int lp, xb;
+  unsigned grid;
+  copy_fine_grid(ni, nj, nk, lp, xb, grid);
+  hipLaunchKernelGGL(k_copy_fine<false>, dim3(grid), dim3(256), 0, s, fd, which, dst, lp, xb);
 }
 
 template <class T>
@@ -5068,6 +5190,10 @@ template void launch_residual<double>(hipStream_t, const Tile *, int, int, const
                                       const LevelDev *, const int *, RedPartial *, int, int);
 template void launch_residual<float>(hipStream_t, const Tile *, int, int, const FineDev *,
                                      const LevelDev *, const int *, RedPartial *, int, int);
+template void launch_set_rhs<double>(hipStream_t, const Tile *, int, int, const FineDev *,
+                                     const LevelDev *, const double *, RedPartial *);
+template void launch_set_rhs<float>(hipStream_t, const Tile *, int, int, const FineDev *,
+                                    const LevelDev *, const double *, RedPartial *);
 template void launch_update<double>(hipStream_t, const Tile *, int, const FineDev *,
                                     const LevelDev *, const int *, int);
 template void launch_update<float>(hipStream_t, const Tile *, int, const FineDev *,

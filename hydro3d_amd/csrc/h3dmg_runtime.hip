@@ -2331,28 +2331,20 @@ h3dmg_status h3dmg_set_rhs_device(h3dmg_handle *h, int b, const double *d_su) {
   h3dmg_status st = check_block(h, b);
   if (st) return st;
   if (!d_su) return fail(H3DMG_ERR_ARG, "null rhs");
-  const FineDev &F = h->fine[b];
   h->rhs_is_f = false;
-  launch_pack_fine(h->stream, h->d_fine + b, 1, d_su, F.ni, F.nj, F.nk);
-  // ||f||: residual with use_p = 0 over this block only
-  std::vector<int> act(h->nb, 0);
-  act[b] = 1;
-  HIP_TRY(hipMemcpyAsync(h->d_active, act.data(), sizeof(int) * h->nb, hipMemcpyHostToDevice,
-                         h->stream));
-  const TileSet &ft = h->fine_tiles;
+  const int t0 = h->tile_begin[b], nt = h->tile_begin[b + 1] - t0;
+  const int kb = h->fine_tiles.h[t0].z1 - h->fine_tiles.h[t0].z0;
   if (is_mixed(h))
-    launch_residual<float>(h->stream, ft.d, ft.n(), ft.depth, h->d_fine, h->d_levs, h->d_active,
-                           h->d_partials, 0);
+    launch_set_rhs<float>(h->stream, h->fine_tiles.d + t0, nt, kb, h->d_fine, h->d_levs, d_su,
+                          h->d_partials + t0);
   else
-    launch_residual<double>(h->stream, ft.d, ft.n(), ft.depth, h->d_fine, h->d_levs, h->d_active,
-                            h->d_partials, 0);
-  launch_finalize(h->stream, h->d_tile_begin, h->nb, h->d_partials, h->d_stats);
+    launch_set_rhs<double>(h->stream, h->fine_tiles.d + t0, nt, kb, h->d_fine, h->d_levs, d_su,
+                           h->d_partials + t0);
+  // this block's norm, straight to the (pinned) host statistics
+  launch_finalize(h->stream, h->d_tile_begin + b, 1, h->d_partials, h->h_stats + b);
   HIP_TRY(hipGetLastError());
-  st = read_stats(h);
-  if (st) return st;
+  HIP_TRY(hipStreamSynchronize(h->stream));
   h->blk[b].fnorm = std::sqrt(h->h_stats[b].ss);
-  st = push_active(h);
-  if (st) return st;
   h->rhs_ready = true;
   return H3DMG_OK;
 }
