@@ -127,10 +127,12 @@ template <class Tf, class Tc>
 void launch_restrict(hipStream_t s, const Tile *tiles, int ntiles, int depth, const LevelDev *levs,
                      const int *active, int src_f, OneDesc one = OneDesc{}, int zbuf = -1);
 // gen != 0: coarse ghosts read through the neighbour table (blocks with
-// neighbours)
+// neighbours); skip_red: a red half-sweep follows, red cells off the open
+// faces are left alone
 template <class Tf, class Tc>
 void launch_prolong(hipStream_t s, const Tile *tiles, int ntiles, const LevelDev *levs,
-                    const int *active, int src_f, int src_c, int gen, OneDesc one = OneDesc{});
+                    const int *active, int src_f, int src_c, int gen, int skip_red = 0,
+                    OneDesc one = OneDesc{});
 template <class T>
 void launch_fill_zero(hipStream_t s, const Tile *tiles, int ntiles, const LevelDev *levs,
                       const int *active, int buf);

@@ -674,6 +674,7 @@ void enqueue_vcycle(h3dmg_handle *h, bool red1 = false) {
       z_nc[g] = z;
     }
   }
+  const int skip_red = nu2 > 0 && h->prm.smoother == H3DMG_SMOOTH_RBGS;
   for (int g = gdown - 1; g >= 1; --g) {
     // mgcorr(g) for blocks with L_b > g
     if (h->prol_nc[g].n() || h->prol_c[g].n()) {
@@ -689,21 +690,21 @@ void enqueue_vcycle(h3dmg_handle *h, bool red1 = false) {
         }
         if (f64)
           launch_prolong<double, double>(h->stream, h->prol_nc[g].d, h->prol_nc[g].n(), h->d_levs,
-                                         h->d_active, buf_nc[g], buf_nc[g + 1], h->connected,
+                                         h->d_active, buf_nc[g], buf_nc[g + 1], h->connected, skip_red,
                                          h->prol_nc[g].one);
         else
           launch_prolong<float, float>(h->stream, h->prol_nc[g].d, h->prol_nc[g].n(), h->d_levs,
-                                       h->d_active, buf_nc[g], buf_nc[g + 1], h->connected,
+                                       h->d_active, buf_nc[g], buf_nc[g + 1], h->connected, skip_red,
                                        h->prol_nc[g].one);
       }
       if (h->prol_c[g].n()) {
         if (f64)
           launch_prolong<double, double>(h->stream, h->prol_c[g].d, h->prol_c[g].n(), h->d_levs,
-                                         h->d_active, buf_nc[g], buf_c[g + 1], h->connected,
+                                         h->d_active, buf_nc[g], buf_c[g + 1], h->connected, skip_red,
                                          h->prol_c[g].one);
         else
           launch_prolong<float, double>(h->stream, h->prol_c[g].d, h->prol_c[g].n(), h->d_levs,
-                                        h->d_active, buf_nc[g], buf_c[g + 1], h->connected,
+                                        h->d_active, buf_nc[g], buf_c[g + 1], h->connected, skip_red,
                                         h->prol_c[g].one);
       }
       bool z = false;
