@@ -661,6 +661,148 @@ __device__ __forceinline__ void rb_dispatch(const Tile &t, const LevelDev &L, in
 }
 
 // ---------------------------------------------------------------------------
+// NS whole sweeps of a mid-size level of one block in one launch.  There a
+// half-sweep is bound by its launch and one round of memory latency, not by
+// its cells: a workgroup takes the 16^3 cells around a tile of (16 - 4 NS)^3
+// into LDS and runs the 2 NS half-sweeps there, each on one layer of cells
+// less, the cells around the tile being computed again by their own tiles.
+// Bound by the latencies inside (a half-sweep, its barrier) and by instruction
+// issue: 16 wavefronts of two entries a thread took 37 us a cycle for one level
+// of 32^3 (FP64, V(2,2)), 8 wavefronts of four 39, half-sweep launches 49.
+//
+// Positions around the tile continue across a periodic face (an even number
+// of cells: the colours continue, too).  A black cell reads across such a
+// face the red value from before the sweep (`old`), as the ghosts hold it;
+// across a wall the product of a zero coefficient and a zero, as the cells
+// beyond are never set.  The result goes to the other buffer, once: the
+// launch is one step of the level's buffers whatever NS.  zero != 0: the
+// level holds zeros.
+constexpr int RBT = 16, RBT_HALF = RBT * RBT * RBT / 2, RBT_THREADS = 1024;
+template <class T, int NS>
+__global__ void __launch_bounds__(RBT_THREADS, sizeof(T) == 4 ? 8 : 4)
+    k_rb_tile(const LevelDev *__restrict__ levs, const int *__restrict__ active, int src, int zero,
+              int one_lev, int one_blk, int tx, int ty, int ntiles) {
+  constexpr int HALO = 2 * NS, TS = RBT - 2 * HALO, U = RBT_HALF / RBT_THREADS;
+  __shared__ T black[RBT_HALF], red[RBT_HALF], old[RBT_HALF];
+  const LevelDev &L = levs[one_lev];
+  const int on = active[one_blk];
+  const int ni = L.ni, nj = L.nj, nk = L.nk, H = L.H;
+  const bool px = L.per & 1, py = L.per & 2, pz = L.per & 4;
+  const int b = xcd_remap((int)blockIdx.x, ntiles);
+  const int bz = b / (tx * ty), by = (b - bz * tx * ty) / tx, bx = b - (bz * ty + by) * tx;
+  const int x0 = bx * TS - HALO, y0 = by * TS - HALO, z0 = bz * TS - HALO;
+  // whether a periodic face cuts the positions
+  const bool cross = (px && (x0 < 0 || x0 + RBT > ni)) || (py && (y0 < 0 || y0 + RBT > nj)) ||
+                     (pz && (z0 < 0 || z0 + RBT > nk));
+  const gmem<T> *P[2] = {(const gmem<T> *)L.phi[src][0], (const gmem<T> *)L.phi[src][1]};
+  const gmem<T> *R[2] = {(const gmem<T> *)L.rhs[0], (const gmem<T> *)L.rhs[1]};
+  gmem<T> *D[2] = {(gmem<T> *)L.phi[1 - src][0], (gmem<T> *)L.phi[1 - src][1]};
+  const int tid = (int)threadIdx.x, m = tid & 7, ry = (tid >> 3) & 15;
+  auto wrap = [](int x, int n, bool per) { return !per ? x : x < 0 ? x + n : x >= n ? x - n : x; };
+  const int y = y0 + ry, yw = wrap(y, nj, py);
+  const bool oky = (unsigned)yw < (unsigned)nj;
+
+  // a thread's entries: plane rz = tid/128 + 4u of both colours; bits 0..5 of
+  // `face`: the cell lies on that face of the block, 6: it exists
+  unsigned face[U][2], ent[U][2];
+  T r[U][2], v1[U], v0[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int rz = (tid >> 7) + RBT_THREADS / 128 * u, z = z0 + rz, zw = wrap(z, nk, pz);
+    const bool okz = (unsigned)zw < (unsigned)nk;
+    const unsigned fyz = (yw == 0 ? 4u : 0u) | (yw == nj - 1 ? 8u : 0u) | (zw == 0 ? 16u : 0u) |
+                         (zw == nk - 1 ? 32u : 0u);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int x = x0 + 2 * m + ((c + y + z) & 1), xw = wrap(x, ni, px);
+      const bool ok = oky && okz && (unsigned)xw < (unsigned)ni;
+      face[u][c] = fyz | (xw == 0 ? 1u : 0u) | (xw == ni - 1 ? 2u : 0u) | (ok ? 64u : 0u);
+      // positions that do not exist read entry 0
+      const unsigned e =
+          ok ? ((unsigned)zw * (unsigned)nj + (unsigned)yw) * (unsigned)H + ((unsigned)xw >> 1)
+             : 0u;
+      ent[u][c] = e;
+      r[u][c] = R[c][e];
+    }
+    v1[u] = zero ? T(0) : P[1][ent[u][1]];
+    v0[u] = zero || !cross ? T(0) : P[0][ent[u][0]];
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int q = tid + u * RBT_THREADS;
+    black[q] = face[u][1] & 64u ? v1[u] : T(0);
+    red[q] = face[u][0] & 64u ? v0[u] : T(0);
+    if (cross) old[q] = T(0);
+  }
+  __syncthreads();
+  const T cx = (T)L.cx, cy = (T)L.cy, cz = (T)L.cz;
+  // the update of entry q of colour c from the six values
+  auto update = [&](unsigned f, T rhs, const T(&v)[6]) -> T {
+    // FP32: the coefficients are formed each time, kept over the sweeps they
+    // take the registers of a second workgroup on the CU (64^3: 107 | 102 us a
+    // cycle); FP64 is bound by its arithmetic and keeps them (32^3: 79 | 81)
+    if (sizeof(T) == 4) asm volatile("" : "+v"(f));
+    const T aw = (!px && (f & 1u)) ? T(0) : cx, ae = (!px && (f & 2u)) ? T(0) : cx;
+    const T as = (!py && (f & 4u)) ? T(0) : cy, an = (!py && (f & 8u)) ? T(0) : cy;
+    const T ab = (!pz && (f & 16u)) ? T(0) : cz, at = (!pz && (f & 32u)) ? T(0) : cz;
+    const T ap = T(-1) * (aw + ae + as + an + ab + at);
+    const T sum = aw * v[0] + ae * v[1] + as * v[2] + an * v[3] + ab * v[4] + at * v[5];
+    return div_ap(rhs - sum, ap, T(1) / ap);
+  };
+  // whether half-sweep h computes the entry: one layer less each
+  auto in = [&](int c, int rz, int h) {
+    const int rx = 2 * m + ((c + y0 + ry + z0 + rz) & 1), lo = h + 1, hi = RBT - 2 - h;
+    return rx >= lo && rx <= hi && ry >= lo && ry <= hi && rz >= lo && rz <= hi;
+  };
+#pragma unroll 1
+  for (int h = 0; h < 2 * NS; h += 2) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = tid + u * RBT_THREADS, rz = (tid >> 7) + RBT_THREADS / 128 * u;
+      if (!in(0, rz, h) || !(face[u][0] & 64u)) continue;
+      const int s = (y0 + ry + z0 + rz) & 1;
+      const T v[6] = {black[q - 1 + s],       black[q + s],
+                      black[q - RBT / 2],     black[q + RBT / 2],
+                      black[q - RBT * RBT / 2], black[q + RBT * RBT / 2]};
+      const T x = update(face[u][0], r[u][0], v);
+      if (cross) old[q] = red[q];
+      red[q] = x;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = tid + u * RBT_THREADS, rz = (tid >> 7) + RBT_THREADS / 128 * u;
+      if (!in(1, rz, h + 1) || !(face[u][1] & 64u)) continue;
+      const int s = (1 + y0 + ry + z0 + rz) & 1;
+      const int at[6] = {q - 1 + s,   q + s, q - RBT / 2, q + RBT / 2, q - RBT * RBT / 2,
+                         q + RBT * RBT / 2};
+      T v[6];
+#pragma unroll
+      for (int f = 0; f < 6; ++f) v[f] = red[at[f]];
+      if (cross) {
+#pragma unroll
+        for (int f = 0; f < 6; ++f) {
+          const T w = old[at[f]];
+          if ((face[u][1] >> f) & 1u) v[f] = w;  // (a wall's coefficient is 0)
+        }
+      }
+      black[q] = update(face[u][1], r[u][1], v);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int q = tid + u * RBT_THREADS, rz = (tid >> 7) + RBT_THREADS / 128 * u;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int x = x0 + 2 * m + ((c + y + z0 + rz) & 1);
+      if (in(c, rz, HALO - 1) && x < ni && y < nj && z0 + rz < nk && on)
+        D[c][ent[u][c]] = c ? black[q] : red[q];
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Fused red-black sweep for small levels: both colour halves of one sweep
 // in one launch (the split sweep costs two launches, and small levels are
 // bound by launch and memory latency, not by bandwidth).  A tile is FX x FY
@@ -4891,6 +5033,17 @@ void launch_lsm_restrict(hipStream_t s, const Tile *tiles, int ntiles, const Lev
 }
 
 template <class T>
+void launch_rb_tile(hipStream_t s, const LevelDev *levs, const int *active, int src, int zero,
+                    OneDesc one, int nsweep, int ni, int nj, int nk) {
+  const int ts = RBT - 4 * nsweep;
+  auto n = [ts](int c) { return (c + ts - 1) / ts; };
+  const int ntiles = n(ni) * n(nj) * n(nk);
+  auto k = nsweep == 2 ? k_rb_tile<T, 2> : k_rb_tile<T, 1>;
+  hipLaunchKernelGGL(k, dim3(ntiles), dim3(RBT_THREADS), 0, s, levs, active, src, zero, one.lev,
+                     one.blk, n(ni), n(nj), ntiles);
+}
+
+template <class T>
 void launch_rb_fused(hipStream_t s, const Tile *tiles, int ntiles, const LevelDev *levs,
                      const int *active, int src, int zero) {
   if (ntiles <= 0) return;
@@ -5211,6 +5364,10 @@ template void launch_residual<double>(hipStream_t, const Tile *, int, int, const
                                       const LevelDev *, const int *, RedPartial *, int, int);
 template void launch_residual<float>(hipStream_t, const Tile *, int, int, const FineDev *,
                                      const LevelDev *, const int *, RedPartial *, int, int);
+template void launch_rb_tile<double>(hipStream_t, const LevelDev *, const int *, int, int, OneDesc,
+                                     int, int, int, int);
+template void launch_rb_tile<float>(hipStream_t, const LevelDev *, const int *, int, int, OneDesc,
+                                    int, int, int, int);
 template void launch_set_rhs<double>(hipStream_t, const Tile *, int, int, const FineDev *,
                                      const LevelDev *, const double *, RedPartial *);
 template void launch_set_rhs<float>(hipStream_t, const Tile *, int, int, const FineDev *,

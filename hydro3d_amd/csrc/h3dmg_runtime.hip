@@ -105,6 +105,7 @@ struct TileSet {
   bool tdma_lines = false;  // TDMA passes in two launches (tiles: one per block)
   int tdma_len[3] = {0, 0, 0};       // their longest line per pass
   OneDesc one;             // every tile on one descriptor: passed to the kernels
+  bool multi = false;      // smoother sets: whole sweeps of one mid-size level per launch
   int n() const { return (int)h.size(); }
 };
 
@@ -493,6 +494,18 @@ void dev_free(h3dmg_handle *h, void *p) {
 template <class T>
 void relax_group(h3dmg_handle *h, const TileSet &ts, int nsweep, int &buf, bool &zero,
                  bool red_done = false) {
+  if (ts.multi && !h->lsm) {  // up to two sweeps a launch, one buffer step each
+    const LevelDev &L = h->levs[ts.one.lev];
+    for (int left = nsweep; left > 0;) {
+      const int n = std::min(left, 2);
+      launch_rb_tile<T>(h->stream, h->d_levs, h->d_active, buf, zero ? 1 : 0, ts.one, n, L.ni, L.nj,
+                        L.nk);
+      left -= n;
+      buf ^= 1;
+      zero = false;
+    }
+    return;
+  }
   for (int s = 0; s < nsweep; ++s) {
     if (h->prm.smoother == H3DMG_SMOOTH_GS)  // tile wavefront (every level FP64)
       for (int d = 0; d + 1 < (int)ts.diag_begin.size(); ++d)
@@ -566,7 +579,8 @@ void fill_any(h3dmg_handle *h, bool is64, const TileSet &ts, int buf) {
 bool red1_write(const h3dmg_handle *h) {
   const h3dmg_params &P = h->prm;
   return !is_mixed(h) && P.smoother == H3DMG_SMOOTH_RBGS && !h->lsm && !h->connected &&
-         P.nu1 > 0 && ((P.nu1 + P.nu2) & 1) == 0 && h->fine_tiles.depth > 0;
+         P.nu1 > 0 && ((P.nu1 + P.nu2) & 1) == 0 && h->fine_tiles.depth > 0 &&
+         !h->relax_nc[1].multi && !h->relax_c[1].multi;
 }
 
 // Enqueue one V-cycle (mgkcyc, mgsolver.for:272-352) on the level-1 rhs that
@@ -597,13 +611,13 @@ void enqueue_vcycle(h3dmg_handle *h, bool red1 = false) {
                       h->restr_nc[g].n() && h->restr_nc[g].depth > 0
                 : red1 && red1_write(h)) &&
         g < Lt && g < Lm && h->prm.nu1 > 0 && h->relax_nc[g].n() && !h->relax_nc[g].fused &&
-        z_nc[g];
+        !h->relax_nc[g].multi && z_nc[g];
     // likewise for the blocks whose coarsest level g is smoothed (not solved)
     const bool red_c_by_restr = g >= 2 && g < Lt && !(exact && g > 1) && h->prm.nu1 > 0 &&
                                 h->prm.smoother == H3DMG_SMOOTH_RBGS && !h->lsm &&
                                 !h->connected && h->restr_c[g].n() &&
                                 h->restr_c[g].depth > 0 && h->relax_c[g].n() &&
-                                !h->relax_c[g].fused;
+                                !h->relax_c[g].fused && !h->relax_c[g].multi;
     if (g >= 2) {
       // mgrestr(g): residual of level g-1 (non-coarsest there) into rhs_g
       const bool f64 = nc_is64(g - 1);
@@ -1513,6 +1527,8 @@ bool gs_big_ok() {
   return ok;
 }
 
+constexpr long RB_TILE_CUS = 256;
+
 // (Re)build the smoother tiles of level g on the host (both block groups)
 h3dmg_status gen_relax(h3dmg_handle *h, int g) {
   for (int grp = 0; grp < 2; ++grp) {
@@ -1662,6 +1678,26 @@ h3dmg_status gen_relax(h3dmg_handle *h, int g) {
       if (ts.depth && t.kind != 4 && t.z1 - t.z0 != ts.depth)
         return fail(H3DMG_ERR_ARG, "internal: tile depth");
     set_one(ts, h->levs, 0);
+    // one block's level of as many tiles of 8^3 as the CUs hold at once (of
+    // 1024 threads: one FP64, two FP32): about 48^3 and 64^3.  Measured, us per
+    // V(2,2) cycle, whole sweeps wherever they fit | half-sweeps on every
+    // level: FP64 32^3 79 | 88, 48^3 92 | 107, 64x64x96 97 | 110 (110 with whole
+    // sweeps on its first level, 768 tiles, too); FP32 48^3 76 | 95, 64^3
+    // 103 | 117, 104x56x40 86 | 103.  A depth asked for by h3dmg_set_march
+    // keeps the half-sweeps.
+    ts.multi = h->prm.smoother == H3DMG_SMOOTH_RBGS && !general && !ts.fused && ts.one.lev >= 0 &&
+               h->march_kb[g] == 0;
+    if (ts.multi) {
+      const LevelDev &L = h->levs[ts.one.lev];
+      const int n[3] = {L.ni, L.nj, L.nk};
+      long tiles = 1;
+      for (int a = 0; a < 3; ++a) {
+        tiles *= (n[a] + 7) / 8;
+        if ((L.per >> a) & 1) ts.multi = ts.multi && n[a] % 2 == 0 && n[a] >= RB_TILE_PER;
+      }
+      const bool is64 = !is_mixed(h) || grp == 1;
+      ts.multi = ts.multi && tiles <= (is64 ? 1 : 2) * RB_TILE_CUS;
+    }
   }
   return H3DMG_OK;
 }
