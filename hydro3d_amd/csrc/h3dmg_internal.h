@@ -133,6 +133,8 @@ void launch_rb_fused(hipStream_t s, const Tile *tiles, int ntiles, const LevelDe
 template <class Tf, class Tc>
 void launch_restrict(hipStream_t s, const Tile *tiles, int ntiles, int depth, const LevelDev *levs,
                      const int *active, int src_f, OneDesc one = OneDesc{}, int zbuf = -1);
+// row pairs of a tile of the kernel for blocks with neighbours, at most
+constexpr int PROL_GEN_ROWS = 32;
 // gen != 0: coarse ghosts read through the neighbour table (blocks with
 // neighbours); skip_red: a red half-sweep follows, red cells off the open
 // faces are left alone

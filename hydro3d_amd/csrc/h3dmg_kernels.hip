@@ -529,7 +529,7 @@ __device__ __forceinline__ void cell_coefs(const LevelDev &L, int c, int i, int 
 // threads, one per cell of the colour.  The buffer rules are k_rb_sweep's.
 // Bound by the launch and one round of loads.  Averages over four levels, us,
 // with a branch per ghost | now: 64 joined blocks of 64x8x64, 18.3 | 5.9
-// (restriction 74 | 11, prolongation 33 | 15); 96x64x80 with variable density
+// (restriction 74 | 11, prolongation 33 | 12); 96x64x80 with variable density
 // 6.1 | 3.9 (restriction 70 | 6.3).
 template <class T, bool LSM>
 __global__ void __launch_bounds__(128)
@@ -1419,14 +1419,16 @@ __global__ void __launch_bounds__(NTHREADS)
 // 2m-1, 2m and planes 2n-1, 2n (coarse row m and plane n in padded numbering):
 // those eight fine cells share the twelve coarse corners x in {l-1, l, l+1},
 // y in {m-1, m}, z in {n-1, n} (interior numbering), which are loaded once.
-// Tile::x0 = first l, y0 = first m (TILE_Y per tile), z0 = n.  The fine
+// Tile::x0 = first l, y0 = first m, z0 = n, kind = lanes per row: short rows
+// share a wavefront (48 blocks of 32 to 128 cells per axis, a row a wavefront:
+// 48 us on level 1, now 27).  The fine
 // level is updated in place (each fine cell by exactly one thread).
 // GEN: blocks with neighbours -- the coarse ghost corners (edges and corners
-// included) may lie in another block.  A wavefront's corner rows and planes
-// are the same for all its lanes, and in x a corner is inside the row or
-// across one of its two ends: twelve lanes resolve the rows and their ends
-// (resolve_cell) into LDS and every lane picks, instead of following the
-// neighbour table for sixteen corners, one after the other.
+// included) may lie in another block.  All lanes of a row pair share its
+// corner rows, and in x a corner is inside the row or across one of its two
+// ends: the rows and their ends are resolved (resolve_cell) into LDS and every
+// lane picks, instead of following the neighbour table for sixteen corners,
+// one after the other.
 // skip_red: a red half-sweep follows.  It replaces every red cell from black
 // neighbours, and of the red values before it only those on open (periodic or
 // shared) faces are read again, as ghosts of the black half-sweep: the other
@@ -1446,32 +1448,35 @@ __global__ void __launch_bounds__(NTHREADS)
   if (!ONE && !active[F.blk]) return;
   const LevelDev &C = levs[ONE ? one_lev2 : F.coarser];
   if (ONE)
-    asm volatile("" ::"s"(t.x0), "s"(t.y0), "s"(t.z0), "s"(on), "s"(F.ni), "s"(F.nj), "s"(F.nk),
-                 "s"(F.H), "s"(F.phi[0][0]), "s"(F.phi[0][1]), "s"(F.phi[1][0]), "s"(F.phi[1][1]),
+    asm volatile("" ::"s"(t.x0), "s"(t.y0), "s"(t.z0), "s"(t.kind), "s"(on), "s"(F.ni), "s"(F.nj),
+                 "s"(F.nk), "s"(F.H), "s"(F.phi[0][0]), "s"(F.phi[0][1]), "s"(F.phi[1][0]), "s"(F.phi[1][1]),
                  "s"(C.ni), "s"(C.nj), "s"(C.nk), "s"(C.H), "s"(C.per), "s"(C.phi[0][0]),
                  "s"(C.phi[0][1]), "s"(C.phi[1][0]), "s"(C.phi[1][1]));
   // a thread holds fine entries l, l+1 (l even): cells 2l .. 2l+3 of the
   // 2x2 rows and planes around coarse row pair m, plane pair n
   typedef typename Vec2<Tf>::type v2;
-  const int l = t.x0 + 2 * (int)threadIdx.x;
-  const int m = t.y0 + (int)threadIdx.y;
+  const int lpr = t.kind;  // lanes per row, a power of two
+  const int l = t.x0 + 2 * ((int)threadIdx.x & (lpr - 1));
+  const int rw = ((int)threadIdx.y * 64 + (int)threadIdx.x) / lpr;  // row pair of the tile
+  const int m = t.y0 + rw;
   const int n = t.z0;
-  // GEN: the wavefront's corner rows (y, z), inside the block's x range,
-  // before it and after it: the row's arrays by the parity of x, and the x of
-  // the end cell
+  // GEN: the corner rows (y, z) of every row pair of the tile, inside the
+  // block's x range, before it and after it: the row's arrays by the parity of
+  // x, and the x of the end cell
   struct RowSrc {
     const gmem<Tc> *p[2];
     int x;
   };
-  __shared__ RowSrc rows[GEN ? TILE_Y : 1][12];
+  __shared__ RowSrc rows[GEN ? PROL_GEN_ROWS : 1][12];
   if (GEN) {
-    const int q = (int)threadIdx.x;
-    if (q < 12) {
-      int x = q % 3 == 0 ? 0 : q % 3 == 1 ? -1 : C.ni;
-      int y = min(m, C.nj) - 1 + (q / 3) % 2, z = min(n, C.nk) - 1 + q / 6;
+    const int nq = 12 * (NTHREADS / lpr);
+    for (int q = (int)threadIdx.y * 64 + (int)threadIdx.x; q < nq; q += NTHREADS) {
+      const int w = q / 12, e = q - 12 * w;
+      int x = e % 3 == 0 ? 0 : e % 3 == 1 ? -1 : C.ni;
+      int y = min(t.y0 + w, C.nj) - 1 + (e / 3) % 2, z = min(n, C.nk) - 1 + e / 6;
       const LevelDev &P = levs[resolve_cell(levs, F.coarser, x, y, z)];
       const size_t row = ((size_t)z * P.nj + y) * P.H;
-      RowSrc &r = rows[threadIdx.y][q];
+      RowSrc &r = rows[w][e];
       r.p[0] = (const gmem<Tc> *)P.phi[src_c][(y + z) & 1] + row;
       r.p[1] = (const gmem<Tc> *)P.phi[src_c][(y + z + 1) & 1] + row;
       r.x = x;
@@ -1501,7 +1506,7 @@ __global__ void __launch_bounds__(NTHREADS)
         if (GEN) {
           const int x = min(l - 1 + a, two ? l + 2 : l + 1);
           const int at = x < 0 ? 1 : x >= C.ni ? 2 : 0;
-          const RowSrc r = rows[threadIdx.y][at + 3 * (b + 2 * c)];
+          const RowSrc r = rows[rw][at + 3 * (b + 2 * c)];
           const int xx = at == 0 ? x : r.x;
           cv[a][b][c] = ((xx & 1) ? r.p[1] : r.p[0])[xx >> 1];
         } else {

@@ -215,14 +215,16 @@ int restrict_depth(const std::vector<LevelDev> &levs, const std::vector<int> &le
 }
 
 // Prolongation tiles of fine level descriptor `lev` (k_prolong): fine entries
-// x0.. (two per thread, 2*TILE_X per tile) x coarse row pairs m = y0..
-// (TILE_Y per tile) x one coarse plane pair n = z0, with m in [0, nj/2] and n
-// in [0, nk/2].
-void add_tiles_prolong(TileSet &ts, int lev, const LevelDev &F) {
+// x0.. (two per thread, kind = lanes per row: 2*kind per tile) x coarse row
+// pairs m = y0.. (NTHREADS/kind per tile) x one coarse plane pair n = z0, with
+// m in [0, nj/2] and n in [0, nk/2].
+void add_tiles_prolong(TileSet &ts, int lev, const LevelDev &F, bool gen) {
   const int ncj = F.nj / 2, nck = F.nk / 2, nfx = F.ni / 2;
+  int lp = gen ? NTHREADS / PROL_GEN_ROWS : 1;
+  while (lp < 64 && 2 * lp < nfx) lp *= 2;
   for (int n = 0; n <= nck; ++n)
-    for (int m = 0; m <= ncj; m += TILE_Y)
-      for (int x = 0; x < nfx; x += 2 * TILE_X) ts.h.push_back(Tile{lev, x, m, n, n + 1, 0});
+    for (int m = 0; m <= ncj; m += NTHREADS / lp)
+      for (int x = 0; x < nfx; x += 2 * lp) ts.h.push_back(Tile{lev, x, m, n, n + 1, lp});
 }
 
 struct BlockInfo {
@@ -1160,7 +1162,8 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
       const LevelDev &L = h->levs[d];
       if (g < B.L) {
         add_tiles(h->nat_nc[g], d, L.ni, L.nj, L.nk);
-        add_tiles_prolong(g + 1 < B.L ? h->prol_nc[g] : h->prol_c[g], d, L);
+        add_tiles_prolong(g + 1 < B.L ? h->prol_nc[g] : h->prol_c[g], d, L,
+                          h->connected);
       } else {
         add_tiles(h->nat_c[g], d, L.ni, L.nj, L.nk);
       }
