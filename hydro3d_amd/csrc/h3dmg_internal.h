@@ -98,7 +98,8 @@ struct RedPartial {
 // one colour half-sweep of the red-black smoother over a tile list whose
 // tiles are all `depth` (1, 2 or 4) planes deep: kinds 0 (march tile, y/z
 // interior), 3 (march tile touching a y/z face); depth 0: natural tiles, cell
-// by cell (blocks with neighbours, levels one cell wide in x)
+// by cell (blocks with neighbours, levels one cell wide in x).  upd (level 1's
+// last black half-sweep, depth > 0): also p += pp
 // A launch whose tiles all belong to one descriptor (lev; lev2: its finer
 // level for a restriction, its coarser for a prolongation; blk its block):
 // the kernel then reads the tile, the descriptors and the block's flag at
@@ -108,14 +109,16 @@ struct OneDesc {
 };
 template <class T>
 void launch_rb_sweep(hipStream_t s, const Tile *tiles, int ntiles, int depth, const LevelDev *levs,
-                     const int *active, int colour, int src, int zero, OneDesc one = OneDesc{});
+                     const int *active, int colour, int src, int zero, OneDesc one = OneDesc{},
+                     const FineDev *upd = nullptr);
 // nsweep (1 or 2) sweeps of a level of ni x nj x nk cells, descriptor one.lev
 // of block one.blk, in one launch, from buffer src to the other: periodic
-// axes of an even number of cells, RB_TILE_PER at least
+// axes of an even number of cells, RB_TILE_PER at least; upd: level 1's last
+// sweeps, also p += pp
 constexpr int RB_TILE_PER = 16;
 template <class T>
 void launch_rb_tile(hipStream_t s, const LevelDev *levs, const int *active, int src, int zero,
-                    OneDesc one, int nsweep, int ni, int nj, int nk);
+                    OneDesc one, int nsweep, int ni, int nj, int nk, const FineDev *upd);
 // one full red-black sweep (both colour halves) of small levels in one
 // launch: tiles of FUSED_X x FUSED_Y x FUSED_Z cells (Tile::x0, y0, z0 in
 // cells), kind 4

@@ -262,10 +262,15 @@ using gmem = __attribute__((address_space(1))) T;
 //   y/z faces (BND tiles only): rows 0 and nj-1 read their image rows;
 //     chunks at plane 0 or nk-1 read the image plane into the window.
 // The arithmetic of every cell is cell_coef's and the sum of mgsolver.for's
-// relaxation, as in march_tile.
-template <class T, int KB, bool ZERO_INT, bool BND>
+// relaxation.
+//
+// UPD (level 1's last black half-sweep): also p = p + (pp - 0) (k_update) of
+// the lane's entries of both colours.  The new black values and, in the
+// window, the red ones are at hand: k_update would read both again (256^3,
+// half-sweep and k_update: FP64 41 + 59 us, now 81; float 19 + 50, now 60).
+template <class T, int KB, bool ZERO_INT, bool BND, bool UPD>
 __device__ __forceinline__ void march_tile_fast(const Tile &t, const LevelDev &L, int colour,
-                                                int src, int zero, bool on) {
+                                                int src, int zero, bool on, const FineDev *F) {
   typedef typename Vec2<T>::type v2;
   constexpr unsigned SZ = sizeof(T);
   const int lpr = L.lpr;
@@ -385,6 +390,19 @@ __device__ __forceinline__ void march_tile_fast(const Tile &t, const LevelDev &L
     }
 #pragma unroll
     for (int p = 0; p < KB; ++p) R2[p] = ld2(aR + cell + p0 + (unsigned)p * plane);
+    typedef typename Vec2<double>::type d2;
+    d2 pr[UPD ? KB : 1], pb[UPD ? KB : 1];
+    auto p_at = [&](int c, int p) {
+      return (gmem<d2> *)((gmem<char> *)F->p[c] +
+                          (cell + p0 + (unsigned)p * plane) * (unsigned)(sizeof(double) / SZ));
+    };
+    if constexpr (UPD) {
+#pragma unroll
+      for (int p = 0; p < KB; ++p) {
+        pr[p] = *p_at(0, p);
+        pb[p] = *p_at(1, p);
+      }
+    }
 #pragma unroll
     for (int p = 0; p < KB; ++p) {
       const int k = k0 + p;
@@ -434,6 +452,16 @@ __device__ __forceinline__ void march_tile_fast(const Tile &t, const LevelDev &L
       } else {
         if (w0) *(gmem<T> *)dq = R2[p].x;
         if (w1) *(gmem<T> *)(dq + SZ) = R2[p].y;
+      }
+      if constexpr (UPD) {  // (pad entries included: they are never read as cells)
+        if (col_ok) {
+          pr[p].x = pr[p].x + ((double)own[p + 1].x - 0.0);
+          pr[p].y = pr[p].y + ((double)own[p + 1].y - 0.0);
+          pb[p].x = pb[p].x + ((double)R2[p].x - 0.0);
+          pb[p].y = pb[p].y + ((double)R2[p].y - 0.0);
+          *p_at(0, p) = pr[p];
+          *p_at(1, p) = pb[p];
+        }
       }
     }
   }
@@ -608,9 +636,9 @@ __global__ void __launch_bounds__(NTHREADS)
 // KB planes deep: kind 0 has every y/z neighbour inside the block, kind 3
 // touches a y/z face; the tiles write disjoint cells.  One instantiation per depth keeps each one's register
 // count to what its own tiles need.
-template <class T, int KB>
+template <class T, int KB, bool UPD>
 __device__ __forceinline__ void rb_dispatch(const Tile &t, const LevelDev &L, int colour, int src,
-                                            int zero, bool on);
+                                            int zero, bool on, const FineDev *F);
 
 // In the one-descriptor kernels, one empty asm statement takes the tile,
 // the block's flag and every descriptor field the kernel reads: all of them
@@ -625,11 +653,11 @@ __device__ __forceinline__ void rb_dispatch(const Tile &t, const LevelDev &L, in
 // flag masks the stores instead of ending inactive workgroups early, so that
 // the data loads wait for none of them but the tile and the descriptor
 // (small levels are bound by this chain of latencies).
-template <class T, int KB, bool ONE>
+template <class T, int KB, bool ONE, bool UPD>
 __global__ void __launch_bounds__(NTHREADS)
     k_rb_sweep(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
                const int *__restrict__ active, int colour, int src, int zero, int one_lev,
-               int one_blk, int ntiles) {
+               int one_blk, int ntiles, const FineDev *__restrict__ fine) {
   const Tile t = tiles[xcd_remap((int)blockIdx.x, ntiles)];
   if (ONE) {
     const LevelDev &L = levs[one_lev];
@@ -638,25 +666,32 @@ __global__ void __launch_bounds__(NTHREADS)
                  "s"(L.nk), "s"(L.H), "s"(L.per), "s"(L.lpr), "s"(L.cx), "s"(L.cy), "s"(L.cz),
                  "s"(L.phi[0][0]), "s"(L.phi[0][1]), "s"(L.phi[1][0]), "s"(L.phi[1][1]),
                  "s"(L.rhs[0]), "s"(L.rhs[1]));
-    rb_dispatch<T, KB>(t, L, colour, src, zero, on != 0);
+    rb_dispatch<T, KB, UPD>(t, L, colour, src, zero, on != 0, UPD ? fine + one_blk : nullptr);
   } else {
     const LevelDev &L = levs[t.lev];
     if (!active[L.blk]) return;
-    rb_dispatch<T, KB>(t, L, colour, src, zero, true);
+    rb_dispatch<T, KB, UPD>(t, L, colour, src, zero, true, UPD ? fine + L.blk : nullptr);
   }
 }
 
-template <class T, int KB>
+template <class T, int KB, bool UPD>
 __device__ __forceinline__ void rb_dispatch(const Tile &t, const LevelDev &L, int colour, int src,
-                                            int zero, bool on) {
+                                            int zero, bool on, const FineDev *F) {
+  if constexpr (UPD) {
+    if (t.kind == 0)
+      march_tile_fast<T, KB, false, false, true>(t, L, 1, src, zero, on, F);
+    else
+      march_tile_fast<T, KB, false, true, true>(t, L, 1, src, zero, on, F);
+    return;
+  }
   // the interior neighbours are zeros in the red half of a zero-state sweep
   const bool zint = zero && colour == 0;
   if (t.kind == 0) {
-    zint ? march_tile_fast<T, KB, true, false>(t, L, colour, src, zero, on)
-         : march_tile_fast<T, KB, false, false>(t, L, colour, src, zero, on);
+    zint ? march_tile_fast<T, KB, true, false, false>(t, L, colour, src, zero, on, F)
+         : march_tile_fast<T, KB, false, false, false>(t, L, colour, src, zero, on, F);
   } else {
-    zint ? march_tile_fast<T, KB, true, true>(t, L, colour, src, zero, on)
-         : march_tile_fast<T, KB, false, true>(t, L, colour, src, zero, on);
+    zint ? march_tile_fast<T, KB, true, true, false>(t, L, colour, src, zero, on, F)
+         : march_tile_fast<T, KB, false, true, false>(t, L, colour, src, zero, on, F);
   }
 }
 
@@ -681,7 +716,8 @@ constexpr int RBT = 16, RBT_HALF = RBT * RBT * RBT / 2, RBT_THREADS = 1024;
 template <class T, int NS>
 __global__ void __launch_bounds__(RBT_THREADS, sizeof(T) == 4 ? 8 : 4)
     k_rb_tile(const LevelDev *__restrict__ levs, const int *__restrict__ active, int src, int zero,
-              int one_lev, int one_blk, int tx, int ty, int ntiles) {
+              int one_lev, int one_blk, int tx, int ty, int ntiles,
+              const FineDev *__restrict__ fine) {
   constexpr int HALO = 2 * NS, TS = RBT - 2 * HALO, U = RBT_HALF / RBT_THREADS;
   __shared__ T black[RBT_HALF], red[RBT_HALF], old[RBT_HALF];
   const LevelDev &L = levs[one_lev];
@@ -796,8 +832,14 @@ __global__ void __launch_bounds__(RBT_THREADS, sizeof(T) == 4 ? 8 : 4)
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int x = x0 + 2 * m + ((c + y + z0 + rz) & 1);
-      if (in(c, rz, HALO - 1) && x < ni && y < nj && z0 + rz < nk && on)
-        D[c][ent[u][c]] = c ? black[q] : red[q];
+      if (in(c, rz, HALO - 1) && x < ni && y < nj && z0 + rz < nk && on) {
+        const T pp = c ? black[q] : red[q];
+        D[c][ent[u][c]] = pp;
+        if (fine) {  // level 1's last sweeps: also p = p + (pp - 0), as k_update
+          gmem<double> *const p = (gmem<double> *)fine[one_blk].p[c] + ent[u][c];
+          *p = *p + ((double)pp - 0.0);
+        }
+      }
     }
   }
 }
@@ -4877,21 +4919,26 @@ __global__ void __launch_bounds__(TDMA_SWEEP_THREADS)
 // ---- launchers -----------------------------------------------------------
 template <class T>
 void launch_rb_sweep(hipStream_t s, const Tile *tiles, int ntiles, int depth, const LevelDev *levs,
-                     const int *active, int colour, int src, int zero, OneDesc one) {
+                     const int *active, int colour, int src, int zero, OneDesc one,
+                     const FineDev *upd) {
   if (ntiles <= 0) return;
   if (depth == 0) {  // natural tiles, cell by cell
     hipLaunchKernelGGL((k_cell_sweep<T, false>), dim3(ntiles), dim3(TILE_X, TILE_Y / 2), 0, s, tiles,
                        levs, active, colour, src, zero, ntiles);
     return;
   }
-  auto k = one.lev >= 0 ? (depth == 4   ? k_rb_sweep<T, 4, true>
-                           : depth == 2 ? k_rb_sweep<T, 2, true>
-                                        : k_rb_sweep<T, 1, true>)
-                        : (depth == 4   ? k_rb_sweep<T, 4, false>
-                           : depth == 2 ? k_rb_sweep<T, 2, false>
-                                        : k_rb_sweep<T, 1, false>);
+  auto pick = [&](auto u) {
+    constexpr bool UPD = decltype(u)::value;
+    return one.lev >= 0 ? (depth == 4   ? k_rb_sweep<T, 4, true, UPD>
+                           : depth == 2 ? k_rb_sweep<T, 2, true, UPD>
+                                        : k_rb_sweep<T, 1, true, UPD>)
+                        : (depth == 4   ? k_rb_sweep<T, 4, false, UPD>
+                           : depth == 2 ? k_rb_sweep<T, 2, false, UPD>
+                                        : k_rb_sweep<T, 1, false, UPD>);
+  };
+  auto k = upd ? pick(std::true_type()) : pick(std::false_type());
   hipLaunchKernelGGL(k, dim3(ntiles), tile_block(), 0, s, tiles, levs, active, colour, src, zero,
-                     one.lev, one.blk, ntiles);
+                     one.lev, one.blk, ntiles, upd);
 }
 
 void launch_lsm_dens_restrict(hipStream_t s, const double *fine, int fni, int fnj, int fnk,
@@ -5039,13 +5086,13 @@ void launch_lsm_restrict(hipStream_t s, const Tile *tiles, int ntiles, const Lev
 
 template <class T>
 void launch_rb_tile(hipStream_t s, const LevelDev *levs, const int *active, int src, int zero,
-                    OneDesc one, int nsweep, int ni, int nj, int nk) {
+                    OneDesc one, int nsweep, int ni, int nj, int nk, const FineDev *upd) {
   const int ts = RBT - 4 * nsweep;
   auto n = [ts](int c) { return (c + ts - 1) / ts; };
   const int ntiles = n(ni) * n(nj) * n(nk);
   auto k = nsweep == 2 ? k_rb_tile<T, 2> : k_rb_tile<T, 1>;
   hipLaunchKernelGGL(k, dim3(ntiles), dim3(RBT_THREADS), 0, s, levs, active, src, zero, one.lev,
-                     one.blk, n(ni), n(nj), ntiles);
+                     one.blk, n(ni), n(nj), ntiles, upd);
 }
 
 template <class T>
@@ -5346,9 +5393,11 @@ template void launch_rb_fused<double>(hipStream_t, const Tile *, int, const Leve
 template void launch_rb_fused<float>(hipStream_t, const Tile *, int, const LevelDev *, const int *,
                                      int, int);
 template void launch_rb_sweep<double>(hipStream_t, const Tile *, int, int, const LevelDev *,
-                                      const int *, int, int, int, OneDesc);
+                                      const int *, int, int, int, OneDesc,
+                                      const FineDev *);
 template void launch_rb_sweep<float>(hipStream_t, const Tile *, int, int, const LevelDev *,
-                                     const int *, int, int, int, OneDesc);
+                                     const int *, int, int, int, OneDesc,
+                                      const FineDev *);
 template void launch_restrict<double, double>(hipStream_t, const Tile *, int, int, const LevelDev *,
                                               const int *, int, OneDesc, int);
 template void launch_restrict<float, float>(hipStream_t, const Tile *, int, int, const LevelDev *,
@@ -5370,9 +5419,9 @@ template void launch_residual<double>(hipStream_t, const Tile *, int, int, const
 template void launch_residual<float>(hipStream_t, const Tile *, int, int, const FineDev *,
                                      const LevelDev *, const int *, RedPartial *, int, int);
 template void launch_rb_tile<double>(hipStream_t, const LevelDev *, const int *, int, int, OneDesc,
-                                     int, int, int, int);
+                                     int, int, int, int, const FineDev *);
 template void launch_rb_tile<float>(hipStream_t, const LevelDev *, const int *, int, int, OneDesc,
-                                    int, int, int, int);
+                                    int, int, int, int, const FineDev *);
 template void launch_set_rhs<double>(hipStream_t, const Tile *, int, int, const FineDev *,
                                      const LevelDev *, const double *, RedPartial *);
 template void launch_set_rhs<float>(hipStream_t, const Tile *, int, int, const FineDev *,

@@ -492,17 +492,18 @@ void dev_free(h3dmg_handle *h, void *p) {
 }
 
 // red_done: the red half of the first sweep (from zero) was written by the
-// restriction into this level (launch_restrict's zbuf)
+// restriction into this level (launch_restrict's zbuf).  upd: the last sweep
+// also adds the result to p (sweep_updates)
 template <class T>
 void relax_group(h3dmg_handle *h, const TileSet &ts, int nsweep, int &buf, bool &zero,
-                 bool red_done = false) {
+                 bool red_done = false, bool upd = false) {
   if (ts.multi && !h->lsm) {  // up to two sweeps a launch, one buffer step each
     const LevelDev &L = h->levs[ts.one.lev];
     for (int left = nsweep; left > 0;) {
       const int n = std::min(left, 2);
-      launch_rb_tile<T>(h->stream, h->d_levs, h->d_active, buf, zero ? 1 : 0, ts.one, n, L.ni, L.nj,
-                        L.nk);
       left -= n;
+      launch_rb_tile<T>(h->stream, h->d_levs, h->d_active, buf, zero ? 1 : 0, ts.one, n, L.ni, L.nj,
+                        L.nk, upd && left == 0 ? h->d_fine : nullptr);
       buf ^= 1;
       zero = false;
     }
@@ -535,7 +536,8 @@ void relax_group(h3dmg_handle *h, const TileSet &ts, int nsweep, int &buf, bool 
     else
       for (int colour = (s == 0 && red_done) ? 1 : 0; colour < 2; ++colour)
         launch_rb_sweep<T>(h->stream, ts.d, ts.n(), ts.depth, h->d_levs, h->d_active, colour,
-                           buf, zero ? 1 : 0, ts.one);
+                           buf, zero ? 1 : 0, ts.one,
+                           upd && s == nsweep - 1 && colour == 1 ? h->d_fine : nullptr);
     buf ^= 1;
     zero = false;
   }
@@ -549,7 +551,7 @@ h3dmg_status upload_tail(h3dmg_handle *h, bool sync = true);
 h3dmg_status gen_tail(h3dmg_handle *h);
 
 void relax_any(h3dmg_handle *h, bool is64, const TileSet &ts, int nsweep, int &buf, bool &zero,
-               bool red_done = false) {
+               bool red_done = false, bool upd = false) {
   if (ts.n() == 0) {
     // keep the bookkeeping identical for empty groups
     if (nsweep > 0) {
@@ -559,9 +561,9 @@ void relax_any(h3dmg_handle *h, bool is64, const TileSet &ts, int nsweep, int &b
     return;
   }
   if (is64)
-    relax_group<double>(h, ts, nsweep, buf, zero, red_done);
+    relax_group<double>(h, ts, nsweep, buf, zero, red_done, upd);
   else
-    relax_group<float>(h, ts, nsweep, buf, zero, red_done);
+    relax_group<float>(h, ts, nsweep, buf, zero, red_done, upd);
 }
 
 void fill_any(h3dmg_handle *h, bool is64, const TileSet &ts, int buf) {
@@ -571,7 +573,7 @@ void fill_any(h3dmg_handle *h, bool is64, const TileSet &ts, int buf) {
     launch_fill_zero<float>(h->stream, ts.d, ts.n(), h->d_levs, h->d_active, buf);
 }
 
-// The residual's fast path (enqueue_update_residual) also writes the red half
+// The residual's fast path (enqueue_residual) also writes the red half
 // of the level-1 relaxation from zero (each red cell rhs/ap, into buffer 1,
 // where the first half-sweep from buffer 0 puts it): an FP64 level 1 (in
 // mixed precision the FP32 residual slows by more than the half-sweep costs),
@@ -585,6 +587,14 @@ bool red1_write(const h3dmg_handle *h) {
          !h->relax_nc[1].multi && !h->relax_c[1].multi;
 }
 
+// Whether level 1's last post-smoothing sweep can add the correction to p: a
+// red-black sweep with constant coefficients of all blocks.
+bool sweep_updates(const h3dmg_handle *h) {
+  const TileSet &ts = h->relax_nc[1];
+  return h->prm.nu2 > 0 && h->prm.smoother == H3DMG_SMOOTH_RBGS && !h->lsm && ts.n() > 0 &&
+         h->relax_c[1].n() == 0 && (ts.multi || (ts.depth > 0 && !ts.fused));
+}
+
 // Enqueue one V-cycle (mgkcyc, mgsolver.for:272-352) on the level-1 rhs that
 // is already in place.  red1: that rhs came from the residual with the red
 // half of the first level-1 sweep (red1_write), so the sweep starts with its
@@ -593,7 +603,8 @@ bool red1_write(const h3dmg_handle *h) {
 // level relax(L, nu1) + relax(L, nu2) (the reference) or the exact solve.
 // Sweep counts per level are nu1 + nu2 for every block, so the buffer that
 // holds a level at mgcorr time is the same for all blocks.
-void enqueue_vcycle(h3dmg_handle *h, bool red1 = false) {
+// update: p = p + (pp - 0) of the result as well.
+void enqueue_vcycle(h3dmg_handle *h, bool red1, bool update) {
   const int nu1 = h->prm.nu1, nu2 = h->prm.nu2, Lm = h->Lmax;
   const bool mixed = is_mixed(h);
   const bool exact = h->prm.coarse == H3DMG_COARSE_EXACT;
@@ -691,6 +702,7 @@ void enqueue_vcycle(h3dmg_handle *h, bool red1 = false) {
     }
   }
   const int skip_red = nu2 > 0 && h->prm.smoother == H3DMG_SMOOTH_RBGS;
+  const bool upd = update && gdown > 1 && sweep_updates(h);
   for (int g = gdown - 1; g >= 1; --g) {
     // mgcorr(g) for blocks with L_b > g
     if (h->prol_nc[g].n() || h->prol_c[g].n()) {
@@ -724,24 +736,24 @@ void enqueue_vcycle(h3dmg_handle *h, bool red1 = false) {
                                         h->prol_c[g].one);
       }
       bool z = false;
-      relax_any(h, f64, h->relax_nc[g], nu2, buf_nc[g], z);
+      relax_any(h, f64, h->relax_nc[g], nu2, buf_nc[g], z, false, upd && g == 1);
     }
   }
   // the level-1 correction pp: blocks with L_b == 1 hold it in buf_c[1]
   h->pp_buf = (h->relax_c[1].n() && !h->relax_nc[1].n()) ? buf_c[1] : buf_nc[1];
+  if (!update || upd) return;
+  const TileSet &ut = h->update_tiles;
+  if (mixed)
+    launch_update<float>(h->stream, ut.d, ut.n(), h->d_fine, h->d_levs, h->d_active, h->pp_buf);
+  else
+    launch_update<double>(h->stream, ut.d, ut.n(), h->d_fine, h->d_levs, h->d_active, h->pp_buf);
 }
 
-// p += pp, r = f - A p, per-block ||r||, max|r| (one outer iteration tail)
+// r = f - A p, per-block ||r||, max|r|
 // finalize = false: the caller reduces the partials itself
-void enqueue_update_residual(h3dmg_handle *h, bool update, bool finalize = true) {
+void enqueue_residual(h3dmg_handle *h, bool finalize = true) {
   const bool f64 = !is_mixed(h);
-  const TileSet &ft = h->fine_tiles, &ut = h->update_tiles;
-  if (update) {
-    if (f64)
-      launch_update<double>(h->stream, ut.d, ut.n(), h->d_fine, h->d_levs, h->d_active, h->pp_buf);
-    else
-      launch_update<float>(h->stream, ut.d, ut.n(), h->d_fine, h->d_levs, h->d_active, h->pp_buf);
-  }
+  const TileSet &ft = h->fine_tiles;
   if (h->lsm)
     launch_lsm_residual(h->stream, ft.d, ft.n(), h->d_fine, h->d_levs, h->d_active,
                         h->d_partials);
@@ -1976,13 +1988,7 @@ void enqueue_rhs_from_f(h3dmg_handle *h) {
 // One iteration of newsolv_mg's loop (newsolv_mg.for:24-55): mgkcyc from su
 // (in the level-1 rhs already, pp = 0), p = p + (pp - 0), calvel + calmas.
 void enqueue_velocity_step(h3dmg_handle *h) {
-  const bool f64 = !is_mixed(h);
-  const TileSet &ut = h->update_tiles;
-  enqueue_vcycle(h);
-  if (f64)
-    launch_update<double>(h->stream, ut.d, ut.n(), h->d_fine, h->d_levs, h->d_active, h->pp_buf);
-  else
-    launch_update<float>(h->stream, ut.d, ut.n(), h->d_fine, h->d_levs, h->d_active, h->pp_buf);
+  enqueue_vcycle(h, false, true);
   enqueue_project(h);
 }
 
@@ -2040,8 +2046,8 @@ h3dmg_status run_cycle(h3dmg_handle *h) {
     if (!h->gexec) {
       std::lock_guard<std::mutex> lock(g_device_mutex);
       HIP_TRY(hipStreamBeginCapture(h->stream, hipStreamCaptureModeRelaxed));
-      enqueue_vcycle(h);
-      enqueue_update_residual(h, true);
+      enqueue_vcycle(h, false, true);
+      enqueue_residual(h);
       hipGraph_t g = nullptr;
       HIP_TRY(hipStreamEndCapture(h->stream, &g));
       h->graph = g;
@@ -2049,8 +2055,8 @@ h3dmg_status run_cycle(h3dmg_handle *h) {
     }
     HIP_TRY(hipGraphLaunch(h->gexec, h->stream));
   } else {
-    enqueue_vcycle(h);
-    enqueue_update_residual(h, true);
+    enqueue_vcycle(h, false, true);
+    enqueue_residual(h);
   }
   HIP_TRY(hipGetLastError());
   return H3DMG_OK;
@@ -2465,7 +2471,7 @@ h3dmg_status h3dmg_vcycle(h3dmg_handle *h) {
   else
     launch_residual<double>(h->stream, ft.d, ft.n(), ft.depth, h->d_fine, h->d_levs, h->d_active,
                             h->d_partials, 0);
-  enqueue_vcycle(h);
+  enqueue_vcycle(h, false, false);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(h->stream));
   return H3DMG_OK;
@@ -2518,8 +2524,8 @@ h3dmg_status decide_setup(h3dmg_handle *h) {
   if (!h->gexec_dec) {
     HIP_TRY(hipStreamBeginCapture(h->stream, hipStreamCaptureModeRelaxed));
     // every level-1 rhs of h3dmg_solve comes from the residual: red1
-    enqueue_vcycle(h, true);
-    enqueue_update_residual(h, true, false);
+    enqueue_vcycle(h, true, true);
+    enqueue_residual(h, false);
     // the partials' reduction and the stopping rule in one launch; its
     // arrival counter shares the 256-byte slot of DecideCtl, a line apart
     launch_finalize_decide(h->stream, h->d_tile_begin, nb, h->d_partials, h->d_stats,
@@ -2659,7 +2665,7 @@ h3dmg_status h3dmg_solve(h3dmg_handle *h, double *hist, int hist_cap, int *ncycl
     B.rel = 0.0;
   }
   h->rhs_is_f = false;
-  enqueue_update_residual(h, false);
+  enqueue_residual(h);
   HIP_TRY(hipGetLastError());
   st = read_stats(h);
   if (st) return st;
@@ -2847,7 +2853,7 @@ h3dmg_status h3dmg_solve_begin(h3dmg_handle *h, const int *blocks, int n) {
   for (int b = 0; b < h->nb; ++b) h->active[b] = pick[b];
   if ((st = push_active(h))) return st;
   h->rhs_is_f = false;
-  enqueue_update_residual(h, false);
+  enqueue_residual(h);
   HIP_TRY(hipGetLastError());
   if ((st = read_stats(h))) return st;
   for (int b = 0; b < h->nb; ++b) {
