@@ -111,14 +111,14 @@ template <class T>
 void launch_rb_sweep(hipStream_t s, const Tile *tiles, int ntiles, int depth, const LevelDev *levs,
                      const int *active, int colour, int src, int zero, OneDesc one = OneDesc{},
                      const FineDev *upd = nullptr);
-// nsweep (1 or 2) sweeps of a level of ni x nj x nk cells, descriptor one.lev
-// of block one.blk, in one launch, from buffer src to the other: periodic
+// two sweeps of a level of ni x nj x nk cells, descriptor one.lev of block
+// one.blk, in one launch, from buffer src to the other: periodic
 // axes of an even number of cells, RB_TILE_PER at least; upd: level 1's last
 // sweeps, also p += pp
 constexpr int RB_TILE_PER = 16;
 template <class T>
 void launch_rb_tile(hipStream_t s, const LevelDev *levs, const int *active, int src, int zero,
-                    OneDesc one, int nsweep, int ni, int nj, int nk, const FineDev *upd);
+                    OneDesc one, int ni, int nj, int nk, const FineDev *upd);
 // one full red-black sweep (both colour halves) of small levels in one
 // launch: tiles of FUSED_X x FUSED_Y x FUSED_Z cells (Tile::x0, y0, z0 in
 // cells), kind 4

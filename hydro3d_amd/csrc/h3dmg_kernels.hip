@@ -696,10 +696,10 @@ __device__ __forceinline__ void rb_dispatch(const Tile &t, const LevelDev &L, in
 }
 
 // ---------------------------------------------------------------------------
-// NS whole sweeps of a mid-size level of one block in one launch.  There a
+// Two whole sweeps of a mid-size level of one block in one launch.  There a
 // half-sweep is bound by its launch and one round of memory latency, not by
-// its cells: a workgroup takes the 16^3 cells around a tile of (16 - 4 NS)^3
-// into LDS and runs the 2 NS half-sweeps there, each on one layer of cells
+// its cells: a workgroup takes the 16^3 cells around a tile of 8^3
+// into LDS and runs the four half-sweeps there, each on one layer of cells
 // less, the cells around the tile being computed again by their own tiles.
 // Bound by the latencies inside (a half-sweep, its barrier) and by instruction
 // issue: 16 wavefronts of two entries a thread took 37 us a cycle for one level
@@ -710,15 +710,15 @@ __device__ __forceinline__ void rb_dispatch(const Tile &t, const LevelDev &L, in
 // face the red value from before the sweep (`old`), as the ghosts hold it;
 // across a wall the product of a zero coefficient and a zero, as the cells
 // beyond are never set.  The result goes to the other buffer, once: the
-// launch is one step of the level's buffers whatever NS.  zero != 0: the
+// launch is one step of the level's buffers.  zero != 0: the
 // level holds zeros.
 constexpr int RBT = 16, RBT_HALF = RBT * RBT * RBT / 2, RBT_THREADS = 1024;
-template <class T, int NS>
+template <class T>
 __global__ void __launch_bounds__(RBT_THREADS, sizeof(T) == 4 ? 8 : 4)
     k_rb_tile(const LevelDev *__restrict__ levs, const int *__restrict__ active, int src, int zero,
               int one_lev, int one_blk, int tx, int ty, int ntiles,
               const FineDev *__restrict__ fine) {
-  constexpr int HALO = 2 * NS, TS = RBT - 2 * HALO, U = RBT_HALF / RBT_THREADS;
+  constexpr int HALO = 4, TS = RBT - 2 * HALO, U = RBT_HALF / RBT_THREADS;
   __shared__ T black[RBT_HALF], red[RBT_HALF], old[RBT_HALF];
   const LevelDev &L = levs[one_lev];
   const int on = active[one_blk];
@@ -791,7 +791,7 @@ __global__ void __launch_bounds__(RBT_THREADS, sizeof(T) == 4 ? 8 : 4)
     return rx >= lo && rx <= hi && ry >= lo && ry <= hi && rz >= lo && rz <= hi;
   };
 #pragma unroll 1
-  for (int h = 0; h < 2 * NS; h += 2) {
+  for (int h = 0; h < HALO; h += 2) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int q = tid + u * RBT_THREADS, rz = (tid >> 7) + RBT_THREADS / 128 * u;
@@ -5086,13 +5086,11 @@ void launch_lsm_restrict(hipStream_t s, const Tile *tiles, int ntiles, const Lev
 
 template <class T>
 void launch_rb_tile(hipStream_t s, const LevelDev *levs, const int *active, int src, int zero,
-                    OneDesc one, int nsweep, int ni, int nj, int nk, const FineDev *upd) {
-  const int ts = RBT - 4 * nsweep;
-  auto n = [ts](int c) { return (c + ts - 1) / ts; };
+                    OneDesc one, int ni, int nj, int nk, const FineDev *upd) {
+  auto n = [](int c) { return (c + 7) / 8; };
   const int ntiles = n(ni) * n(nj) * n(nk);
-  auto k = nsweep == 2 ? k_rb_tile<T, 2> : k_rb_tile<T, 1>;
-  hipLaunchKernelGGL(k, dim3(ntiles), dim3(RBT_THREADS), 0, s, levs, active, src, zero, one.lev,
-                     one.blk, n(ni), n(nj), ntiles, upd);
+  hipLaunchKernelGGL(k_rb_tile<T>, dim3(ntiles), dim3(RBT_THREADS), 0, s, levs, active, src, zero,
+                     one.lev, one.blk, n(ni), n(nj), ntiles, upd);
 }
 
 template <class T>
@@ -5419,9 +5417,9 @@ template void launch_residual<double>(hipStream_t, const Tile *, int, int, const
 template void launch_residual<float>(hipStream_t, const Tile *, int, int, const FineDev *,
                                      const LevelDev *, const int *, RedPartial *, int, int);
 template void launch_rb_tile<double>(hipStream_t, const LevelDev *, const int *, int, int, OneDesc,
-                                     int, int, int, int, const FineDev *);
+                                     int, int, int, const FineDev *);
 template void launch_rb_tile<float>(hipStream_t, const LevelDev *, const int *, int, int, OneDesc,
-                                    int, int, int, int, const FineDev *);
+                                     int, int, int, const FineDev *);
 template void launch_set_rhs<double>(hipStream_t, const Tile *, int, int, const FineDev *,
                                      const LevelDev *, const double *, RedPartial *);
 template void launch_set_rhs<float>(hipStream_t, const Tile *, int, int, const FineDev *,

@@ -105,7 +105,7 @@ struct TileSet {
   bool tdma_lines = false;  // TDMA passes in two launches (tiles: one per block)
   int tdma_len[3] = {0, 0, 0};       // their longest line per pass
   OneDesc one;             // every tile on one descriptor: passed to the kernels
-  bool multi = false;      // smoother sets: whole sweeps of one mid-size level per launch
+  bool multi = false;      // smoother sets: pairs of sweeps of one mid-size level per launch
   int n() const { return (int)h.size(); }
 };
 
@@ -497,19 +497,17 @@ void dev_free(h3dmg_handle *h, void *p) {
 template <class T>
 void relax_group(h3dmg_handle *h, const TileSet &ts, int nsweep, int &buf, bool &zero,
                  bool red_done = false, bool upd = false) {
-  if (ts.multi && !h->lsm) {  // up to two sweeps a launch, one buffer step each
+  int done = 0;
+  if (ts.multi && !h->lsm) {  // pairs of sweeps, one buffer step each
     const LevelDev &L = h->levs[ts.one.lev];
-    for (int left = nsweep; left > 0;) {
-      const int n = std::min(left, 2);
-      left -= n;
-      launch_rb_tile<T>(h->stream, h->d_levs, h->d_active, buf, zero ? 1 : 0, ts.one, n, L.ni, L.nj,
-                        L.nk, upd && left == 0 ? h->d_fine : nullptr);
+    for (; nsweep - done >= 2; done += 2) {
+      launch_rb_tile<T>(h->stream, h->d_levs, h->d_active, buf, zero ? 1 : 0, ts.one, L.ni, L.nj,
+                        L.nk, upd && done + 2 == nsweep ? h->d_fine : nullptr);
       buf ^= 1;
       zero = false;
     }
-    return;
   }
-  for (int s = 0; s < nsweep; ++s) {
+  for (int s = done; s < nsweep; ++s) {
     if (h->prm.smoother == H3DMG_SMOOTH_GS)  // tile wavefront (every level FP64)
       for (int d = 0; d + 1 < (int)ts.diag_begin.size(); ++d)
         launch_gs_tiles(h->stream, ts.d + ts.diag_begin[d], ts.diag_begin[d + 1] - ts.diag_begin[d],
@@ -584,7 +582,7 @@ bool red1_write(const h3dmg_handle *h) {
   const h3dmg_params &P = h->prm;
   return !is_mixed(h) && P.smoother == H3DMG_SMOOTH_RBGS && !h->lsm && !h->connected &&
          P.nu1 > 0 && ((P.nu1 + P.nu2) & 1) == 0 && h->fine_tiles.depth > 0 &&
-         !h->relax_nc[1].multi && !h->relax_c[1].multi;
+         !(P.nu1 >= 2 && (h->relax_nc[1].multi || h->relax_c[1].multi));
 }
 
 // Whether level 1's last post-smoothing sweep can add the correction to p: a
@@ -624,13 +622,13 @@ void enqueue_vcycle(h3dmg_handle *h, bool red1, bool update) {
                       h->restr_nc[g].n() && h->restr_nc[g].depth > 0
                 : red1 && red1_write(h)) &&
         g < Lt && g < Lm && h->prm.nu1 > 0 && h->relax_nc[g].n() && !h->relax_nc[g].fused &&
-        !h->relax_nc[g].multi && z_nc[g];
+        !(nu1 >= 2 && h->relax_nc[g].multi) && z_nc[g];
     // likewise for the blocks whose coarsest level g is smoothed (not solved)
     const bool red_c_by_restr = g >= 2 && g < Lt && !(exact && g > 1) && h->prm.nu1 > 0 &&
                                 h->prm.smoother == H3DMG_SMOOTH_RBGS && !h->lsm &&
                                 !h->connected && h->restr_c[g].n() &&
                                 h->restr_c[g].depth > 0 && h->relax_c[g].n() &&
-                                !h->relax_c[g].fused && !h->relax_c[g].multi;
+                                !h->relax_c[g].fused && !(nu1 >= 2 && h->relax_c[g].multi);
     if (g >= 2) {
       // mgrestr(g): residual of level g-1 (non-coarsest there) into rhs_g
       const bool f64 = nc_is64(g - 1);
