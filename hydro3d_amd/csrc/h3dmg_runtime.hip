@@ -1753,22 +1753,32 @@ size_t tail_lds_at(const h3dmg_handle *h, int g, bool padded) {
 // Automatic tail level, 0 < g < the coarsest: the first level from which every
 // block's remaining levels fit in one workgroup's LDS and whose cells the tail
 // kernel keeps in registers (TAIL_FAST_ENTRIES per colour: 16^3), for handles
-// whose blocks all have the same number of levels.  Measured per cycle, tail
-// from 16^3 | every level its own launches, us: one 64^3 of 4 levels, mixed,
-// exact coarsest 122 | 135, FP64 smoothed 119 | 137; 48 of them 458 | 489 and
-// 653 | 677; 96 of 32^3, FP64 300 | 351.  The coarsest level alone is left to
-// its launches: an exact solve there takes 62 (16^3 blocks) to 74 (28^3) us a
-// two-level cycle in the tail's one workgroup, 55 to 59 spread over the chip,
-// a smoothed one as long either way.  Handles of unequal depths: with the
-// exact solve the first level from the shallowest block's coarsest down that
-// fits (the deeper blocks' levels and all exact solves in one launch).
+// whose blocks all have the same number of levels, and where the sweeps saved
+// pay for the kernel: three levels or more with two sweeps or more per visit
+// pair (nu1 + nu2), two levels with three sweeps or more, and five where the
+// launches would take pairs of sweeps (one block, TileSet::multi).  Measured per cycle, tail from 16^3 | every level its own launches, us:
+// three levels (32^3 of 4, FP64) V(2,2) 81 | 90, V(1,1) 73 | 83, 48 blocks
+// V(2,2) 134 | 181; two levels (32^3 of 3), one block, mixed exact, V(2,2)
+// 72 | 66, V(3,3) 84 | 88, FP64 smoothed 74 | 72 and 89 | 107; 48 blocks
+// V(2,2) 126 | 150, V(2,1) 115 | 127, 16 blocks V(1,1) 72 | 69; V(1,0) of three
+// levels 82 | 78.  The coarsest level alone is left to its launches: an exact
+// solve there takes 62 (16^3 blocks) to 74 (28^3) us a two-level cycle in the
+// tail's one workgroup, 55 to 59 spread over the chip, a smoothed one as long
+// either way.  Handles of unequal depths: with the exact solve the first level
+// from the shallowest block's coarsest down that fits (the deeper blocks'
+// levels and all exact solves in one launch).
 int auto_tail_level(const h3dmg_handle *h) {
   const bool exact = h->prm.coarse == H3DMG_COARSE_EXACT;
   int t0 = h->Lmax;
   for (const BlockInfo &B : h->blk) t0 = std::min(t0, B.L);
   const bool equal = t0 == h->Lmax;
   for (int g = 1; g <= h->Lmax; ++g) {
-    bool want = equal ? g < h->Lmax : exact && g >= t0;
+    const int levels = h->Lmax - g + 1, sweeps = h->prm.nu1 + h->prm.nu2;
+    bool pairs = h->nb == 1;  // the launches in place of the tail take pairs of sweeps
+    for (int q = g; q <= h->Lmax; ++q)
+      pairs = pairs && (q < h->Lmax ? h->relax_nc[q].multi : exact || h->relax_c[q].multi);
+    bool want = equal ? g < h->Lmax && sweeps >= (levels >= 3 ? 2 : pairs ? 5 : 3)
+                      : exact && g >= t0;
     if (equal)
       for (const BlockInfo &B : h->blk) {
         const LevelDev &L = h->levs[B.desc[g]];
