@@ -107,6 +107,8 @@ struct TileSet {
   OneDesc one;             // every tile on one descriptor: passed to the kernels
   bool multi = false;      // smoother sets: pairs of sweeps of one mid-size level per launch
   int n() const { return (int)h.size(); }
+  // buffer steps of `sweeps` sweeps: one each, or one a pair
+  int steps(int sweeps) const { return multi ? (sweeps + 1) / 2 : sweeps; }
 };
 
 // ts.one: the descriptor of every tile of the set, if they share one, with
@@ -498,7 +500,7 @@ template <class T>
 void relax_group(h3dmg_handle *h, const TileSet &ts, int nsweep, int &buf, bool &zero,
                  bool red_done = false, bool upd = false) {
   int done = 0;
-  if (ts.multi && !h->lsm) {  // pairs of sweeps, one buffer step each
+  if (ts.multi) {  // pairs of sweeps, one buffer step each
     const LevelDev &L = h->levs[ts.one.lev];
     for (; nsweep - done >= 2; done += 2) {
       launch_rb_tile<T>(h->stream, h->d_levs, h->d_active, buf, zero ? 1 : 0, ts.one, L.ni, L.nj,
@@ -599,8 +601,11 @@ bool sweep_updates(const h3dmg_handle *h) {
 // black half.  Per level the schedule is relax(g, nu1) on the way
 // down and relax(g, nu2) after mgcorr on the way up; at a block's coarsest
 // level relax(L, nu1) + relax(L, nu2) (the reference) or the exact solve.
-// Sweep counts per level are nu1 + nu2 for every block, so the buffer that
-// holds a level at mgcorr time is the same for all blocks.
+// The buffer that holds a level is tracked per group (blocks that go on
+// coarsening, buf_nc, and blocks whose coarsest level it is, buf_c): a group
+// that takes pairs of sweeps (TileSet::multi) makes fewer buffer steps.  At
+// the end of level 1 both groups' corrections lie in one buffer, pp_buf
+// (gen_relax sees to it).
 // update: p = p + (pp - 0) of the result as well.
 void enqueue_vcycle(h3dmg_handle *h, bool red1, bool update) {
   const int nu1 = h->prm.nu1, nu2 = h->prm.nu2, Lm = h->Lmax;
@@ -737,7 +742,8 @@ void enqueue_vcycle(h3dmg_handle *h, bool red1, bool update) {
       relax_any(h, f64, h->relax_nc[g], nu2, buf_nc[g], z, false, upd && g == 1);
     }
   }
-  // the level-1 correction pp: blocks with L_b == 1 hold it in buf_c[1]
+  // the level-1 correction pp of every block: where both groups have blocks,
+  // buf_c[1] == buf_nc[1]
   h->pp_buf = (h->relax_c[1].n() && !h->relax_nc[1].n()) ? buf_c[1] : buf_nc[1];
   if (!update || upd) return;
   const TileSet &ut = h->update_tiles;
@@ -1698,8 +1704,8 @@ h3dmg_status gen_relax(h3dmg_handle *h, int g) {
     // sweeps on its first level, 768 tiles, too); FP32 48^3 76 | 95, 64^3
     // 103 | 117, 104x56x40 86 | 103.  A depth asked for by h3dmg_set_march
     // keeps the half-sweeps.
-    ts.multi = h->prm.smoother == H3DMG_SMOOTH_RBGS && !general && !ts.fused && ts.one.lev >= 0 &&
-               h->march_kb[g] == 0;
+    ts.multi = h->prm.smoother == H3DMG_SMOOTH_RBGS && !h->lsm && !general && !ts.fused &&
+               ts.one.lev >= 0 && h->march_kb[g] == 0;
     if (ts.multi) {
       const LevelDev &L = h->levs[ts.one.lev];
       const int n[3] = {L.ni, L.nj, L.nk};
@@ -1710,6 +1716,14 @@ h3dmg_status gen_relax(h3dmg_handle *h, int g) {
       }
       const bool is64 = !is_mixed(h) || grp == 1;
       ts.multi = ts.multi && tiles <= (is64 ? 1 : 2) * RB_TILE_CUS;
+    }
+    // Level 1 ends in one buffer for every block (pp_buf, read by the update
+    // and h3dmg_get_pp).  Blocks of one level beside deeper ones are two
+    // groups, each with its own rule above: pairs only where they end in the
+    // buffer that single sweeps end in (V(2,2) and V(1,1) do, V(2,1) does not).
+    if (ts.multi && g == 1 && !std::all_of(h->blk.begin(), h->blk.end(), member)) {
+      const int nu1 = h->prm.nu1, nu2 = h->prm.nu2;
+      ts.multi = ((ts.steps(nu1) + ts.steps(nu2) + nu1 + nu2) & 1) == 0;
     }
   }
   return H3DMG_OK;
