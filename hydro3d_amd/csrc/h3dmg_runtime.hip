@@ -578,13 +578,18 @@ void fill_any(h3dmg_handle *h, bool is64, const TileSet &ts, int buf) {
 // where the first half-sweep from buffer 0 puts it): an FP64 level 1 (in
 // mixed precision the FP32 residual slows by more than the half-sweep costs),
 // the red-black smoother, constant coefficients, no neighbours, nu1 > 0, and
-// nu1 + nu2 even (the correction pp then lies in buffer 0 and stays
-// untouched).
+// the correction pp in buffer 0, where it stays untouched: after an even number
+// of buffer steps, which are the sweeps (in the tail, too) or fewer where
+// sweeps go in pairs; a pair computes that half itself.
 bool red1_write(const h3dmg_handle *h) {
   const h3dmg_params &P = h->prm;
+  bool pp0 = ((P.nu1 + P.nu2) & 1) == 0, pair = false;
+  for (const TileSet *ts : {&h->relax_nc[1], &h->relax_c[1]}) {
+    pp0 = pp0 && ((ts->steps(P.nu1) + ts->steps(P.nu2)) & 1) == 0;
+    pair = pair || (ts->multi && P.nu1 >= 2);
+  }
   return !is_mixed(h) && P.smoother == H3DMG_SMOOTH_RBGS && !h->lsm && !h->connected &&
-         P.nu1 > 0 && ((P.nu1 + P.nu2) & 1) == 0 && h->fine_tiles.depth > 0 &&
-         !(P.nu1 >= 2 && (h->relax_nc[1].multi || h->relax_c[1].multi));
+         P.nu1 > 0 && pp0 && !pair && h->fine_tiles.depth > 0;
 }
 
 // Whether level 1's last post-smoothing sweep can add the correction to p: a
