@@ -313,6 +313,7 @@ struct h3dmg_handle {
   int proj_kb = 1, proj_groups = 1;
   VelDev *d_vel = nullptr;
   ProjDt *d_projdt = nullptr;
+  std::vector<char> vel_img;  // host image of both, the source of their upload
   RedPartial *d_pparts = nullptr;  // proj_groups partials per block
   int *d_pp_begin = nullptr;
   // an input array of the velocity loop overlaps an output one: per-axis
@@ -3365,9 +3366,11 @@ bool velocity_overlap(const h3dmg_handle *h) {
   return ranges_overlap(in, out);
 }
 
-// the blocks' arrays and the time step to the tables k_project reads
+// the blocks' arrays and the time step to the tables k_project reads; the
+// copy's source stays in the handle until the caller has waited for the stream
 h3dmg_status push_velocity(h3dmg_handle *h) {
-  std::vector<char> img(h->nb * sizeof(VelDev) + sizeof(ProjDt));
+  std::vector<char> &img = h->vel_img;
+  img.resize(h->nb * sizeof(VelDev) + sizeof(ProjDt));
   VelDev *t = (VelDev *)img.data();
   for (int b = 0; b < h->nb; ++b) {
     const h3dmg_handle::VelBlock &V = h->vel[b];
