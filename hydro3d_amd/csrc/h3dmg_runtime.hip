@@ -259,6 +259,10 @@ struct h3dmg_handle {
 
   char *arena = nullptr;
   size_t arena_bytes = 0;
+  // workspace of the two-launch line passes (LevelDev::tdma_ws), or null
+  bool want_line_ws = true;
+  char *line_ws = nullptr;
+  size_t line_ws_bytes = 0;
 
   std::vector<LevelDev> levs;  // level-major: all blocks' level 1 first
   std::vector<int> lev_is64;   // storage type of each descriptor
@@ -1131,21 +1135,33 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
       tdma_off[d] = boff[L.blk];
       boff[L.blk] = align_up(boff[L.blk] + (size_t)32 * (L.ni + L.nj + L.nk) * 8, 256);
     }
-  // line passes in two launches: one workspace per block, as large as its
-  // largest level that takes them needs
-  std::vector<size_t> tws_off(nblocks, 0), tws_len(nblocks, 0);
-  if (h->prm.smoother == H3DMG_SMOOTH_TDMA)
-    for (int b = 0; b < nblocks; ++b) {
-      for (int g = 1; g <= h->blk[b].L; ++g) {
-        const LevelDev &L = h->levs[h->blk[b].desc[g]];
-        if (tdma_lines_fit(L)) tws_len[b] = std::max(tws_len[b], tdma_ws_doubles(L));
-      }
-      tws_off[b] = boff[b];
-      boff[b] = align_up(boff[b] + tws_len[b] * 8, 256);
-    }
   if (region_bytes) {
     for (int b = 0; b < nblocks; ++b) region_bytes[b] = boff[b];
     return H3DMG_OK;
+  }
+  // Line passes in two launches: one workspace per block, as large as its
+  // largest level that takes them needs (8.3 MB for 64^3 cells, whose region
+  // has 12).  It is an allocation beside the arena and optional: a pooled
+  // handle, which allocates nothing, and one that memory does not suffice for
+  // run the sweeps that need none.
+  std::vector<size_t> tws_off(nblocks, 0);
+  if (h->prm.smoother == H3DMG_SMOOTH_TDMA && h->want_line_ws && !h->pool) {
+    size_t total = 0;
+    for (int b = 0; b < nblocks; ++b) {
+      size_t len = 0;
+      for (int g = 1; g <= h->blk[b].L; ++g) {
+        const LevelDev &L = h->levs[h->blk[b].desc[g]];
+        if (tdma_lines_fit(L)) len = std::max(len, tdma_ws_doubles(L));
+      }
+      tws_off[b] = total;
+      total = align_up(total + len * 8, 256);
+    }
+    if (total && hipMalloc((void **)&h->line_ws, total) == hipSuccess) {
+      h->line_ws_bytes = total;
+    } else {
+      h->line_ws = nullptr;
+      (void)hipGetLastError();  // not an error of the launches to come
+    }
   }
   // staging: largest padded level-1 array (a pooled handle takes device
   // arrays only, and has none)
@@ -1369,10 +1385,12 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
     total += off;
     h->arena_bytes = total;
     hipError_t e = hipMalloc((void **)&h->arena, total);
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+      h->arena = nullptr;
       return fail(H3DMG_ERR_NOMEM, "hipMalloc(%zu bytes) failed: %s", total,
                   hipGetErrorString(e));
-    h->bytes = total;
+    }
+    h->bytes = total + h->line_ws_bytes;
     for (int b = 0; b < nblocks; ++b) R[b] = h->arena + rbase[b];
     A = h->arena + gbase;
   }
@@ -1383,7 +1401,7 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
       for (int c = 0; c < 2; ++c) L.phi[bb][c] = R[P.b] + P.phi[bb][c];
     for (int c = 0; c < 2; ++c) L.rhs[c] = R[P.b] + P.rhs[c];
     if (h->prm.smoother == H3DMG_SMOOTH_TDMA) L.tdma = (double *)(R[P.b] + tdma_off[P.d]);
-    if (tws_len[P.b] && tdma_lines_fit(L)) L.tdma_ws = (double *)(R[P.b] + tws_off[P.b]);
+    if (h->line_ws && tdma_lines_fit(L)) L.tdma_ws = (double *)(h->line_ws + tws_off[P.b]);
   }
   h->fine.resize(nblocks);
   for (int b = 0; b < nblocks; ++b) {
@@ -1628,9 +1646,9 @@ h3dmg_status gen_relax(h3dmg_handle *h, int g) {
         }
         ts.diag_begin.push_back(ts.n());
       } else {
-        // every axis of every block within a wavefront's lanes: two launches
-        // per pass (constant coefficients)
-        bool lines = !h->lsm;
+        // every axis of every block within a wavefront's lanes, and the
+        // workspace there: two launches per pass (constant coefficients)
+        bool lines = !h->lsm && h->line_ws;
         for (int pass = 0; pass < 3; ++pass) ts.tdma_len[pass] = 0;
         for (const BlockInfo &B : h->blk)
           if (member(B)) {
@@ -2134,6 +2152,7 @@ static void destroy_locked(h3dmg_handle *h) {
   if (h->h_stats) (void)hipHostFree(h->h_stats);
   if (h->vel_store) (void)hipFree(h->vel_store);
   if (h->lsm_store) (void)hipFree(h->lsm_store);
+  if (h->line_ws) (void)hipFree(h->line_ws);
   if (h->arena) (void)hipFree(h->arena);
   if (h->own_stream && h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
@@ -2160,7 +2179,8 @@ h3dmg_status check_params(const h3dmg_params &P) {
 // h3dmg_create and h3dmg_create_pooled; the caller holds g_device_mutex
 h3dmg_status create_locked(const h3dmg_block *blocks, int nblocks, const h3dmg_params *prm,
                            h3dmg_pool *pool, const unsigned long long *offsets,
-                           const int *fresh, void *stream, h3dmg_handle **out) {
+                           const int *fresh, void *stream, h3dmg_handle **out,
+                           bool line_ws = true) {
   if (!out) return fail(H3DMG_ERR_ARG, "null output handle pointer");
   *out = nullptr;
   if (!blocks || nblocks < 1) return fail(H3DMG_ERR_ARG, "no blocks");
@@ -2187,6 +2207,7 @@ h3dmg_status create_locked(const h3dmg_block *blocks, int nblocks, const h3dmg_p
   h3dmg_handle *h = new h3dmg_handle();
   h->prm = P;
   h->device = dev;
+  h->want_line_ws = line_ws;
   int lds = 0;
   if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
     lds = 65536;
@@ -2209,8 +2230,11 @@ h3dmg_status create_locked(const h3dmg_block *blocks, int nblocks, const h3dmg_p
   }
   h3dmg_status st = build(h, blocks, nblocks, fresh);
   if (st != H3DMG_OK) {
+    const bool had_ws = h->line_ws;
     destroy_locked(h);
-    return st;
+    if (st != H3DMG_ERR_NOMEM || !had_ws) return st;
+    (void)hipGetLastError();  // the workspace took the room: without it
+    return create_locked(blocks, nblocks, prm, pool, offsets, fresh, stream, out, false);
   }
   h->running.assign(nblocks, 0);
   h->outcome.assign(nblocks, -1);

@@ -15,12 +15,11 @@ typedef struct {
 } Copy;
 static Copy pending[4096];
 static int npending, late;
-static size_t room = (size_t)-1, largest; /* bytes hipMalloc still gives */
+static size_t room = (size_t)1 << 40; /* bytes hipMalloc still gives */
 
 int fake_late_sources(void) { return late; }
 void fake_set_room(size_t bytes) { room = bytes; }
 size_t fake_room(void) { return room; }
-size_t fake_largest(void) { return largest; }
 
 static void finish(void) {
   for (int q = 0; q < npending; ++q) {
@@ -32,22 +31,27 @@ static void finish(void) {
   npending = 0;
 }
 
-int hipMalloc(void **p, size_t n) {
-  if (n > room) return 2; /* hipErrorOutOfMemory */
-  room -= n;
-  largest = n > largest ? n : largest;
-  return (*p = calloc(n, 1)) ? 0 : 2;
+int hipMalloc(void **p, size_t n) { /* its size lies before the memory */
+  size_t *q = n > room ? NULL : calloc(n + 64, 1);
+  if (!q) return 2; /* hipErrorOutOfMemory */
+  room -= *q = n;
+  *p = q + 8;
+  return 0;
 }
 int hipFree(void *p) {
   finish();
-  free(p);
+  if (p) room += *((size_t *)p - 8), free((size_t *)p - 8);
   return 0;
 }
 int hipHostMalloc(void **p, size_t n, unsigned f) {
   (void)f;
   return (*p = calloc(n, 1)) ? 0 : 2;
 }
-int hipHostFree(void *p) { return hipFree(p); }
+int hipHostFree(void *p) {
+  finish();
+  free(p);
+  return 0;
+}
 int hipHostGetDevicePointer(void **d, void *h, unsigned f) {
   (void)f;
   *d = h;

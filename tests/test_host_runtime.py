@@ -54,3 +54,44 @@ for _ in range(2):
 print(before, fake.fake_late_sources())
 """)
     assert out == ["0", "0"]
+
+
+def test_line_workspace_is_optional(fake):
+    """A line-TDMA block's region is what its levels, p, f and tables take
+    (the line passes' workspace is not in it), and a handle is made where
+    memory suffices for everything but that workspace."""
+    out = fake("""
+from hydro3d_amd.solver import block_bytes
+al = lambda x: (x + 255) // 256 * 256
+def expect(n, nlev):
+    tot = 0
+    for g in range(nlev):
+        ni, nj, nk = (x >> g for x in n)
+        tot += 6 * al((((ni + 1) // 2 + 1) & ~1) * nj * nk * 8) + al(32 * (ni + nj + nk) * 8)
+    return tot + 4 * al((((n[0] + 1) // 2 + 1) & ~1) * n[1] * n[2] * 8)
+ok = True
+for n, nlev in (((64, 64, 64), 5), ((32, 32, 32), 1), ((48, 16, 130), 2)):
+    spec = dict(n=n, h=(0.1,) * 3, bc=(0,) * 6, nlev=nlev)
+    ok = ok and block_bytes(spec, smoother="tdma") == expect(n, nlev)
+fake.fake_set_room.argtypes = [ctypes.c_size_t]
+fake.fake_room.restype = ctypes.c_size_t
+fake.fake_set_room(1 << 30)
+blocks = [((32, 32, 32), 3), ((16, 24, 20), 2)]
+S = handle(blocks, smoother="tdma")
+used = (1 << 30) - fake.fake_room()
+assert S.device_bytes == used, (S.device_bytes, used)
+S.close()
+fake.fake_set_room(used - 1)  # either allocation fits, not both
+S = handle(blocks, smoother="tdma")
+small = S.device_bytes
+assert small == used - 1 - fake.fake_room()
+S.close()
+fake.fake_set_room(small)
+handle(blocks, smoother="tdma").close()
+fake.fake_set_room(small - 1)
+try:
+    handle(blocks, smoother="tdma")
+except L.H3dError as e:
+    print(ok, e.status == L.ERR_NOMEM)
+""")
+    assert out == ["True", "True"]
