@@ -318,7 +318,7 @@ struct h3dmg_handle {
   VelDev *d_vel = nullptr;
   ProjDt *d_projdt = nullptr;
   std::vector<char> vel_img;  // host image of both, the source of their upload
-  RedPartial *d_pparts = nullptr;  // proj_groups partials per block
+  RedPartial *d_pparts = nullptr;  // proj_groups partials per block (not pooled)
   int *d_pp_begin = nullptr;
   // an input array of the velocity loop overlaps an output one: per-axis
   // launches (k_calvel*, k_calmas), which read each face before they write it
@@ -1348,12 +1348,15 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
           h->proj_groups, project_tiles(blocks[b].ni, blocks[b].nj, blocks[b].nk, h->proj_kb));
     h->proj_groups = std::min(h->proj_groups, PROJ_MAX_GROUPS);
   }
+  // the velocity loop's tables and partials (a pooled handle has no such loop;
+  // a projection of one block uses its range of d_proj)
+  const size_t nvel = h->pool ? 0 : nblocks;
   const size_t vel_tab_off = off;
-  off = align_up(off + nblocks * sizeof(VelDev) + sizeof(ProjDt), 256);
+  off = align_up(off + nvel * sizeof(VelDev) + (nvel ? sizeof(ProjDt) : 0), 256);
   const size_t pparts_off = off;
-  off = align_up(off + (size_t)nblocks * h->proj_groups * sizeof(RedPartial), 256);
+  off = align_up(off + nvel * h->proj_groups * sizeof(RedPartial), 256);
   const size_t ppb_off = off;
-  off = align_up(off + (nblocks + 1) * sizeof(int), 256);
+  off = align_up(off + (nvel ? nvel + 1 : 0) * sizeof(int), 256);
   const size_t eptr_off = off;
   off = align_up(off + (size_t)nblocks * 8 * sizeof(double *), 256);
 
@@ -1455,11 +1458,11 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
   h->d_proj = (RedPartial *)(A + proj_off);
   h->d_proj_begin = (int *)(A + pb_off);
   put(pb_off, h->proj_begin.data(), (nblocks + 1) * sizeof(int));
-  h->d_vel = (VelDev *)(A + vel_tab_off);
-  h->d_projdt = (ProjDt *)(A + vel_tab_off + nblocks * sizeof(VelDev));
-  h->d_pparts = (RedPartial *)(A + pparts_off);
-  h->d_pp_begin = (int *)(A + ppb_off);
-  {
+  if (nvel) {
+    h->d_vel = (VelDev *)(A + vel_tab_off);
+    h->d_projdt = (ProjDt *)(A + vel_tab_off + nblocks * sizeof(VelDev));
+    h->d_pparts = (RedPartial *)(A + pparts_off);
+    h->d_pp_begin = (int *)(A + ppb_off);
     std::vector<int> pp_begin(nblocks + 1);
     for (int b = 0; b <= nblocks; ++b) pp_begin[b] = b * h->proj_groups;
     put(ppb_off, pp_begin.data(), (nblocks + 1) * sizeof(int));
@@ -3000,9 +3003,8 @@ h3dmg_status h3dmg_project_device(h3dmg_handle *h, int b, const double *d_ustar,
   if (project_one_overlaps(h, b, V)) {
     groups = enqueue_project_axes(h, b, V, dt * alfapr, parts);
   } else {
-    parts = h->d_pparts + (size_t)b * h->proj_groups;
-    groups = h->proj_groups;
-    const ProjLaunch a = project_shape(h);
+    ProjLaunch a = project_shape(h);
+    a.groups = groups = std::min(a.groups, h->proj_begin[b + 1] - h->proj_begin[b]);
     launch_project(h->stream, a, h->d_fine, h->d_levs, nullptr, nullptr, nullptr, V,
                    ProjDt{dt * alfapr, dt}, b, 1, parts);
   }

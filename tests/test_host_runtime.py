@@ -95,3 +95,24 @@ except L.H3dError as e:
     print(ok, e.status == L.ERR_NOMEM)
 """)
     assert out == ["True", "True"]
+
+
+@pytest.mark.parametrize("kw,before", [(dict(precision="mixed", coarse="exact"), 564736),
+                                       (dict(), 550656), (dict(smoother="tdma"), 488960)],
+                         ids=["mixed", "fp64", "tdma"])
+def test_pooled_tables_have_not_grown(fake, kw, before):
+    """The pool piece of a pooled handle's tables, for one large block and
+    many small ones: no more than before the projection had partials and
+    tables for every block (a pooled handle has no velocity loop)."""
+    out = fake(f"""
+from hydro3d_amd import MultigridSolver
+from hydro3d_amd.solver import DevicePool, block_bytes
+kw = {kw!r}
+specs = [dict(n=n, h=(0.1,) * 3, bc=(0,) * 6, nlev=q)
+         for n, q in [((256, 256, 32), 4)] + [((16, 16, 16), 3)] * 20]
+P = DevicePool(1 << 28, 64)
+offs = [P.alloc(block_bytes(s, **kw)) for s in specs]
+S = MultigridSolver(specs, pool=P, offsets=offs, **kw)
+print(S.device_bytes)
+""")
+    assert int(out[0]) <= before
