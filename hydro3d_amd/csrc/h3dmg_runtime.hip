@@ -2862,6 +2862,8 @@ h3dmg_status h3dmg_set_block_state(h3dmg_handle *h, int b, const h3dmg_block_sta
   B.fnorm = in->fnorm;
   B.rel = in->rel;
   B.tol = in->tol;
+  // (the velocity loop's last projection left a block enabled here out)
+  if (B.enabled != (in->enabled != 0)) h->rhs_is_f = false;
   B.enabled = in->enabled != 0;
   h->running[b] = (in->running && B.enabled) ? 1 : 0;
   h->outcome[b] = in->status;
