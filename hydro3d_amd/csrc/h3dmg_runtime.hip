@@ -986,6 +986,12 @@ h3dmg_status validate_blocks(const h3dmg_block *blocks, int nblocks, const h3dmg
   return validate_neighbours(blocks, nblocks, P);
 }
 
+// workgroups of k_project over block b alone
+int project_groups(const h3dmg_handle *h, int b) {
+  const h3dmg_block &S = h->blk[b].spec;
+  return std::min(project_tiles(S.ni, S.nj, S.nk, h->proj_kb), PROJ_MAX_GROUPS);
+}
+
 // dynamic LDS the exact solve's kernels may use (a process-wide attribute of
 // the kernels: set once, to the device's budget)
 size_t exact_lds_budget(const h3dmg_handle *h) {
@@ -1319,18 +1325,6 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
   off = align_up(off + std::max<size_t>(1, h->fine_tiles.h.size()) * sizeof(RedPartial), 256);
   const size_t stats_off = off;
   off = align_up(off + nblocks * sizeof(RedPartial), 256);
-  // calmas partials: one range per block (its workgroup count)
-  h->proj_begin.assign(nblocks + 1, 0);
-  for (int b = 0; b < nblocks; ++b) {
-    const BlockInfo &B = h->blk[b];
-    const size_t cells = (size_t)B.spec.ni * B.spec.nj * B.spec.nk;
-    h->proj_begin[b + 1] =
-        h->proj_begin[b] + (int)std::min<size_t>((cells + 255) / 256, CALMAS_MAX_GROUPS);
-  }
-  const size_t proj_off = off;
-  off = align_up(off + (size_t)h->proj_begin[nblocks] * sizeof(RedPartial), 256);
-  const size_t pb_off = off;
-  off = align_up(off + (nblocks + 1) * sizeof(int), 256);
   // k_project: as many planes per tile (at most 8) as leave ~1024 tiles over
   // all blocks, and one workgroup per tile up to PROJ_MAX_GROUPS per block.
   // Deeper tiles read their bottom plane of p and w* less often, fewer tiles
@@ -1342,12 +1336,26 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
     for (int b = 0; b < nblocks; ++b)
       tiles += project_tiles(blocks[b].ni, blocks[b].nj, blocks[b].nk, 1);
     h->proj_kb = (int)std::min<long>(8, std::max<long>(1, tiles / 1024));
-    h->proj_groups = 1;
-    for (int b = 0; b < nblocks; ++b)
-      h->proj_groups = std::max(
-          h->proj_groups, project_tiles(blocks[b].ni, blocks[b].nj, blocks[b].nk, h->proj_kb));
-    h->proj_groups = std::min(h->proj_groups, PROJ_MAX_GROUPS);
   }
+  // calmas partials: one range per block (its workgroup count); a projection
+  // of one block takes them too, or, with more workgroups than they have
+  // (blocks of few or short rows), the entries after the last range
+  h->proj_begin.assign(nblocks + 1, 0);
+  h->proj_groups = 1;
+  int proj_more = 0;
+  for (int b = 0; b < nblocks; ++b) {
+    const BlockInfo &B = h->blk[b];
+    const size_t cells = (size_t)B.spec.ni * B.spec.nj * B.spec.nk;
+    const int own = (int)std::min<size_t>((cells + 255) / 256, CALMAS_MAX_GROUPS);
+    const int groups = project_groups(h, b);
+    h->proj_begin[b + 1] = h->proj_begin[b] + own;
+    h->proj_groups = std::max(h->proj_groups, groups);
+    if (groups > own) proj_more = std::max(proj_more, groups);
+  }
+  const size_t proj_off = off;
+  off = align_up(off + ((size_t)h->proj_begin[nblocks] + proj_more) * sizeof(RedPartial), 256);
+  const size_t pb_off = off;
+  off = align_up(off + (nblocks + 1) * sizeof(int), 256);
   // the velocity loop's tables and partials (a pooled handle has no such loop;
   // a projection of one block uses its range of d_proj)
   const size_t nvel = h->pool ? 0 : nblocks;
@@ -3006,7 +3014,8 @@ h3dmg_status h3dmg_project_device(h3dmg_handle *h, int b, const double *d_ustar,
     groups = enqueue_project_axes(h, b, V, dt * alfapr, parts);
   } else {
     ProjLaunch a = project_shape(h);
-    a.groups = groups = std::min(a.groups, h->proj_begin[b + 1] - h->proj_begin[b]);
+    a.groups = groups = project_groups(h, b);
+    if (groups > h->proj_begin[b + 1] - h->proj_begin[b]) parts = h->d_proj + h->proj_begin[h->nb];
     launch_project(h->stream, a, h->d_fine, h->d_levs, nullptr, nullptr, nullptr, V,
                    ProjDt{dt * alfapr, dt}, b, 1, parts);
   }
