@@ -259,9 +259,8 @@ struct h3dmg_handle {
 
   char *arena = nullptr;
   size_t arena_bytes = 0;
-  // workspace of the two-launch line passes (LevelDev::tdma_ws), or null
+  // workspace of the two-launch line passes (LevelDev::tdma_ws); 0: none
   bool want_line_ws = true;
-  char *line_ws = nullptr;
   size_t line_ws_bytes = 0;
 
   std::vector<LevelDev> levs;  // level-major: all blocks' level 1 first
@@ -1147,28 +1146,21 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
   }
   // Line passes in two launches: one workspace per block, as large as its
   // largest level that takes them needs (8.3 MB for 64^3 cells, whose region
-  // has 12).  It is an allocation beside the arena and optional: a pooled
+  // has 12), after everything else in the arena.  It is optional: a pooled
   // handle, which allocates nothing, and one that memory does not suffice for
   // run the sweeps that need none.
   std::vector<size_t> tws_off(nblocks, 0);
-  if (h->prm.smoother == H3DMG_SMOOTH_TDMA && h->want_line_ws && !h->pool) {
-    size_t total = 0;
+  h->line_ws_bytes = 0;
+  if (h->prm.smoother == H3DMG_SMOOTH_TDMA && h->want_line_ws && !h->pool)
     for (int b = 0; b < nblocks; ++b) {
       size_t len = 0;
       for (int g = 1; g <= h->blk[b].L; ++g) {
         const LevelDev &L = h->levs[h->blk[b].desc[g]];
         if (tdma_lines_fit(L)) len = std::max(len, tdma_ws_doubles(L));
       }
-      tws_off[b] = total;
-      total = align_up(total + len * 8, 256);
+      tws_off[b] = h->line_ws_bytes;
+      h->line_ws_bytes = align_up(h->line_ws_bytes + len * 8, 256);
     }
-    if (total && hipMalloc((void **)&h->line_ws, total) == hipSuccess) {
-      h->line_ws_bytes = total;
-    } else {
-      h->line_ws = nullptr;
-      (void)hipGetLastError();  // not an error of the launches to come
-    }
-  }
   // staging: largest padded level-1 array (a pooled handle takes device
   // arrays only, and has none)
   size_t stage = 0;
@@ -1372,6 +1364,7 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
   // in a pool) at the caller's pool offsets plus a piece of the pool
   std::vector<char *> R(nblocks);
   char *A = nullptr;  // the global region
+  char *line_ws = nullptr;
   if (h->pool) {
     for (int b = 0; b < nblocks; ++b) {
       const size_t have = pool_size_at(h->pool, h->blk_off[b]);
@@ -1393,7 +1386,9 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
       total = align_up(total + boff[b], 256);
     }
     const size_t gbase = total;
-    total += off;
+    total = align_up(total + off, 256);
+    const size_t wbase = total;
+    total += h->line_ws_bytes;
     h->arena_bytes = total;
     hipError_t e = hipMalloc((void **)&h->arena, total);
     if (e != hipSuccess) {
@@ -1401,9 +1396,10 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
       return fail(H3DMG_ERR_NOMEM, "hipMalloc(%zu bytes) failed: %s", total,
                   hipGetErrorString(e));
     }
-    h->bytes = total + h->line_ws_bytes;
+    h->bytes = total;
     for (int b = 0; b < nblocks; ++b) R[b] = h->arena + rbase[b];
     A = h->arena + gbase;
+    line_ws = h->arena + wbase;
   }
 
   for (const Pending &P : pend) {
@@ -1412,7 +1408,7 @@ h3dmg_status build(h3dmg_handle *h, const h3dmg_block *blocks, int nblocks,
       for (int c = 0; c < 2; ++c) L.phi[bb][c] = R[P.b] + P.phi[bb][c];
     for (int c = 0; c < 2; ++c) L.rhs[c] = R[P.b] + P.rhs[c];
     if (h->prm.smoother == H3DMG_SMOOTH_TDMA) L.tdma = (double *)(R[P.b] + tdma_off[P.d]);
-    if (h->line_ws && tdma_lines_fit(L)) L.tdma_ws = (double *)(h->line_ws + tws_off[P.b]);
+    if (h->line_ws_bytes && tdma_lines_fit(L)) L.tdma_ws = (double *)(line_ws + tws_off[P.b]);
   }
   h->fine.resize(nblocks);
   for (int b = 0; b < nblocks; ++b) {
@@ -1659,7 +1655,7 @@ h3dmg_status gen_relax(h3dmg_handle *h, int g) {
       } else {
         // every axis of every block within a wavefront's lanes, and the
         // workspace there: two launches per pass (constant coefficients)
-        bool lines = !h->lsm && h->line_ws;
+        bool lines = !h->lsm && h->line_ws_bytes > 0;
         for (int pass = 0; pass < 3; ++pass) ts.tdma_len[pass] = 0;
         for (const BlockInfo &B : h->blk)
           if (member(B)) {
@@ -2163,7 +2159,6 @@ static void destroy_locked(h3dmg_handle *h) {
   if (h->h_stats) (void)hipHostFree(h->h_stats);
   if (h->vel_store) (void)hipFree(h->vel_store);
   if (h->lsm_store) (void)hipFree(h->lsm_store);
-  if (h->line_ws) (void)hipFree(h->line_ws);
   if (h->arena) (void)hipFree(h->arena);
   if (h->own_stream && h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
@@ -2241,7 +2236,7 @@ h3dmg_status create_locked(const h3dmg_block *blocks, int nblocks, const h3dmg_p
   }
   h3dmg_status st = build(h, blocks, nblocks, fresh);
   if (st != H3DMG_OK) {
-    const bool had_ws = h->line_ws;
+    const bool had_ws = h->line_ws_bytes > 0;
     destroy_locked(h);
     if (st != H3DMG_ERR_NOMEM || !had_ws) return st;
     (void)hipGetLastError();  // the workspace took the room: without it
