@@ -2219,7 +2219,8 @@ __device__ __forceinline__ void decide_body(const DecideBlock *__restrict__ bloc
     gmax = gmax < s.rmax ? s.rmax : gmax;
   }
   bad = __any(bad);
-  for (int w = 32; w > 0; w >>= 1) {
+  // the maxima over the lanes that have a block (the others read neither)
+  for (int w = nb > 32 ? 32 : nb > 1 ? 1 << (31 - __clz(nb - 1)) : 0; w > 0; w >>= 1) {
     const double x = __shfl_xor(worst, w), g = __shfl_xor(gmax, w);
     worst = worst < x ? x : worst;
     gmax = gmax < g ? g : gmax;
