@@ -2617,7 +2617,10 @@ __global__ void __launch_bounds__(256)
 // latency and on-chip barriers replace ~3 full-chip launches per level.
 //
 // Every cell's value is the expression of the per-level kernels, in the same
-// order (a wall's term is the product with zero).  The tail's one CU is bound
+// order; a wall's term is the product with zero, where they multiply zero by
+// the cell's own value before the sweep: NaN where that is not finite, so a
+// run whose result is not finite is done again that way (tail_relax_walls).
+// The tail's one CU is bound
 // by instruction issue and, since it runs every piece of code a few times
 // only, by instruction fetches: a thread sets up its entries once per visit
 // of a level (TailCells) and the neighbours then lie constant steps away; no
@@ -2876,17 +2879,70 @@ __device__ __forceinline__ void tail_fill_zero(const TailLev &L, int buf) {
   __syncthreads();
 }
 
+// tail_relax with every wall's term as the per-level kernels have it, cell by
+// cell
+template <class T>
+__device__ __forceinline__ void tail_relax_walls(const TailLev &L, int nsweep, int &buf, bool zero,
+                                                 bool resid) {
+  if (zero) tail_fill_zero<T>(L, buf);
+  const TailSplit split(L);
+  const bool px = L.per & 1, py = L.per & 2, pz = L.per & 4;
+  const T cx = (T)L.cx, cy = (T)L.cy, cz = (T)L.cz;
+  auto at = [&](int b, int c, unsigned e) {
+    return L.phi + (unsigned)(2 * b + c) * L.ps + e * (unsigned)sizeof(T);
+  };
+#pragma clang loop unroll(disable)
+  for (int h = 0; h < 2 * nsweep + (resid ? 2 : 0); ++h) {
+    const int c = h & 1;
+    const bool res = h >= 2 * nsweep;
+#pragma clang loop unroll(disable)
+    for (int e = (int)threadIdx.x; e < L.n; e += TAIL_THREADS) {
+      int m, j, k;
+      split(e, m, j, k);
+      const int i = 2 * m + ((c + j + k) & 1);
+      if (i >= L.ni) continue;
+      // a neighbour inside the level: the other colour, for a black cell after
+      // the red half (a residual reads one buffer only); else its image
+      auto val = [&](int x, int y, int z, bool ghost) -> T {
+        x = image(x, L.ni, px);
+        y = image(y, L.nj, py);
+        z = image(z, L.nk, pz);
+        const int b = !ghost && !res && c ? 1 - buf : buf;
+        return tail_ld<T>(at(b, (x + y + z) & 1, (unsigned)cidx32(L.H, L.nj, x, y, z)));
+      };
+      const T W = val(i - 1, j, k, i == 0), E = val(i + 1, j, k, i == L.ni - 1);
+      const T S = val(i, j - 1, k, j == 0), N = val(i, j + 1, k, j == L.nj - 1);
+      const T B = val(i, j, k - 1, k == 0), U = val(i, j, k + 1, k == L.nk - 1);
+      const T aw = (!px && i == 0) ? T(0) : cx, ae = (!px && i == L.ni - 1) ? T(0) : cx;
+      const T as = (!py && j == 0) ? T(0) : cy, an = (!py && j == L.nj - 1) ? T(0) : cy;
+      const T ab = (!pz && k == 0) ? T(0) : cz, au = (!pz && k == L.nk - 1) ? T(0) : cz;
+      const T ap = T(-1) * (aw + ae + as + an + ab + au);
+      const T r = tail_ld<T>(L.rhs + (unsigned)c * L.rs + (unsigned)e * (unsigned)sizeof(T));
+      const T sum = aw * W + ae * E + as * S + an * N + ab * B + au * U;
+      const T P = res ? tail_ld<T>(at(buf, c, (unsigned)e)) : T(0);
+      tail_st<T>(at(1 - buf, c, (unsigned)e),
+                 res ? r - (sum + ap * P) : div_ap(r - sum, ap, T(1) / ap));
+    }
+    __syncthreads();
+    if (!res) buf ^= c;
+  }
+}
+
 // nsweep sweeps of a level from buffer `buf` (zero: it starts from zeros,
 // filled in here) and, with resid, the residual into the free buffer.  Levels
 // of more than TAIL_U*TAIL_THREADS entries set their cells anew in every
 // pass.
 template <class T>
 __device__ __forceinline__ void tail_relax(const TailLev &L, int nsweep, int &buf, bool zero,
-                                           bool resid) {
-  if (threadIdx.x == 0) tail_st<T>(L.phi + 4 * L.ps, T(0));  // the zero slot
-  if (zero) tail_fill_zero<T>(L, buf);
-  else
-    __syncthreads();
+                                           bool resid, bool walls) {
+  if (__builtin_expect(walls, 0)) {
+    tail_relax_walls<T>(L, nsweep, buf, zero, resid);
+    return;
+  }
+  if (zero) {  // (the level's first visit: on the way up the zero slot is set)
+    if (threadIdx.x == 0) tail_st<T>(L.phi + 4 * L.ps, T(0));
+    tail_fill_zero<T>(L, buf);
+  }
   TailCells<T> W;
   if (L.n <= TAIL_U * TAIL_THREADS) {
     W.set(L, 0);
@@ -3012,12 +3068,26 @@ __host__ __device__ inline unsigned tail_eig_bytes(int ni, int nj, int nk) {
   return tail_eig_axis(ni) + tail_eig_axis(nj) + tail_eig_axis(nk);
 }
 
-template <bool MIXED>
+// A barrier that waits for the wave's LDS
+// accesses only (the loads and stores of global memory in flight stay so)
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// EX: mixed precision with the exact coarsest solve (its blocks have two
+// levels or more): no FP64 sweeps in the kernel.  A second copy of the sweeps
+// makes registers spill (51; none with one copy): us a cycle, 32^3 of 4 levels,
+// 74.0 with both copies, now 69.9; FP64, whose coarsest level shares the copy
+// of the others, 79.1 and 77.1.
+template <bool MIXED, bool EX>
 __global__ void __launch_bounds__(TAIL_THREADS)
     k_vtail(const Tile *__restrict__ tiles, const LevelDev *__restrict__ levs,
             const int *__restrict__ active, const double *const *__restrict__ eig_q,
             const double *const *__restrict__ eig_l, int nu1, int nu2, int exact) {
   extern __shared__ __align__(16) char smem[];
+  __shared__ int bad;
   const Tile t = tiles[blockIdx.x];
   const int nl = t.z1;  // the block's levels from the tail level down
   const LevelDev &G = levs[t.lev];
@@ -3028,7 +3098,8 @@ __global__ void __launch_bounds__(TAIL_THREADS)
   const int last = nl - 1;
   const int tid = (int)threadIdx.x;
   const TailLev L0 = tail_level<MIXED>(G, 0, nl), Z = tail_level<MIXED>(G, last, nl);
-  const bool do_exact = exact && (nl > 1 || G.finer >= 0);  // as the host: not for a 1-level block
+  // as the host: not for a 1-level block
+  const bool do_exact = MIXED ? EX : exact && (nl > 1 || G.finer >= 0);
   // the exact solve's tables (Q and lambda of each axis, one contiguous image
   // in the block's region, each part 256-byte aligned) and scratch follow the
   // levels
@@ -3039,6 +3110,7 @@ __global__ void __launch_bounds__(TAIL_THREADS)
     for (unsigned e = (unsigned)tid * 8u; e < bytes; e += TAIL_THREADS * 8u)
       tail_st<double>(eo + e, *(const gmem<double> *)(eg + e));
   }
+  if (tid == 0) bad = 0;
   // the top level's rhs into LDS; its phi starts from zero
   const bool top64 = !MIXED || nl == 1;
   for (int c = 0; c < 2; ++c) {
@@ -3048,58 +3120,84 @@ __global__ void __launch_bounds__(TAIL_THREADS)
       tail_copy((lds<float> *)(smem + L0.rhs + c * L0.rs), (const gmem<float> *)G.rhs[c], L0.n);
   }
   __syncthreads();
-  // coarsest level of the block (always FP64)
-  auto coarsest = [&]() __attribute__((always_inline)) {
-    const TailLev &L = Z;
-    if (do_exact) {
-      const unsigned q1 = eo + tail_eig_axis(L.ni), q2 = q1 + tail_eig_axis(L.nj),
-                     sc = q2 + tail_eig_axis(L.nk), n3 = (unsigned)(L.ni * L.nj * L.nk) * 8u;
-      auto at = [&](unsigned o) { return (ldsd)((lds<char> *)smem + o); };
-      coarse_exact_lds(L.ni, L.nj, L.nk, L.H, at(L.rhs), at(L.rhs + L.rs),
-                       at(L.phi + (unsigned)(2 * fin) * L.ps),
-                       at(L.phi + (unsigned)(2 * fin + 1) * L.ps), at(eo), at(q1), at(q2),
-                       at(eo + tail_eig_q(L.ni)), at(q1 + tail_eig_q(L.nj)),
-                       at(q2 + tail_eig_q(L.nk)), at(sc), at(sc + n3));
-      return;
+  // the top level's phi (buffer fin) back to global; `bad` when a cell of it
+  // is not finite
+  auto write_top = [&](auto zero) __attribute__((always_inline)) {
+    typedef decltype(zero) S;
+    for (int c = 0; c < 2; ++c) {
+      const unsigned o = L0.phi + (unsigned)(2 * fin + c) * L0.ps;
+      gmem<S> *const out = (gmem<S> *)G.phi[fin][c];
+      for (int e = tid; e < L0.n; e += TAIL_THREADS) {
+        const S v = tail_ld<S>(o + (unsigned)e * (unsigned)sizeof(S));
+        out[e] = v;
+        if (__builtin_expect(!isfinite(v), 0)) {
+          int m, j, k;
+          TailSplit{L0}(e, m, j, k);
+          if (2 * m + ((c + j + k) & 1) < L0.ni) bad = 1;  // (not a pad entry)
+        }
+      }
     }
-    int buf = 0;
-    tail_relax<double>(L, nu1 + nu2, buf, true, false);
   };
+  // the coarsest level's exact solve
+  auto coarsest_exact = [&]() __attribute__((always_inline)) {
+    const TailLev &L = Z;
+    const unsigned q1 = eo + tail_eig_axis(L.ni), q2 = q1 + tail_eig_axis(L.nj),
+                   sc = q2 + tail_eig_axis(L.nk), n3 = (unsigned)(L.ni * L.nj * L.nk) * 8u;
+    auto at = [&](unsigned o) { return (ldsd)((lds<char> *)smem + o); };
+    coarse_exact_lds(L.ni, L.nj, L.nk, L.H, at(L.rhs), at(L.rhs + L.rs),
+                     at(L.phi + (unsigned)(2 * fin) * L.ps),
+                     at(L.phi + (unsigned)(2 * fin + 1) * L.ps), at(eo), at(q1), at(q2),
+                     at(eo + tail_eig_q(L.ni)), at(q1 + tail_eig_q(L.nj)),
+                     at(q2 + tail_eig_q(L.nk)), at(sc), at(sc + n3));
+  };
+  bool walls = false;
   // One copy of every piece of code, run level by level: the kernel runs each
   // only a few times per launch, and its instruction fetches count (a cold
   // kilobyte of code costs ~0.8 us here).
 #pragma clang loop unroll(disable)
-  for (int q = 0, up = 0; q >= 0; up ? --q : ++q) {
-    // one level on the way down (up = 0) or up; the coarsest turns around
-    if (q == last) {
-      coarsest();
-      up = 1;
-      continue;
+  for (;;) {
+#pragma clang loop unroll(disable)
+    for (int q = 0, up = 0; q >= 0; up ? --q : ++q) {
+      // one level on the way down (up = 0) or up; the coarsest (always FP64)
+      // turns around
+      const bool bottom = q == last;
+      if (bottom && (do_exact || MIXED)) {
+        int buf = 0;
+        if (do_exact)
+          coarsest_exact();
+        else
+          tail_relax<double>(Z, nu1 + nu2, buf, true, false, walls);
+        up = 1;
+        continue;
+      }
+      const TailLev L = tail_level<MIXED>(G, q, nl), C = tail_level<MIXED>(G, q + 1, nl);
+      const bool c64 = !MIXED || q + 1 == last;
+      int buf = up ? nu1 & 1 : 0;
+      if (up) {
+        if (c64)
+          tail_prolong<T, double>(L, C, buf, fin);
+        else
+          tail_prolong<T, T>(L, C, buf, fin);
+      }
+      tail_relax<T>(L, bottom ? nu1 + nu2 : up ? nu2 : nu1, buf, !up, !up && !bottom, walls);
+      if (!up && !bottom) {
+        if (c64)
+          tail_sum8<T, double>(L, C, buf);
+        else
+          tail_sum8<T, T>(L, C, buf);
+      }
+      if (bottom) up = 1;
     }
-    const TailLev L = tail_level<MIXED>(G, q, nl), C = tail_level<MIXED>(G, q + 1, nl);
-    const bool c64 = !MIXED || q + 1 == last;
-    int buf = up ? nu1 & 1 : 0;
-    if (up) {
-      if (c64)
-        tail_prolong<T, double>(L, C, buf, fin);
-      else
-        tail_prolong<T, T>(L, C, buf, fin);
-    }
-    tail_relax<T>(L, up ? nu2 : nu1, buf, !up, !up);
-    if (!up) {
-      if (c64)
-        tail_sum8<T, double>(L, C, buf);
-      else
-        tail_sum8<T, T>(L, C, buf);
-    }
-  }
-  // top level's phi (buffer fin) back to global
-  for (int c = 0; c < 2; ++c) {
-    const unsigned o = L0.phi + (unsigned)(2 * fin + c) * L0.ps;
     if (top64)
-      tail_copy((gmem<double> *)G.phi[fin][c], (const lds<double> *)(smem + o), L0.n);
+      write_top(0.0);
     else
-      tail_copy((gmem<float> *)G.phi[fin][c], (const lds<float> *)(smem + o), L0.n);
+      write_top(0.0f);
+    // An infinity or NaN stays in a level once a black cell has it, and goes
+    // up with the corrections: a finite result has met none, and zero was
+    // every wall's term.
+    lds_barrier();
+    if (__builtin_expect(walls || !bad, 1)) break;
+    walls = true;
   }
 }
 
@@ -4669,14 +4767,6 @@ __global__ void __launch_bounds__(NTHREADS)
   if (v == 0) first[(size_t)p * A.nl + u] = PASS == 2 ? val(-1, j, k) : val(i, j, -1);
 }
 
-// LDS and barrier of k_tdma_lines: a barrier waits for the wave's LDS
-// accesses only (the loads and stores of global memory in flight stay so)
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // back substitution of k_tdma_lines: phi(p) = c(p) - a(p)*phi(p+1), the
 // operands a chunk ahead of the chain.  SHORT: any chunk may lie past the
 // line's end, not just part of the last one.
@@ -5242,20 +5332,19 @@ void launch_vtail(hipStream_t s, const Tile *tiles, int ntiles, const LevelDev *
                   const int *active, const double *const *eig_q, const double *const *eig_l,
                   int nu1, int nu2, int exact, int mixed, size_t lds_bytes) {
   if (ntiles <= 0) return;
-  if (mixed)
-    hipLaunchKernelGGL(k_vtail<true>, dim3(ntiles), dim3(TAIL_THREADS), lds_bytes, s, tiles, levs,
-                       active, eig_q, eig_l, nu1, nu2, exact);
-  else
-    hipLaunchKernelGGL(k_vtail<false>, dim3(ntiles), dim3(TAIL_THREADS), lds_bytes, s, tiles, levs,
-                       active, eig_q, eig_l, nu1, nu2, exact);
+  auto k = !mixed ? k_vtail<false, false> : exact ? k_vtail<true, true> : k_vtail<true, false>;
+  hipLaunchKernelGGL(k, dim3(ntiles), dim3(TAIL_THREADS), lds_bytes, s, tiles, levs, active, eig_q,
+                     eig_l, nu1, nu2, exact);
 }
 
 hipError_t vtail_allow_lds(size_t lds_bytes) {
-  hipError_t e = hipFuncSetAttribute((const void *)k_vtail<true>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
-  if (e != hipSuccess) return e;
-  return hipFuncSetAttribute((const void *)k_vtail<false>,
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+  for (const void *f : {(const void *)k_vtail<false, false>, (const void *)k_vtail<true, true>,
+                        (const void *)k_vtail<true, false>}) {
+    const hipError_t e =
+        hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 size_t vtail_lds_bytes(const LevelDev *levs_host, int top, bool mixed, bool exact, bool padded) {
