@@ -1474,9 +1474,10 @@ __global__ void __launch_bounds__(NTHREADS)
 // skip_red: a red half-sweep follows.  It replaces every red cell from black
 // neighbours, and of the red values before it only those on open (periodic or
 // shared) faces are read again, as ghosts of the black half-sweep: the other
-// red cells are left as they are.  The kernel streams the fine level, so that
-// takes up to half its traffic (four levels of 256^3, FP64: 18.0 us a launch, now
-// 14.0; float 10.2 and 9.4).
+// red cells are left as they are, unless a correction is not finite (a wall's
+// term is zero times the cell's own value: NaN after an infinite correction).
+// The kernel streams the fine level, so that takes up to half its traffic (four
+// levels of 256^3, FP64: 18.0 us a launch, now 14.0; float 10.2 and 9.4).
 // ONE, scalar arguments: as k_rb_sweep (one_lev the fine descriptor,
 // one_lev2 its coarser level).
 template <class Tf, class Tc, bool GEN, bool ONE>
@@ -1557,6 +1558,10 @@ __global__ void __launch_bounds__(NTHREADS)
           cv[a][b][c] = ((xc[a] + yc[b] + zc[c]) & 1) ? C1[off] : C0[off];
         }
       }
+  Tc all = cv[0][0][0];  // finite: every corner is
+#pragma unroll
+  for (int q = 1; q < 16; ++q) all = all + cv[q >> 2][(q >> 1) & 1][q & 1];
+  const bool finite = isfinite(all);
   gmem<Tf> *F0 = (gmem<Tf> *)F.phi[src_f][0];
   gmem<Tf> *F1 = (gmem<Tf> *)F.phi[src_f][1];
   // lanes with a cell on an open x face (the fine and coarse level have the
@@ -1573,7 +1578,7 @@ __global__ void __launch_bounds__(NTHREADS)
       if (j < 0 || j >= F.nj) continue;
       const unsigned fq = ((unsigned)k * (unsigned)F.nj + (unsigned)j) * (unsigned)F.H + (unsigned)l;
       // the row's cells 2l+e with e = (j+k) & 1 are red
-      bool red = !skip_red || x_open;
+      bool red = !skip_red || x_open || !finite;
       if (GEN)
         red = red || (j == 0 && !wall_face(F, 2)) || (j == F.nj - 1 && !wall_face(F, 3)) ||
               (k == 0 && !wall_face(F, 4)) || (k == F.nk - 1 && !wall_face(F, 5));

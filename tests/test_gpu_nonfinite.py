@@ -33,6 +33,7 @@ def _rhs(n, seed, value, at):
 @pytest.mark.parametrize("value", [np.inf, np.nan, 1e300], ids=str)
 @pytest.mark.parametrize("n,nlev,routes", [
     ((16, 16, 16), 3, "tail"), ((20, 8, 12), 3, "tail"), ((16, 16, 16), 5, "tail"),
+    ((16, 36, 52), 2, "half"), ((20, 24, 16), 3, "half"),
 ])
 def test_gpu_nonfinite_values_equal_oracle(gpu_lib, n, nlev, routes, value):
     from oracle import oracle as O
