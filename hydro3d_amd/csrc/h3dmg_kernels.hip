@@ -709,9 +709,14 @@ __device__ __forceinline__ void rb_dispatch(const Tile &t, const LevelDev &L, in
 // of cells: the colours continue, too).  A black cell reads across such a
 // face the red value from before the sweep (`old`), as the ghosts hold it;
 // across a wall the product of a zero coefficient and a zero, as the cells
-// beyond are never set.  The result goes to the other buffer, once: the
-// launch is one step of the level's buffers.  zero != 0: the
-// level holds zeros.
+// beyond are never set, where the other kernels multiply zero by the cell's own
+// value before the sweep: NaN where that is not finite.  A tile that has loaded
+// values beyond the middle of the exponent range (smaller ones stay finite over
+// two sweeps) runs again that way: as the only way it took 9% of a 48^3 cycle
+// (FP64), one path with a flag 4%, a second copy of the sweeps none (FP32, bound
+// by its registers: 2% at 104x56x40).  The result goes to the other buffer, once:
+// the launch is one step of the level's buffers.  zero != 0: the level holds
+// zeros.
 constexpr int RBT = 16, RBT_HALF = RBT * RBT * RBT / 2, RBT_THREADS = 1024;
 template <class T>
 __global__ void __launch_bounds__(RBT_THREADS, sizeof(T) == 4 ? 8 : 4)
@@ -720,6 +725,7 @@ __global__ void __launch_bounds__(RBT_THREADS, sizeof(T) == 4 ? 8 : 4)
               const FineDev *__restrict__ fine) {
   constexpr int HALO = 4, TS = RBT - 2 * HALO, U = RBT_HALF / RBT_THREADS;
   __shared__ T black[RBT_HALF], red[RBT_HALF], old[RBT_HALF];
+  __shared__ int large;  // a thread has loaded such values
   const LevelDev &L = levs[one_lev];
   const int on = active[one_blk];
   const int ni = L.ni, nj = L.nj, nk = L.nk, H = L.H;
@@ -730,6 +736,7 @@ __global__ void __launch_bounds__(RBT_THREADS, sizeof(T) == 4 ? 8 : 4)
   // whether a periodic face cuts the positions
   const bool cross = (px && (x0 < 0 || x0 + RBT > ni)) || (py && (y0 < 0 || y0 + RBT > nj)) ||
                      (pz && (z0 < 0 || z0 + RBT > nk));
+  const unsigned walls = (px ? 0u : 3u) | (py ? 0u : 12u) | (pz ? 0u : 48u);
   const gmem<T> *P[2] = {(const gmem<T> *)L.phi[src][0], (const gmem<T> *)L.phi[src][1]};
   const gmem<T> *R[2] = {(const gmem<T> *)L.rhs[0], (const gmem<T> *)L.rhs[1]};
   gmem<T> *D[2] = {(gmem<T> *)L.phi[1 - src][0], (gmem<T> *)L.phi[1 - src][1]};
@@ -763,14 +770,24 @@ __global__ void __launch_bounds__(RBT_THREADS, sizeof(T) == 4 ? 8 : 4)
     v1[u] = zero ? T(0) : P[1][ent[u][1]];
     v0[u] = zero || !cross ? T(0) : P[0][ent[u][0]];
   }
+  T most = T(0);
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int q = tid + u * RBT_THREADS;
-    black[q] = face[u][1] & 64u ? v1[u] : T(0);
-    red[q] = face[u][0] & 64u ? v0[u] : T(0);
-    if (cross) old[q] = T(0);
-  }
-  __syncthreads();
+  for (int u = 0; u < U; ++u)
+    most = most + fabs(r[u][0]) + fabs(r[u][1]) + fabs(v1[u]) + fabs(v0[u]);
+  const bool big = !(most < (sizeof(T) == 4 ? T(0x1p64) : T(0x1p500)));
+  auto fill = [&]() {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = tid + u * RBT_THREADS;
+      black[q] = face[u][1] & 64u ? v1[u] : T(0);
+      red[q] = face[u][0] & 64u ? v0[u] : T(0);
+      if (cross) old[q] = T(0);
+    }
+    if (tid == 0) large = 0;
+    __syncthreads();
+  };
+  fill();
+  if (__builtin_expect(big, 0)) large = 1;
   const T cx = (T)L.cx, cy = (T)L.cy, cz = (T)L.cz;
   // the update of entry q of colour c from the six values
   auto update = [&](unsigned f, T rhs, const T(&v)[6]) -> T {
@@ -785,46 +802,66 @@ __global__ void __launch_bounds__(RBT_THREADS, sizeof(T) == 4 ? 8 : 4)
     const T sum = aw * v[0] + ae * v[1] + as * v[2] + an * v[3] + ab * v[4] + at * v[5];
     return div_ap(rhs - sum, ap, T(1) / ap);
   };
+  auto at_walls = [&](unsigned f, T own, T(&v)[6]) {
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+      if ((f & walls) >> q & 1u) v[q] = own;
+  };
   // whether half-sweep h computes the entry: one layer less each
   auto in = [&](int c, int rz, int h) {
     const int rx = 2 * m + ((c + y0 + ry + z0 + rz) & 1), lo = h + 1, hi = RBT - 2 - h;
     return rx >= lo && rx <= hi && ry >= lo && ry <= hi && rz >= lo && rz <= hi;
   };
+  auto sweeps = [&](auto own) __attribute__((always_inline)) {
+    constexpr bool OWN = decltype(own)::value;
 #pragma unroll 1
-  for (int h = 0; h < HALO; h += 2) {
+    for (int h = 0; h < HALO; h += 2) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int q = tid + u * RBT_THREADS, rz = (tid >> 7) + RBT_THREADS / 128 * u;
-      if (!in(0, rz, h) || !(face[u][0] & 64u)) continue;
-      const int s = (y0 + ry + z0 + rz) & 1;
-      const T v[6] = {black[q - 1 + s],       black[q + s],
-                      black[q - RBT / 2],     black[q + RBT / 2],
-                      black[q - RBT * RBT / 2], black[q + RBT * RBT / 2]};
-      const T x = update(face[u][0], r[u][0], v);
-      if (cross) old[q] = red[q];
-      red[q] = x;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int q = tid + u * RBT_THREADS, rz = (tid >> 7) + RBT_THREADS / 128 * u;
-      if (!in(1, rz, h + 1) || !(face[u][1] & 64u)) continue;
-      const int s = (1 + y0 + ry + z0 + rz) & 1;
-      const int at[6] = {q - 1 + s,   q + s, q - RBT / 2, q + RBT / 2, q - RBT * RBT / 2,
-                         q + RBT * RBT / 2};
-      T v[6];
-#pragma unroll
-      for (int f = 0; f < 6; ++f) v[f] = red[at[f]];
-      if (cross) {
-#pragma unroll
-        for (int f = 0; f < 6; ++f) {
-          const T w = old[at[f]];
-          if ((face[u][1] >> f) & 1u) v[f] = w;  // (a wall's coefficient is 0)
-        }
+      for (int u = 0; u < U; ++u) {
+        const int q = tid + u * RBT_THREADS, rz = (tid >> 7) + RBT_THREADS / 128 * u;
+        if (!in(0, rz, h) || !(face[u][0] & 64u)) continue;
+        const int s = (y0 + ry + z0 + rz) & 1;
+        T v[6] = {black[q - 1 + s],       black[q + s],
+                  black[q - RBT / 2],     black[q + RBT / 2],
+                  black[q - RBT * RBT / 2], black[q + RBT * RBT / 2]};
+        if constexpr (OWN) at_walls(face[u][0], red[q], v);
+        const T x = update(face[u][0], r[u][0], v);
+        if (cross) old[q] = red[q];
+        red[q] = x;
       }
-      black[q] = update(face[u][1], r[u][1], v);
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = tid + u * RBT_THREADS, rz = (tid >> 7) + RBT_THREADS / 128 * u;
+        if (!in(1, rz, h + 1) || !(face[u][1] & 64u)) continue;
+        const int s = (1 + y0 + ry + z0 + rz) & 1;
+        const int at[6] = {q - 1 + s,   q + s, q - RBT / 2, q + RBT / 2, q - RBT * RBT / 2,
+                           q + RBT * RBT / 2};
+        T v[6];
+#pragma unroll
+        for (int f = 0; f < 6; ++f) v[f] = red[at[f]];
+        if (cross) {
+#pragma unroll
+          for (int f = 0; f < 6; ++f) {
+            const T w = old[at[f]];
+            if ((face[u][1] >> f) & 1u) v[f] = w;  // (at a wall its coefficient is 0)
+          }
+        }
+        if constexpr (OWN) at_walls(face[u][1], black[q], v);
+        black[q] = update(face[u][1], r[u][1], v);
+      }
+      __syncthreads();
     }
-    __syncthreads();
+  };
+  sweeps(std::false_type());
+  if (__builtin_expect(large, 0)) {
+    __syncthreads();  // every wavefront has read `large`
+    for (int u = 0; u < U; ++u) {
+      v1[u] = zero ? T(0) : P[1][ent[u][1]];
+      v0[u] = zero ? T(0) : P[0][ent[u][0]];
+    }
+    fill();
+    sweeps(std::true_type());
   }
 #pragma unroll
   for (int u = 0; u < U; ++u) {

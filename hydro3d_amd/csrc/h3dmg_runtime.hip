@@ -1747,6 +1747,9 @@ h3dmg_status gen_relax(h3dmg_handle *h, int g) {
       }
       const bool is64 = !is_mixed(h) || grp == 1;
       ts.multi = ts.multi && tiles <= (is64 ? 1 : 2) * RB_TILE_CUS;
+      // (a single cell between walls divides by zero: k_rb_tile looks for
+      // values near the ends of the exponent range in what it loads only)
+      ts.multi = ts.multi && n[0] * n[1] * n[2] > 1;
     }
     // Level 1 ends in one buffer for every block (pp_buf, read by the update
     // and h3dmg_get_pp).  Blocks of one level beside deeper ones are two

@@ -33,7 +33,8 @@ def _rhs(n, seed, value, at):
 @pytest.mark.parametrize("value", [np.inf, np.nan, 1e300], ids=str)
 @pytest.mark.parametrize("n,nlev,routes", [
     ((16, 16, 16), 3, "tail"), ((20, 8, 12), 3, "tail"), ((16, 16, 16), 5, "tail"),
-    ((16, 36, 52), 2, "half"), ((20, 24, 16), 3, "half"),
+    ((32, 24, 16), 1, "pairs"), ((16, 18, 20), 2, "pairs"), ((16, 36, 52), 2, "half"), ((20, 24, 16), 3, "half"),
+    ((16, 16, 16), 5, "pairs"), ((16, 16, 16), 5, "half"),
 ])
 def test_gpu_nonfinite_values_equal_oracle(gpu_lib, n, nlev, routes, value):
     from oracle import oracle as O
@@ -46,3 +47,19 @@ def test_gpu_nonfinite_values_equal_oracle(gpu_lib, n, nlev, routes, value):
                 tail = 1 if routes == "tail" else nlev + 1
                 got = _pp(n, nlev, bc, f, nu, tail, 1 if routes == "half" else 0)
                 assert np.array_equal(got, want, equal_nan=True), (bc, at, nu)
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan, 1e38], ids=str)
+@pytest.mark.parametrize("n,nlev", [((16, 16, 16), 3), ((18, 20, 28), 2)])
+def test_gpu_nonfinite_values_mixed_routes_agree(gpu_lib, n, nlev, value):
+    for bc in BCS:
+        for at in ("low", "mid", "high"):
+            f = _rhs(n, 17, value, at)
+            for nu in ((2, 2), (0, 1), (2, 1), (0, 3), (4, 0)):
+                print(f"case: mixed {n} bc {bc} {value} at {at} nu {nu}", flush=True)
+                ref = _pp(n, nlev, bc, f, nu, nlev + 1, 1, precision="mixed")
+                for tail, march in ((1, 0), (nlev + 1, 0)):
+                    if tail == 1 and max(n) > 16:
+                        continue
+                    got = _pp(n, nlev, bc, f, nu, tail, march, precision="mixed")
+                    assert np.array_equal(got, ref, equal_nan=True), (bc, at, nu, tail, march)
