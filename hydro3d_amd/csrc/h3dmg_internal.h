@@ -291,7 +291,7 @@ struct ProjLaunch {
   int groups;     // workgroups per block (and partials per block)
   int kb;         // planes per tile
   int connected;  // near faces belong to the block across them
-  int to_fine;    // su into f and the level-1 rhs (else VelDev::su)
+  int to_fine;    // su into f, 2: and the level-1 rhs (0: VelDev::su)
   int calmas;     // 0: the faces only
   int lsm, f32;   // variable density; level 1 in FP32
   int even;       // every block of the launch has an even ni

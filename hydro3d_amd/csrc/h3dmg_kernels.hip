@@ -3516,8 +3516,9 @@ __global__ void __launch_bounds__(256)
 // expression.
 //   connected: a near face across which a block lies takes that block's far
 //     face -- its u* and this face's pressures, the value k_face_copy copies;
-//   to_fine: su goes into the block's f arrays and the level-1 rhs in the
-//     level's type T (the next V-cycle starts from it), else to V.su if any;
+//   to_fine: su goes into the block's f arrays and, to_fine = 2, the level-1
+//     rhs in the level's type T (the next V-cycle starts from it); 0: to V.su
+//     if any;
 //   calmas = 0: faces only (calmas' 4th-order branch follows on its own).
 // Bound by memory: 192^3 takes 113 us (453 MB, 4.0 TB/s) where calvel x 3 +
 // calmas took 174; 128x128x96 28 us where they took 47; the 64 blocks of a
@@ -3562,8 +3563,8 @@ __global__ void __launch_bounds__(NTHREADS)
     gmem<double> *const U = (gmem<double> *)V.u, *const Vv = (gmem<double> *)V.v,
                  *const W = (gmem<double> *)V.w;
     gmem<double> *const F0 = (gmem<double> *)F.f[0], *const F1 = (gmem<double> *)F.f[1];
-    gmem<T> *const R0 = to_fine ? (gmem<T> *)levs[b].rhs[0] : nullptr,
-                  *const R1 = to_fine ? (gmem<T> *)levs[b].rhs[1] : nullptr;
+    gmem<T> *const R0 = (gmem<T> *)levs[b].rhs[0], *const R1 = (gmem<T> *)levs[b].rhs[1];
+    const bool to_rhs = to_fine == 2;
     const size_t pu = (size_t)(ni + 1), plane = (size_t)ni * nj;
     // u = us - dta*(ph - pl)/h, over the face density of an L_LSM handle
     auto corr = [&](double us, double pl, double ph, double h, double dl, double dh) -> double {
@@ -3732,11 +3733,11 @@ __global__ void __launch_bounds__(NTHREADS)
             const bool odd = (jc + k) & 1;
             if (ok) {
               (odd ? F1 : F0)[o] = ra;
-              (odd ? R1 : R0)[o] = (T)ra;
+              if (to_rhs) (odd ? R1 : R0)[o] = (T)ra;
             }
             if (okb) {
               (odd ? F0 : F1)[o] = rb;
-              (odd ? R0 : R1)[o] = (T)rb;
+              if (to_rhs) (odd ? R0 : R1)[o] = (T)rb;
             }
           } else if (V.su) {
             st((gmem<double> *)V.su, qw, d2{ra, rb});

@@ -325,6 +325,9 @@ struct h3dmg_handle {
   // the level-1 rhs arrays hold su (f) of every enabled block: the velocity
   // step's V-cycle starts without copying it there
   bool rhs_is_f = false;
+  // the projection writes su there, too: not while a block's stepped solve
+  // runs, whose next V-cycle starts from the residual they hold
+  bool proj_rhs = true;
   hipGraph_t vgraph = nullptr;
   hipGraphExec_t vgexec = nullptr;
 
@@ -1961,7 +1964,7 @@ ProjLaunch project_shape(const h3dmg_handle *h) {
 void enqueue_project(h3dmg_handle *h) {
   if (!h->vel_overlap) {
     ProjLaunch a = project_shape(h);
-    a.to_fine = 1;
+    a.to_fine = h->proj_rhs ? 2 : 1;
     a.calmas = h->differencing == 2 ? 0 : 1;
     launch_project(h->stream, a, h->d_fine, h->d_levs, h->d_active, h->d_vel, h->d_projdt,
                    VelDev{}, ProjDt{}, 0, h->nb, a.calmas ? h->d_pparts : nullptr);
@@ -2048,10 +2051,30 @@ void enqueue_velocity_step(h3dmg_handle *h) {
   enqueue_project(h);
 }
 
+// drops the captured velocity step
+h3dmg_status drop_velocity_graph(h3dmg_handle *h) {
+  std::lock_guard<std::mutex> lock(g_device_mutex);
+  HIP_TRY(hipStreamSynchronize(h->stream));
+  if (h->vgexec) (void)hipGraphExecDestroy(h->vgexec);
+  if (h->vgraph) (void)hipGraphDestroy(h->vgraph);
+  h->vgexec = nullptr;
+  h->vgraph = nullptr;
+  return H3DMG_OK;
+}
+
+// proj_rhs for the projections to come; the captured step follows
+h3dmg_status choose_proj_rhs(h3dmg_handle *h) {
+  const bool rhs = std::none_of(h->running.begin(), h->running.end(), [](char r) { return r; });
+  if (rhs == h->proj_rhs) return H3DMG_OK;
+  h->proj_rhs = rhs;
+  return drop_velocity_graph(h);
+}
+
 h3dmg_status run_velocity_step(h3dmg_handle *h) {
   if (!h->rhs_is_f) enqueue_rhs_from_f(h);
-  // k_project leaves su in f and in the level-1 rhs, calmas on its own in f
-  h->rhs_is_f = !h->vel_overlap && h->differencing == 1;
+  // k_project leaves su in f and (proj_rhs) in the level-1 rhs, calmas on its
+  // own in f
+  h->rhs_is_f = !h->vel_overlap && h->differencing == 1 && h->proj_rhs;
   if (h->prm.use_graph) {
     if (!h->vgexec) {
       std::lock_guard<std::mutex> lock(g_device_mutex);
@@ -2830,12 +2853,7 @@ h3dmg_status h3dmg_set_block_enabled(h3dmg_handle *h, int b, int enabled) {
   // the velocity loop's block set (and its captured step, which projects
   // the blocks chosen at h3dmg_velocity_begin) is no longer this one
   if (h->vel_ready || h->vgexec) {
-    std::lock_guard<std::mutex> lock(g_device_mutex);
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    if (h->vgexec) (void)hipGraphExecDestroy(h->vgexec);
-    if (h->vgraph) (void)hipGraphDestroy(h->vgraph);
-    h->vgexec = nullptr;
-    h->vgraph = nullptr;
+    if ((st = drop_velocity_graph(h))) return st;
     h->vel_ready = false;
   }
   return H3DMG_OK;
@@ -3369,12 +3387,7 @@ h3dmg_status h3dmg_set_differencing(h3dmg_handle *h, int differencing) {
   if (h->differencing == differencing) return H3DMG_OK;
   h->differencing = differencing;
   // the captured velocity step launches the other calmas
-  std::lock_guard<std::mutex> lock(g_device_mutex);
-  HIP_TRY(hipStreamSynchronize(h->stream));
-  if (h->vgexec) (void)hipGraphExecDestroy(h->vgexec);
-  if (h->vgraph) (void)hipGraphDestroy(h->vgraph);
-  h->vgexec = nullptr;
-  h->vgraph = nullptr;
+  if (h3dmg_status st = drop_velocity_graph(h)) return st;
   h->vel_ready = false;
   return H3DMG_OK;
 }
@@ -3469,14 +3482,9 @@ h3dmg_status h3dmg_velocity_begin(h3dmg_handle *h, const double *const *d_ustar,
          (!baked || (same && h->vel_ready && h->vel_dta == h->prm.dt * alfapr &&
                      h->vel_dt == h->prm.dt));
   h->vel_overlap = overlap;
-  if (!same) {
-    std::lock_guard<std::mutex> lock(g_device_mutex);
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    if (h->vgexec) (void)hipGraphExecDestroy(h->vgexec);
-    if (h->vgraph) (void)hipGraphDestroy(h->vgraph);
-    h->vgexec = nullptr;
-    h->vgraph = nullptr;
-  }
+  if (!same)
+    if (h3dmg_status st = drop_velocity_graph(h)) return st;
+  if (h3dmg_status st = choose_proj_rhs(h)) return st;
   h->vel_dta = h->prm.dt * alfapr;
   h->vel_dt = h->prm.dt;
   h->vel_ready = true;
@@ -3484,7 +3492,7 @@ h3dmg_status h3dmg_velocity_begin(h3dmg_handle *h, const double *const *d_ustar,
   h3dmg_status st = push_active(h);
   if (st) return st;
   if ((st = push_velocity(h))) return st;
-  h->rhs_is_f = !h->vel_overlap && h->differencing == 1;
+  h->rhs_is_f = !h->vel_overlap && h->differencing == 1 && h->proj_rhs;
   enqueue_project(h);
   HIP_TRY(hipGetLastError());
   st = read_stats(h);
@@ -3506,6 +3514,7 @@ h3dmg_status h3dmg_velocity_step(h3dmg_handle *h, double *rmax) {
   reset_active(h);
   h3dmg_status st = push_active(h);
   if (st) return st;
+  if ((st = choose_proj_rhs(h))) return st;
   st = run_velocity_step(h);
   if (st) return st;
   st = read_stats(h);
