@@ -1807,17 +1807,17 @@ size_t tail_lds_at(const h3dmg_handle *h, int g, bool padded) {
 // whose blocks all have the same number of levels, and where the sweeps saved
 // pay for the kernel: three levels or more with two sweeps or more per visit
 // pair (nu1 + nu2), two levels with three sweeps or more, and five where the
-// launches would take pairs of sweeps (one block, TileSet::multi).  Measured per cycle, tail from 16^3 | every level its own launches, us:
-// three levels (32^3 of 4, FP64) V(2,2) 81 | 90, V(1,1) 73 | 83, 48 blocks
-// V(2,2) 134 | 181; two levels (32^3 of 3), one block, mixed exact, V(2,2)
-// 72 | 66, V(3,3) 84 | 88, FP64 smoothed 74 | 72 and 89 | 107; 48 blocks
-// V(2,2) 126 | 150, V(2,1) 115 | 127, 16 blocks V(1,1) 72 | 69; V(1,0) of three
-// levels 82 | 78.  The coarsest level alone is left to its launches: an exact
-// solve there takes 62 (16^3 blocks) to 74 (28^3) us a two-level cycle in the
-// tail's one workgroup, 55 to 59 spread over the chip, a smoothed one as long
-// either way.  Handles of unequal depths: with the exact solve the first level
-// from the shallowest block's coarsest down that fits (the deeper blocks'
-// levels and all exact solves in one launch).
+// launches would take pairs of sweeps (one block, TileSet::multi).  Measured
+// per cycle, tail from 16^3 | every level its own launches, us: three levels
+// (32^3 of 4, FP64) V(2,2) 78 | 87, V(1,1) 71 | 80, 48 blocks V(2,2) 127 | 178,
+// V(1,0) 68 | 64; two levels (32^3 of 3), one block, mixed exact, V(2,2) 66 | 65,
+// V(3,3) 79 | 87, FP64 smoothed 70 | 70 and 85 | 105; 48 blocks, mixed exact,
+// V(2,2) 105 | 123, V(2,1) 95 | 107, 16 blocks V(1,1) 69 | 67.  The coarsest
+// level alone is left to its launches: an exact solve in the tail's one
+// workgroup gains 0 to 2 us a cycle up to 8^3 cells and loses 5 (96^3 of 4) and 6
+// (48^3 of 3) at 12^3, a smoothed one gains 1 to 4.  Handles of unequal depths:
+// with the exact solve the first level from the shallowest block's coarsest down
+// that fits (the deeper blocks' levels and all exact solves in one launch).
 int auto_tail_level(const h3dmg_handle *h) {
   const bool exact = h->prm.coarse == H3DMG_COARSE_EXACT;
   int t0 = h->Lmax;
