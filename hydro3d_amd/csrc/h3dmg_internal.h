@@ -62,7 +62,7 @@ struct LevelDev {
   // 1/(ap - alo*a(p-1)) at every position p of the line
   double *tdma;
   // workspace of the two-launch line passes (tdma_ws_doubles; the block's,
-  // shared by its levels), or null
+  // shared by its levels), or null where the handle has none
   double *tdma_ws;
 };
 
@@ -140,7 +140,7 @@ void launch_restrict(hipStream_t s, const Tile *tiles, int ntiles, int depth, co
 constexpr int PROL_GEN_ROWS = 32;
 // gen != 0: coarse ghosts read through the neighbour table (blocks with
 // neighbours); skip_red: a red half-sweep follows, red cells off the open
-// faces are left alone
+// faces are left alone (while the correction is finite)
 template <class Tf, class Tc>
 void launch_prolong(hipStream_t s, const Tile *tiles, int ntiles, const LevelDev *levs,
                     const int *active, int src_f, int src_c, int gen, int skip_red = 0,
@@ -169,7 +169,6 @@ void launch_update(hipStream_t s, const Tile *tiles, int ntiles, const FineDev *
                    const LevelDev *levs, const int *active, int buf);
 void launch_finalize(hipStream_t s, const int *tile_begin, int nblocks, const RedPartial *partials,
                      RedPartial *out);
-// one workgroup per tile; Tile::lev = coarsest descriptor, Tile::x0 = block
 // grid and LDS of the exact solve of a list of blocks (exact_grid_add of each)
 struct ExactGrid {
   bool split = true;  // every block's planes and columns fit in LDS
@@ -179,6 +178,7 @@ struct ExactGrid {
 };
 void exact_grid_add(ExactGrid &g, const LevelDev &L, size_t lds_budget);
 hipError_t exact_allow_lds(size_t lds_bytes);
+// Tile::lev = coarsest descriptor, Tile::x0 = block, one tile per block
 void launch_coarse_exact(hipStream_t s, const Tile *tiles, int ntiles, const ExactGrid &grid,
                          const LevelDev *levs, const int *active, const double *const *eig_q,
                          const double *const *eig_l, double *const *scratch, int buf);

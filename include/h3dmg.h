@@ -262,7 +262,8 @@ h3dmg_status h3dmg_set_density_device(h3dmg_handle *h, int b, const double *d_de
 h3dmg_status h3dmg_set_differencing(h3dmg_handle *h, int differencing);
 
 /* The time step of the next solve (params.dt): the reference's dt changes
- * from step to step (checkdt.for:117-137). */
+ * from step to step (checkdt.for:117-137).  A velocity loop that has begun
+ * keeps the dt of its h3dmg_velocity_begin. */
 h3dmg_status h3dmg_set_dt(h3dmg_handle *h, double dt);
 
 /* su of block b as the rhs arrays hold it (after h3dmg_set_rhs*, or the
@@ -320,8 +321,9 @@ h3dmg_status h3dmg_set_block_enabled(h3dmg_handle *h, int b, int enabled);
  * and return them on h3dmg_destroy (H3DMG_ERR_NOMEM when the pool is full).
  * A pooled handle holds independent blocks only (no H3DMG_BC_NEIGHBOUR
  * faces), and refuses the velocity loop and the variable-density operator
- * (H3DMG_ERR_UNSUPPORTED).  One pool serves several handles at once, on
- * several streams and host threads. */
+ * (H3DMG_ERR_UNSUPPORTED).  Its line-TDMA sweeps do without the workspace that
+ * other handles' have outside the block regions.  One pool serves several
+ * handles at once, on several streams and host threads. */
 typedef struct h3dmg_pool h3dmg_pool;
 /* `bytes` of device memory and `max_blocks` pinned per-block statistics
  * entries (the blocks of all the pool's live handles together). */
@@ -388,7 +390,9 @@ h3dmg_status h3dmg_set_stream(h3dmg_handle *h, void *stream);
  * Planes each smoother workgroup walks at `level` (every block): 1, 2 or 4
  * (larger requests use 4; the depth in use is the largest power of two not
  * above the request that divides every block's nk at that level); 0 restores
- * the built-in choice.  Results do not depend on it.  Drops a captured graph.
+ * the built-in choice, which on mid-size levels of one block also takes sweeps
+ * in pairs, one launch each.  Results do not depend on it.  Drops a captured
+ * graph.
  * h3dmg_get_march returns the depth in use (or -1 for a bad level). */
 h3dmg_status h3dmg_set_march(h3dmg_handle *h, int level, int planes);
 int h3dmg_get_march(const h3dmg_handle *h, int level);
@@ -410,10 +414,12 @@ h3dmg_status h3dmg_set_fused(h3dmg_handle *h, long long max_cells);
 long long h3dmg_get_fused(const h3dmg_handle *h);
 /* Levels >= `level` of every block run as one workgroup per block in a
  * single launch with every level in LDS (the V-cycle tail); 0 restores the
- * automatic choice (with H3DMG_COARSE_EXACT the first level, from the
- * shallowest block's coarsest down, whose remaining levels fit in one
- * workgroup's LDS: the tail then runs the blocks' exact coarse solves;
- * otherwise off), a level above every block's coarsest turns the tail off; a level that does not fit returns H3DMG_ERR_ARG.  Results are
+ * automatic choice (blocks of equal depths: the first level of at most 16^3
+ * cells whose remaining levels fit in one workgroup's LDS, above the coarsest,
+ * where the sweeps it saves pay for it; unequal depths: with
+ * H3DMG_COARSE_EXACT the first level, from the shallowest block's coarsest
+ * down, that fits; otherwise off), a level above every block's coarsest turns
+ * the tail off; a level that does not fit returns H3DMG_ERR_ARG.  Results are
  * identical either way.  Drops a captured graph.  h3dmg_get_tail returns the
  * level in use (nlevels_max + 1 when off).  Red-black smoother only: with GS
  * or TDMA the tail is off and a level that would turn it on returns
