@@ -3677,7 +3677,7 @@ __global__ void __launch_bounds__(NTHREADS)
           pe = ((xe + jc + k) & 1) ? E1[o] : E0[o];
           if (EVEN || ac + 2 <= ni) u2 = US[qu + 2];
         }
-        d2 ds, dn, dp;
+        d2 ds = d2{1.0, 1.0}, dn = ds, dp = ds;
         double dw = 1.0, de = 1.0;
         if (LSM) {
           ds = dens2(ys, k);
